@@ -39,7 +39,7 @@
 //  [17]     flags (int bits): vertex-order code (bits 0..7), degenerate (8),
 //           linear, i.e. one Newton step (9), opaque: Oi >= (1,1,1)
 //           component-wise, color.h:432-435 (10)
-//  [18]     grid index (int bits)  [19] unused
+//  [18]     grid index (int bits)  [19] surface (int bits)
 #define RH_MPREC_FLOATS 20
 #define RH_MPREC_GRID 18
 // Motion-frame micropolygon record, in floats:
@@ -52,17 +52,21 @@
 #define RH_MB_MOVING (1u << 11)
 // Device counters: 0..4 the hider's SPL counters (sample tests, bound hits,
 // stored hits, point-in-polygon hits, second Newton steps), 5 tasks whose
-// list overflowed, 6 micropolygon-bucket references, 7 transparent-hit
-// arena entries taken (may exceed the capacity: then the frame is redone
-// with a larger arena), 8 unused.
+// list overflowed, 6 micropolygon-bucket references, 7 and 8 unused.
 #define RH_NCOUNTERS 9
-// Hit-list entries (its occluding hit included) the combine kernel sorts in
+// Hit-list entries (its occluding hit included) the combine kernels sort in
 // LDS; a sample with more transparent hits goes to the long-list pass.
 #define RH_MAX_HITS 64
-// Transparent-hit arena control words: 0 entries taken, 1 samples left to
-// the long-list pass, 2 combine-list entries, 3 their hit-list entries,
-// 4 and 5 the long-list pass's work offsets.
+// Transparent-hit arena control words: 0 entries that found no room (then the
+// frame is redone with a larger arena), 1 samples left to the long-list pass,
+// 2 samples on the deep list, 3 the long-list pass's hit-list entries, 4 and 5
+// its work offsets.
 #define RH_HITCTL_WORDS 8
+// The arena's parts, the words between their counters (a cache line), and
+// the first entry index that stands for no entry.
+#define RH_HIT_SHARDS 16
+#define RH_HIT_SHARD_WORDS 32
+#define RH_HIT_NOROOM 0x80000000u
 // Sphere parameter layout (see front.h)
 #define SPH_RADIUS_D 0
 #define SPH_MAT_D 1
@@ -146,9 +150,10 @@ struct SampleLaunch {
     const uchar4* pixPattern;
     float4* samples;
     float4* hitData;                      // per transparent hit: u, v, depth, id
-    uint32_t* hitNext;                    // per transparent hit: list link, surface
-    uint32_t* hitCounter;
-    uint4* combineList;
+    uint2* hitNext;                       // per transparent hit: list link, surface
+    uint32_t* hitCtl;
+    uint32_t* hitShards;
+    uint2* hitHeads;                      // per sample: newest transparent hit, their number (null: none kept)
     float* frontDepth;
     uint32_t* rowCounts;
     int rowBase;

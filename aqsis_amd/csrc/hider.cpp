@@ -32,12 +32,13 @@ extern "C" hipError_t rh_launch_sample_dof(hipStream_t, const SampleLaunch*, int
 extern "C" hipError_t rh_sample_occupancy(int, int*);
 extern "C" hipError_t rh_launch_plan_items(hipStream_t, const FrameDev*, const TaskDev*, int, const uint32_t*,
                                            uint32_t, int, uint2*, uint32_t*, uint32_t*);
-extern "C" hipError_t rh_launch_frame_begin(hipStream_t, unsigned long long*, uint32_t*);
-extern "C" hipError_t rh_launch_combine_long(hipStream_t, const FrameDev*, size_t, const uint4*, uint32_t*,
-                                             const float4*, const uint32_t*, const PrimDev*, const float*, int, int,
-                                             const GridDev*, int, float4*, float*, float*, uint32_t*, int*);
-extern "C" hipError_t rh_launch_combine(hipStream_t, const FrameDev*, size_t, const uint4*, uint32_t*,
-                                        const float4*, const uint32_t*, const PrimDev*, const float*, int, int,
+extern "C" hipError_t rh_launch_frame_begin(hipStream_t, unsigned long long*, uint32_t*, uint32_t*);
+extern "C" hipError_t rh_launch_combine_long(hipStream_t, const FrameDev*, size_t, const uint2*,
+                                             const unsigned long long*, uint32_t*, const float4*, const uint2*,
+                                             const PrimDev*, const float*, int, int, const GridDev*, int, float4*,
+                                             float*, float*, uint32_t*, int*);
+extern "C" hipError_t rh_launch_combine(hipStream_t, const FrameDev*, size_t, const uint2*, unsigned long long*,
+                                        uint32_t*, const float4*, const uint2*, const PrimDev*, const float*, int, int,
                                         const GridDev*, int, float4*, float*);
 extern "C" hipError_t rh_launch_reduce_counters(hipStream_t, const uint32_t*, int, const uint32_t*, int,
                                                 unsigned long long*);
@@ -155,7 +156,7 @@ struct rh_ctx {
     DBuf dMprec, dMpbound, dLists, dListCount, dSamples, dChannels, dRgba, dCounters, dBucketRefs;
     DBuf dMprecMB;                        // motion-frame micropolygon records
     // transparent hits: arena of (u, v, depth, id) and (link, surface) pairs
-    DBuf dHitData, dHitNext, dHitCtl, dCombine, dFrontDepth;
+    DBuf dHitData, dHitNext, dHitCtl, dHitShards, dHitHeads, dDeepList, dFrontDepth;
     DBuf dLongWork;                       // the long-list combine's work arrays (grown on demand)
     bool transparent = false;             // some posted surface has Os < 1
     bool anyMatte = false;                // some posted surface is a matte (RH_MATTE)
@@ -192,7 +193,7 @@ struct rh_ctx {
                        &dGrids, &dParams,
                        &dPrims, &dCandStart, &dCandGrid, &dCapStart, &dMprec, &dMpbound, &dLists,
                        &dListCount, &dSamples, &dChannels, &dRgba, &dCounters, &dBucketRefs,
-                       &dHitData, &dHitNext, &dHitCtl, &dCombine, &dFrontDepth, &dLongWork, &dItemsStatic, &dItems,
+                       &dHitData, &dHitNext, &dHitCtl, &dHitShards, &dHitHeads, &dDeepList, &dFrontDepth, &dLongWork, &dItemsStatic, &dItems,
                        &dItemCount, &dQueue, &dRows, &dSegBucket, &dSegCounts, &dMprecMB, &dCullTrees, &dCullPyr,
                        &dCullBounds, &dCullRanges, &dCullStart, &dCullPairMax, &dProbeOut, &dProbeItems,
                        &dProbeTasks, &dProbeCut, &dProbeB, &dProbeC};
@@ -425,6 +426,7 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
         (e = c->dListCount.ensure(s.tasks.size() * sizeof(uint32_t))) != hipSuccess ||
         (e = c->dBucketRefs.ensure(s.buckets.size() * sizeof(uint32_t))) != hipSuccess ||
         (e = c->dHitCtl.ensure(RH_HITCTL_WORDS * sizeof(uint32_t))) != hipSuccess ||
+        (e = c->dHitShards.ensure(RH_HIT_SHARDS * RH_HIT_SHARD_WORDS * sizeof(uint32_t))) != hipSuccess ||
         (e = upload(c->dCounters, zero, c->st)) != hipSuccess ||
         (s.dof && ((e = upload(c->dShuffled, c->plan.shuffled, c->st)) != hipSuccess ||
                    (e = upload(c->dLens, c->plan.lens, c->st)) != hipSuccess ||
@@ -528,7 +530,7 @@ static rh_status set_hit_capacity(rh_ctx* c, uint64_t n) {
     if (n < 64) n = 64;
     if (n > 0x7fffffffull) return fail(RH_ERR_CAPACITY, "transparent hits exceed 2^31 entries");
     HIP_TRY(c->dHitData.ensure(n * sizeof(float4)));
-    HIP_TRY(c->dHitNext.ensure(n * 2 * sizeof(uint32_t)));
+    HIP_TRY(c->dHitNext.ensure(n * sizeof(uint2)));
     c->frame.hitCapacity = (uint32_t)n;
     c->dropGraph();
     std::vector<FrameDev> fv(1, c->frame);
@@ -642,7 +644,8 @@ static rh_status upload_schedule(rh_ctx* c) {
     c->anyMatte = anyMatte;
     const uint64_t nsamp = (uint64_t)s.extW * s.extH * s.ns;
     const uint64_t want = transparent ? arena_guess(s, S, c->prims.data()) : 64;
-    HIP_TRY(c->dCombine.ensure((transparent ? nsamp : 1) * sizeof(uint4)));
+    HIP_TRY(c->dHitHeads.ensure((transparent ? nsamp : 1) * sizeof(uint2)));
+    HIP_TRY(c->dDeepList.ensure((transparent ? nsamp : 1) * sizeof(unsigned long long)));
     HIP_TRY(c->dFrontDepth.ensure((transparent ? nsamp : 1) * sizeof(float)));
     if (want > c->frame.hitCapacity) {
         rh_status r = set_hit_capacity(c, want);
@@ -712,7 +715,7 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
     hipError_t e;
 #define ENQ(x) do { if ((e = (x)) != hipSuccess) return e; } while (0)
     if (timed) ENQ(hipEventRecord(c->ev[0], c->st));
-    ENQ(rh_launch_frame_begin(c->st, k.counters, k.hitCtl));
+    ENQ(rh_launch_frame_begin(c->st, k.counters, k.hitCtl, c->dHitShards.as<uint32_t>()));
     ENQ(rh_launch_dice(c->st, f, c->dGrids.as<GridDev>(), (int)S.grids.size(), c->dPrims.as<PrimDev>(),
                        c->dParams.as<float>(), c->dMprec.as<float>(), c->dMpbound.as<float4>(),
                        S.motion ? c->dMprecMB.as<float4>() : nullptr));
@@ -733,8 +736,9 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
     a.lists = c->dLists.as<uint32_t>(); a.mprec = c->dMprec.as<float>(); a.grids = c->dGrids.as<GridDev>();
     a.prims = c->dPrims.as<PrimDev>(); a.pos2d = c->dPos2d.as<float>(); a.pos1d = c->dPos1d.as<float>();
     a.pixPattern = c->dPix.as<uchar4>(); a.samples = c->dSamples.as<float4>(); a.hitData = c->dHitData.as<float4>();
-    a.hitNext = c->dHitNext.as<uint32_t>(); a.hitCounter = k.hitCtl;
-    a.combineList = c->dCombine.as<uint4>(); a.frontDepth = c->transparent ? c->dFrontDepth.as<float>() : nullptr;
+    a.hitNext = c->dHitNext.as<uint2>(); a.hitCtl = k.hitCtl; a.hitShards = c->dHitShards.as<uint32_t>();
+    a.hitHeads = c->transparent ? c->dHitHeads.as<uint2>() : nullptr;
+    a.frontDepth = c->transparent ? c->dFrontDepth.as<float>() : nullptr;
     a.rowCounts = k.rows; a.rowBase = 0;
     a.idCut = 0xffffffffu; a.depthOnly = 0;
     a.itemCut = nullptr; a.taskList = nullptr;
@@ -775,8 +779,9 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
     }
     if (timed) ENQ(hipEventRecord(c->ev[5], c->st));
     if (c->transparent)
-        ENQ(rh_launch_combine(c->st, f, (size_t)s.extW * s.extH * s.ns, c->dCombine.as<uint4>(),
-                              k.hitCtl, c->dHitData.as<float4>(), c->dHitNext.as<uint32_t>(),
+        ENQ(rh_launch_combine(c->st, f, (size_t)s.extW * s.extH * s.ns, c->dHitHeads.as<uint2>(),
+                              c->dDeepList.as<unsigned long long>(), k.hitCtl, c->dHitData.as<float4>(),
+                              c->dHitNext.as<uint2>(),
                               c->dPrims.as<PrimDev>(), occl_records(c), S.motion ? RH_MPREC_MB_FLOATS : RH_MPREC_FLOATS,
                               S.motion ? RH_MPREC_MB_GRID : RH_MPREC_GRID, c->dGrids.as<GridDev>(), combine_full(c),
                               c->dSamples.as<float4>(),
@@ -793,7 +798,6 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
 // the long-list combine over work arrays sized from the frame's counts
 // (hc[1] samples, hc[3] list entries), then the filter again.
 static rh_status combine_long_lists(rh_ctx* c, const FrameCtl& k, const uint32_t* hc) {
-    const rh::Shape& s = c->shape;
     const size_t entries = hc[3], deferred = hc[1];
     const size_t bytes = entries * (sizeof(float) + sizeof(uint32_t)) + deferred * 192 * sizeof(int);
     HIP_TRY(c->dLongWork.ensure(bytes));
@@ -802,9 +806,9 @@ static rh_status combine_long_lists(rh_ctx* c, const FrameCtl& k, const uint32_t
     uint32_t* workX = reinterpret_cast<uint32_t*>(w + entries * sizeof(float));
     int* workStk = reinterpret_cast<int*>(w + entries * (sizeof(float) + sizeof(uint32_t)));
     const bool motion = c->sched.motion;
-    HIP_TRY(rh_launch_combine_long(c->st, c->dFrame.as<FrameDev>(), (size_t)s.extW * s.extH * s.ns,
-                                   c->dCombine.as<uint4>(), k.hitCtl, c->dHitData.as<float4>(),
-                                   c->dHitNext.as<uint32_t>(), c->dPrims.as<PrimDev>(), occl_records(c),
+    HIP_TRY(rh_launch_combine_long(c->st, c->dFrame.as<FrameDev>(), (size_t)hc[2], c->dHitHeads.as<uint2>(),
+                                   c->dDeepList.as<unsigned long long>(), k.hitCtl, c->dHitData.as<float4>(),
+                                   c->dHitNext.as<uint2>(), c->dPrims.as<PrimDev>(), occl_records(c),
                                    motion ? RH_MPREC_MB_FLOATS : RH_MPREC_FLOATS, motion ? RH_MPREC_MB_GRID : RH_MPREC_GRID,
                                    c->dGrids.as<GridDev>(), combine_full(c), c->dSamples.as<float4>(),
                                    c->dFrontDepth.as<float>(), workD, workX, workStk));
@@ -825,8 +829,8 @@ static SampleLaunch depth_launch(rh_ctx* c) {
     a.lists = c->dLists.as<uint32_t>(); a.mprec = c->dMprec.as<float>(); a.grids = c->dGrids.as<GridDev>();
     a.prims = c->dPrims.as<PrimDev>(); a.pos2d = c->dPos2d.as<float>(); a.pos1d = c->dPos1d.as<float>();
     a.pixPattern = c->dPix.as<uchar4>(); a.samples = c->dSamples.as<float4>(); a.hitData = c->dHitData.as<float4>();
-    a.hitNext = c->dHitNext.as<uint32_t>(); a.hitCounter = c->dHitCtl.as<uint32_t>();
-    a.combineList = c->dCombine.as<uint4>(); a.frontDepth = nullptr;
+    a.hitNext = c->dHitNext.as<uint2>(); a.hitCtl = c->dHitCtl.as<uint32_t>();
+    a.hitShards = c->dHitShards.as<uint32_t>(); a.hitHeads = nullptr; a.frontDepth = nullptr;
     a.rowCounts = c->dRows.as<uint32_t>(); a.rowBase = 0;
     a.idCut = 0xffffffffu; a.depthOnly = 1;
     // with the midpoint store the occluding depth is the second nearest
@@ -841,7 +845,8 @@ static hipError_t enqueue_depth_pass(rh_ctx* c, bool sample) {
     const rh::Shape& s = c->shape;
     const FrameDev* f = c->dFrame.as<FrameDev>();
     hipError_t e;
-    if ((e = rh_launch_frame_begin(c->st, c->dCounters.as<unsigned long long>(), c->dHitCtl.as<uint32_t>())) != hipSuccess)
+    if ((e = rh_launch_frame_begin(c->st, c->dCounters.as<unsigned long long>(), c->dHitCtl.as<uint32_t>(),
+                                   c->dHitShards.as<uint32_t>())) != hipSuccess)
         return e;
     if ((e = rh_launch_dice(c->st, f, c->dGrids.as<GridDev>(), (int)S.grids.size(), c->dPrims.as<PrimDev>(),
                             c->dParams.as<float>(), c->dMprec.as<float>(), c->dMpbound.as<float4>(),
@@ -1060,10 +1065,11 @@ static rh_status render_frame(rh_ctx* c, bool eager) {
         HIP_TRY(hipMemcpy(cnt, c->dCounters.p, sizeof(cnt), hipMemcpyDeviceToHost));
         uint32_t hc[4];
         HIP_TRY(hipMemcpy(hc, c->dHitCtl.p, sizeof(hc), hipMemcpyDeviceToHost));
-        if (hc[0] > c->frame.hitCapacity) {
+        if (hc[0] > 0) {
             // The arena ran out: redo the frame with room for every hit.
             if (attempt >= 2) return fail(RH_ERR_CAPACITY, "transparent-hit arena kept overflowing");
-            rh_status r = set_hit_capacity(c, (uint64_t)hc[0] + hc[0] / 4 + 64);
+            const uint64_t need = (uint64_t)c->frame.hitCapacity + hc[0];
+            rh_status r = set_hit_capacity(c, need + need / 4 + 64);
             if (r != RH_OK) return r;
             continue;
         }
@@ -1142,8 +1148,9 @@ rh_status rh_render_device_noalloc(rh_ctx* c) {
     uint32_t hc[4];
     HIP_TRY(hipMemcpy(cnt, k.counters, sizeof(cnt), hipMemcpyDeviceToHost));
     HIP_TRY(hipMemcpy(hc, k.hitCtl, sizeof(hc), hipMemcpyDeviceToHost));
-    if (hc[0] > c->frame.hitCapacity)
-        return fail(RH_ERR_CAPACITY, "the frame needs " + std::to_string(hc[0]) + " transparent-hit entries and the "
+    if (hc[0] > 0)
+        return fail(RH_ERR_CAPACITY, "the frame needs " + std::to_string((uint64_t)c->frame.hitCapacity + hc[0]) +
+                                         " transparent-hit entries and the "
                                      "context holds " + std::to_string(c->frame.hitCapacity) +
                                      " (rh_render_device grows the arena)");
     if (hc[1] != 0)
@@ -1416,7 +1423,8 @@ uint64_t rh_internal_device_bytes(const rh_ctx* c) {
                          &c->dFilter, &c->dBoxMask, &c->dGrids, &c->dParams, &c->dPrims, &c->dCandStart,
                          &c->dCandGrid, &c->dCapStart, &c->dSegBucket, &c->dSegCounts, &c->dMprec, &c->dMpbound, &c->dLists,
                          &c->dListCount, &c->dSamples, &c->dChannels, &c->dRgba, &c->dCounters,
-                         &c->dBucketRefs, &c->dHitData, &c->dHitNext, &c->dHitCtl, &c->dCombine, &c->dFrontDepth,
+                         &c->dBucketRefs, &c->dHitData, &c->dHitNext, &c->dHitCtl, &c->dHitShards, &c->dHitHeads,
+                         &c->dDeepList, &c->dFrontDepth,
                          &c->dItemsStatic, &c->dItems, &c->dItemCount, &c->dQueue, &c->dRows, &c->dMprecMB,
                          &c->dCullTrees, &c->dCullPyr, &c->dCullBounds, &c->dCullRanges, &c->dCullStart,
                          &c->dCullPairMax, &c->dProbeOut, &c->dProbeItems, &c->dProbeTasks, &c->dProbeCut,
@@ -1447,7 +1455,7 @@ static uint64_t footprint_bytes(const rh::Shape& s, const rh::Schedule& S, const
     for (int32_t i = 0; i < n; ++i)
         if (rh::hits_listed(s.o, prims[i])) transparent = true;
     if (transparent) {
-        // hit arena (24 B an entry), combine list and front depths
+        // hit arena (24 B an entry), list heads, deep list and front depths
         const uint64_t nsamp = (uint64_t)s.extW * s.extH * s.ns;
         bytes += arena_guess(s, S, prims) * 24 + nsamp * 20;
     }
