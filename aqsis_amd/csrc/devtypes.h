@@ -182,6 +182,22 @@ struct DofTables {
     const float4* cells;
 };
 
+// The strip filter's list (rh_filter_strip): the samples of a halo row that
+// add to a pixel, in the reference's order (filter columns, samples), in
+// groups of four of one column; ngroups is even, and two more groups follow.
+// An entry is RH_FILTER_ENTRY(ym) words: the sample's word offset from the
+// pixel's first staged column (int bits), then its weight for each fy + ym.
+// groups: a word each: the four samples' indices (6 bits each), the column
+// fx + xm (bits 24..26), whether a box test of theirs varies between pixels
+// (bit 31).  always: per fx, fy the samples (bits) whose test always holds.
+struct FilterDev {
+    const float* entries;
+    const uint32_t* groups;
+    int ngroups, nvary;                   // nvary: groups with bit 31
+    const uint2* always;
+};
+#define RH_FILTER_ENTRY(ym) ((ym) < 2 ? 4 : 8)
+
 // Sampling kernel variants: LDS chunk of CH records, SLOTS blocks per wave.
 #define RH_SAMPLE_VARIANTS 4
 #define RH_VARIANT_CH(v) ((v) < 2 ? 216 : 96)

@@ -42,12 +42,12 @@ extern "C" hipError_t rh_launch_combine(hipStream_t, const FrameDev*, size_t, co
                                         const GridDev*, int, float4*, float*);
 extern "C" hipError_t rh_launch_reduce_counters(hipStream_t, const uint32_t*, int, const uint32_t*, int,
                                                 unsigned long long*);
-extern "C" size_t rh_filter_tile_lds(int, int, int);
+extern "C" hipError_t rh_launch_box_classes(hipStream_t, const FrameDev*, int, const uchar4*, const float*, uint32_t*);
 extern "C" hipError_t rh_launch_box_masks(hipStream_t, const FrameDev*, size_t, const uchar4*, const float*,
-                                          uint16_t*);
+                                          uint2*);
 extern "C" hipError_t rh_launch_filter(hipStream_t, const FrameDev*, int, int, int, int, int, const float4*,
-                                       const uint16_t*, const uchar4*, const float*, const float*, const float*,
-                                       float*, uchar4*);
+                                       const uint2*, const FilterDev*, const uchar4*, const float*, const float*,
+                                       const float*, float*, uchar4*, int);
 extern "C" hipError_t rh_launch_cull_pyramid(hipStream_t, const FrameDev*, const CullTreeDev*, int, const float4*, float*);
 extern "C" hipError_t rh_launch_cull_pairs(hipStream_t, const CullTreeDev*, int, int, int, const float4*, const int4*,
                                            const unsigned long long*, int, unsigned long long, const float*, float*);
@@ -149,7 +149,10 @@ struct rh_ctx {
     // frame shape
     DBuf dFrame, dBuckets, dTasks, dPos2d, dPos1d, dPix, dDither, dFilter, dBoxMask;
     DBuf dShuffled, dLens, dPixDof, dDofCells;   // depth of field: lens tables (DofTables)
-    bool tiledFilter = false;
+    // the strip filter's list (FilterDev)
+    bool boxVaries = false;
+    int filtGroups = 0, filtVary = 0;
+    DBuf dFiltEntries, dFiltGroups, dFiltAlways;
     // schedule
     DBuf dGrids, dParams, dPrims, dCandStart, dCandGrid, dCapStart, dSegBucket, dSegCounts;
     // per frame
@@ -189,7 +192,7 @@ struct rh_ctx {
     }
     template <typename F> void each_buffer(F f) {
         DBuf* all[] = {&dFrame, &dBuckets, &dTasks, &dPos2d, &dPos1d, &dPix, &dDither, &dFilter, &dBoxMask,
-                       &dShuffled, &dLens, &dPixDof, &dDofCells,
+                       &dFiltEntries, &dFiltGroups, &dFiltAlways, &dShuffled, &dLens, &dPixDof, &dDofCells,
                        &dGrids, &dParams,
                        &dPrims, &dCandStart, &dCandGrid, &dCapStart, &dMprec, &dMpbound, &dLists,
                        &dListCount, &dSamples, &dChannels, &dRgba, &dCounters, &dBucketRefs,
@@ -344,6 +347,87 @@ hipError_t scratch_address(void** out) {
 }
 }  // namespace
 
+// The strip filter's lists, from the box tests of the frame shape's sample
+// positions: per filter column an entry for each sample that lies in the box
+// of some pixel there, in sample order, with weight 0 in the rows where its
+// test never holds.
+static hipError_t filter_lists(rh_ctx* c) {
+    const rh::Shape& s = c->shape;
+    const int ns = s.ns, xm = s.shiftX, ym = s.shiftY, rows = 2 * ym + 1, ent = RH_FILTER_ENTRY(ym);
+    const size_t nsamp = (size_t)s.extW * s.extH * ns;
+    const int wgs = (int)std::min<size_t>(512, nsamp / 256 + 1);
+    std::vector<uint32_t> cls((size_t)wgs * 64);
+    hipError_t e = c->dItems.ensure(cls.size() * sizeof(uint32_t));   // scratch until the work items are set up
+    if (e == hipSuccess)
+        e = rh_launch_box_classes(c->st, c->dFrame.as<FrameDev>(), wgs, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
+                                  c->dItems.as<uint32_t>());
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(cls.data(), c->dItems.p, cls.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
+    if (e != hipSuccess) return e;
+    std::vector<uint32_t> all(ns, 0xffffu), any(ns, 0u);
+    for (int w = 0; w < wgs; ++w)
+        for (int si = 0; si < ns; ++si) {
+            all[si] &= cls[(size_t)w * 64 + si] & 0xffffu;
+            any[si] |= cls[(size_t)w * 64 + si] >> 16;
+        }
+    std::vector<float> entries;
+    std::vector<uint32_t> groups;
+    std::vector<unsigned long long> always((size_t)(2 * xm + 1) * rows, 0ull);
+    c->boxVaries = false;
+    auto push = [&](int off) {
+        const size_t at = entries.size();
+        entries.resize(at + ent, 0.0f);
+        std::memcpy(&entries[at], &off, sizeof(off));
+        return at + 1;
+    };
+    for (int fx = 0; fx <= 2 * xm; ++fx) {
+        const int column = fx * 8 * (ns | 1);             // words to the column's staged pixel
+        int n = 0;
+        for (int si = 0; si < ns; ++si) {
+            size_t g = 0;
+            for (int r = 0; r < rows; ++r) {
+                const uint32_t need = (1u << fx) | (1u << (8 + r));
+                if ((any[si] & need) != need) continue;
+                if (g == 0) {
+                    g = push(column + si * 8);
+                    if (n % 4 == 0) groups.push_back((uint32_t)fx << 24);
+                    groups.back() |= (uint32_t)si << (6 * (n % 4));
+                    ++n;
+                }
+                entries[g + r] = s.filterTab[((size_t)r * (2 * xm + 1) + fx) * ns + si];
+                if ((all[si] & need) == need) {
+                    always[(size_t)fx * rows + r] |= 1ull << si;
+                } else {
+                    groups.back() |= 1u << 31;
+                    c->boxVaries = true;
+                }
+            }
+        }
+        for (; n % 4; ++n) push(column);                  // zero weights fill the column's last group
+    }
+    auto fill = [&] {
+        for (int k = 0; k < 4; ++k) push(0);
+        groups.push_back(0);
+    };
+    if (groups.size() % 2) fill();
+    c->filtGroups = (int)groups.size();
+    c->filtVary = (int)std::count_if(groups.begin(), groups.end(), [](uint32_t g) { return (g >> 31) != 0; });
+    fill();
+    fill();
+    if ((e = upload(c->dFiltEntries, entries, c->st)) != hipSuccess || (e = upload(c->dFiltGroups, groups, c->st)) != hipSuccess ||
+        (e = upload(c->dFiltAlways, always, c->st)) != hipSuccess)
+        return e;
+    if (c->boxVaries) {
+        const size_t npix = (size_t)s.extW * s.extH;
+        if ((e = c->dBoxMask.ensure(npix * (2 * xm + 1 + rows) * 8)) != hipSuccess) return e;
+        if ((e = rh_launch_box_masks(c->st, c->dFrame.as<FrameDev>(), npix, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
+                                     c->dBoxMask.as<uint2>())) != hipSuccess)
+            return e;
+    }
+    return hipStreamSynchronize(c->st);   // the lists' host copies end here
+}
+
 extern "C" {
 
 rh_status rh_create(const rh_options* opt, rh_ctx** out) {
@@ -435,18 +519,10 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
         delete c;
         return fail(e == hipErrorOutOfMemory ? RH_ERR_NOMEM : RH_ERR_DEVICE, std::string("device set-up: ") + hipGetErrorString(e));
     }
-    // The tiled filter reads each sample's box-test mask, fixed by the frame
-    // shape's sample positions.
-    c->tiledFilter = rh_filter_tile_lds(s.ns, s.shiftX, s.shiftY) != 0;
-    if (c->tiledFilter) {
-        const size_t nsamp = (size_t)s.extW * s.extH * s.ns;
-        if ((e = c->dBoxMask.ensure(nsamp * sizeof(uint16_t))) != hipSuccess ||
-            (e = rh_launch_box_masks(c->st, c->dFrame.as<FrameDev>(), nsamp, c->dPix.as<uchar4>(),
-                                     c->dPos2d.as<float>(), c->dBoxMask.as<uint16_t>())) != hipSuccess) {
-            delete c;
-            return fail(e == hipErrorOutOfMemory ? RH_ERR_NOMEM : RH_ERR_DEVICE,
-                        std::string("device set-up: ") + hipGetErrorString(e));
-        }
+    if ((e = filter_lists(c)) != hipSuccess) {
+        delete c;
+        return fail(e == hipErrorOutOfMemory ? RH_ERR_NOMEM : RH_ERR_DEVICE,
+                    std::string("device set-up: ") + hipGetErrorString(e));
     }
     // Work items: one per task for the static forms; up to one per block
     // for the batched form.
@@ -676,10 +752,13 @@ static FrameCtl context_ctl(rh_ctx* c) {
 // The filter + expose + quantise stage of a frame.
 static hipError_t enqueue_filter(rh_ctx* c) {
     const rh::Shape& s = c->shape;
+    const FilterDev fp{c->dFiltEntries.as<float>(), c->dFiltGroups.as<uint32_t>(), c->filtGroups, c->filtVary,
+                       c->dFiltAlways.as<uint2>()};
     return rh_launch_filter(c->st, c->dFrame.as<FrameDev>(), s.width(), s.height(), s.ns, s.shiftX, s.shiftY,
-                            c->dSamples.as<float4>(), c->tiledFilter ? c->dBoxMask.as<uint16_t>() : nullptr,
-                            c->dPix.as<uchar4>(), c->dPos2d.as<float>(), c->dFilter.as<float>(),
-                            c->dDither.as<float>(), c->dChannels.as<float>(), c->dRgba.as<uchar4>());
+                            c->dSamples.as<float4>(), c->boxVaries ? c->dBoxMask.as<uint2>() : nullptr,
+                            &fp, c->dPix.as<uchar4>(), c->dPos2d.as<float>(), c->dFilter.as<float>(),
+                            c->dDither.as<float>(), c->dChannels.as<float>(), c->dRgba.as<uchar4>(),
+                            c->frame.exposureGamma != 1.0f ? 1 : 0);
 }
 
 // Whether the combine takes its full form: a depth filter other than min, or
@@ -1420,7 +1499,8 @@ void rh_internal_trim_pool(uint64_t keep) { release_pool_memory(keep); }
 
 uint64_t rh_internal_device_bytes(const rh_ctx* c) {
     const DBuf* all[] = {&c->dFrame, &c->dBuckets, &c->dTasks, &c->dPos2d, &c->dPos1d, &c->dPix, &c->dDither,
-                         &c->dFilter, &c->dBoxMask, &c->dGrids, &c->dParams, &c->dPrims, &c->dCandStart,
+                         &c->dFilter, &c->dBoxMask, &c->dFiltEntries, &c->dFiltGroups, &c->dFiltAlways,
+                         &c->dGrids, &c->dParams, &c->dPrims, &c->dCandStart,
                          &c->dCandGrid, &c->dCapStart, &c->dSegBucket, &c->dSegCounts, &c->dMprec, &c->dMpbound, &c->dLists,
                          &c->dListCount, &c->dSamples, &c->dChannels, &c->dRgba, &c->dCounters,
                          &c->dBucketRefs, &c->dHitData, &c->dHitNext, &c->dHitCtl, &c->dHitShards, &c->dHitHeads,

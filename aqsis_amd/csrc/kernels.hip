@@ -19,9 +19,8 @@
 //   rh_combine          samples with transparent hits: depth sort as
 //                       std::sort, back-to-front compositing.
 //   rh_box_masks        per frame shape: each sample's filter-box tests.
-//   rh_filter_tiled     8x8-pixel tiles, halo in LDS: the filter gather,
-//                       exposure, quantise + dither (rh_filter: the general
-//                       thread-per-pixel form).
+//   rh_filter_strip     strips of 8 pixel columns, a halo row in LDS: the filter,
+//                       exposure, quantise + dither.
 //
 // All single-precision code is built with -ffp-contract=off and correctly
 // rounded division; every expression keeps the operand order of the aqsis
@@ -2664,6 +2663,9 @@ rh_combine_long(const FrameDev* __restrict__ fr, const uint2* __restrict__ heads
 // FilterBucket's tail (bucketprocessor.cpp:640-707), ExposeBucket
 // (bucketprocessor.cpp:766-806) and FormatBucketForDisplay
 // (ddmanager.cpp:1045-1118).  acc = weighted Ci.rgb, Oi.rgb, z.
+// GAMMA: the frame's gamma may be other than 1 (without, the registers of pow
+// are not taken).
+template <bool GAMMA>
 __device__ __forceinline__ void finish_pixel(const FrameDev* __restrict__ fr, const float* acc, float gTot, int count,
                                              int ns, size_t t, const float* __restrict__ dither,
                                              float* __restrict__ channels, uchar4* __restrict__ rgba8) {
@@ -2687,7 +2689,7 @@ __device__ __forceinline__ void finish_pixel(const FrameDev* __restrict__ fr, co
         float oog = 1.0f / gamma;
         for (int k = 0; k < 3; ++k) {
             if (gain != 1.0f) ch[k] *= gain;
-            if (gamma != 1.0f) ch[k] = (float)pow((double)ch[k], (double)oog);
+            if (GAMMA && gamma != 1.0f) ch[k] = (float)pow((double)ch[k], (double)oog);
         }
     }
     float* out = channels + t * 9;
@@ -2707,17 +2709,13 @@ __device__ __forceinline__ void finish_pixel(const FrameDev* __restrict__ fr, co
     rgba8[t] = make_uchar4(q[0], q[1], q[2], q[3]);
 }
 
-// General filter: one thread per display pixel, samples read straight from
-// HBM.  Used when a tile's halo does not fit the tiled kernel's LDS.
-// FilterBucket, non-separable branch (bucketprocessor.cpp:561-663).
-__global__ void __launch_bounds__(256) rh_filter(const FrameDev* __restrict__ fr, const float4* __restrict__ samples,
-                                                 const uchar4* __restrict__ pixPattern, const float* __restrict__ pos2d,
-                                                 const float* __restrict__ filterTab, const float* __restrict__ dither,
-                                                 float* __restrict__ channels, uchar4* __restrict__ rgba8) {
-    const int W = fr->cropX1 - fr->cropX0, H = fr->cropY1 - fr->cropY0;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= W * H) return;
-    const int x = fr->cropX0 + t % W, y = fr->cropY0 + t / W;
+// One display pixel by the reference's own loop, samples read straight from
+// HBM: FilterBucket, non-separable branch (bucketprocessor.cpp:561-663).
+template <bool GAMMA>
+__device__ __forceinline__ void filter_pixel(const FrameDev* __restrict__ fr, const float4* __restrict__ samples,
+                                             const uchar4* __restrict__ pixPattern, const float* __restrict__ pos2d,
+                                             const float* __restrict__ filterTab, const float* __restrict__ dither,
+                                             float* __restrict__ channels, uchar4* __restrict__ rgba8, int x, int y) {
     const int ns = fr->ns, xm = fr->shiftX, ym = fr->shiftY;
     const float xf = fr->xfwo2, yf = fr->yfwo2;
     const float xcent = x + 0.5f, ycent = y + 0.5f;
@@ -2746,23 +2744,18 @@ __global__ void __launch_bounds__(256) rh_filter(const FrameDev* __restrict__ fr
                 }
             }
         }
-    finish_pixel(fr, acc, gTot, count, ns, (size_t)t, dither, channels, rgba8);
+    const size_t t = (size_t)(y - fr->cropY0) * (fr->cropX1 - fr->cropX0) + (x - fr->cropX0);
+    finish_pixel<GAMMA>(fr, acc, gTot, count, ns, t, dither, channels, rgba8);
 }
 
-// Box-test masks of every sample of the extended region, once per frame
-// shape: bit (fx + xm) says that the sample of pixel qx lies inside the
-// filter box of pixel qx - fx (|position - pixel centre| <= ceil(width)/2,
-// bucketprocessor.cpp:600-612, evaluated exactly as the filter loop does),
-// bit (8 + fy + ym) the same for rows.
-__global__ void __launch_bounds__(256) rh_box_masks(const FrameDev* __restrict__ fr,
-                                                    const uchar4* __restrict__ pixPattern,
-                                                    const float* __restrict__ pos2d, uint16_t* __restrict__ masks) {
+// The box tests of one sample of the extended region: bit (fx + xm) says that
+// the sample of pixel qx lies inside the filter box of pixel qx - fx
+// (|position - pixel centre| <= ceil(width)/2, bucketprocessor.cpp:600-612,
+// evaluated exactly as the filter loop does), bit (8 + fy + ym) the same for
+// rows.
+__device__ __forceinline__ uint32_t box_tests(const FrameDev* __restrict__ fr, const uchar4* __restrict__ pixPattern,
+                                              const float* __restrict__ pos2d, size_t q, int si) {
     const int ns = fr->ns, xm = fr->shiftX, ym = fr->shiftY, extW = fr->extW;
-    const size_t n = (size_t)extW * fr->extH * ns;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const size_t q = t / ns;
-    const int si = (int)(t - q * ns);
     const int qx = fr->extX0 + (int)(q % extW), qy = fr->extY0 + (int)(q / extW);
     const int pat = pixPattern[q].x;
     const float sx = (float)qx + pos2d[2 * (pat * ns + si)];
@@ -2779,185 +2772,356 @@ __global__ void __launch_bounds__(256) rh_box_masks(const FrameDev* __restrict__
         const float vy = sy - ycent;
         if (vy >= -yf && vy <= yf) mask |= 1u << (8 + fy + ym);
     }
-    masks[t] = (uint16_t)mask;
+    return mask;
 }
 
-// Tiled filter.  One workgroup per RH_FT x RH_FT tile of display pixels,
-// four waves over the channels: wave 0 sums Ci.r and Ci.g (with the weight
-// total and the count), wave 1 Ci.b and z, wave 2 Oi.r and Oi.g, wave 3
-// Oi.b; each lane one pixel, each sum in the reference's order (filter rows,
-// filter columns, samples), so the split changes no rounding.  The tile's halo of samples is
-// staged in LDS once, with RH_FU coalesced loads in flight per lane, as 8
-// dwords per sample: Ci.rgb, z, Oi.rgb and a word holding the sample's
-// box-test mask (bits 0..15) and whether it holds a surface (bit 31).  Halo
-// pixel records are 8*ns+RH_FPAD dwords apart so that the lanes of a wave read
-// different LDS banks.
-#define RH_FT 8
-#define RH_FU 16
-#define RH_FTHREADS 256
-#ifndef RH_FPAD
-#define RH_FPAD 1
-#endif
-
-// The weighted sums of one pixel over its filter footprint, in the
-// reference's order (filter rows, filter columns, samples): NC channels
-// starting at `rec0` of each staged sample record (8 words apart), the
-// sample's mask word at offset `mw`.  A sample outside the pixel's box adds
-// nothing, one inside adds its weight to gTot, and one holding a surface also
-// adds weight x value to each channel sum (gTot and count only with TOT).
-// The adds are unconditional with the weight zeroed where the reference
-// skips: x + 0 * v == x exactly, since the sums start at +0 and never become
-// -0.  Weights are read with uniform (scalar) loads.
-template <int NC, bool TOT>
-__device__ __forceinline__ void filter_taps(const float* __restrict__ rec0, const float* __restrict__ filterTab,
-                                            int ns, int xm, int ym, int HX, int S, int lx, int ly, int mw,
-                                            float* acc, float& gTot, int& count) {
-    for (int fy = -ym; fy <= ym; ++fy)
-        for (int fx = -xm; fx <= xm; ++fx) {
-            const float* rec = rec0 + ((ly + fy + ym) * HX + (lx + fx + xm)) * S;
-            const float* wt = filterTab + ((fy + ym) * (2 * xm + 1) + fx + xm) * ns;
-            const uint32_t need = (1u << (fx + xm)) | (1u << (8 + fy + ym));
-            // four samples at a time, every LDS read issued first
-            int si = 0;
-            for (; si + 4 <= ns; si += 4) {
-                uint32_t m[4];
-                float d[4][NC];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float* r = rec + (si + q) * 8;
-                    m[q] = __float_as_uint(r[mw]);
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) d[q][c] = r[c];
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const bool in = (m[q] & need) == need;
-                    const bool hit = in && (m[q] >> 31);
-                    const float g = wt[si + q];
-                    const float ghit = hit ? g : 0.0f;
-                    if (TOT) {
-                        gTot = gTot + (in ? g : 0.0f);
-                        count += hit ? 1 : 0;
-                    }
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) acc[c] = acc[c] + d[q][c] * ghit;
-                }
-            }
-            for (; si < ns; ++si) {
-                const float* r = rec + si * 8;
-                const uint32_t mm = __float_as_uint(r[mw]);
-                const bool in = (mm & need) == need;
-                const bool hit = in && (mm >> 31);
-                const float g = wt[si];
-                const float ghit = hit ? g : 0.0f;
-                if (TOT) {
-                    gTot = gTot + (in ? g : 0.0f);
-                    count += hit ? 1 : 0;
-                }
-#pragma unroll
-                for (int c = 0; c < NC; ++c) acc[c] = acc[c] + r[c] * ghit;
-            }
+// Once per frame shape: for each sample index of a pixel, the box tests that
+// hold in every pixel of the extended region (low 16 bits) and those that
+// hold in any (high 16 bits); one row of 64 words per workgroup, for the host
+// to merge.  A thread's stride is a multiple of ns, so it sees one index.
+__global__ void __launch_bounds__(256) rh_box_classes(const FrameDev* __restrict__ fr,
+                                                      const uchar4* __restrict__ pixPattern,
+                                                      const float* __restrict__ pos2d, uint32_t* __restrict__ rows) {
+    __shared__ uint32_t all[64], any[64];
+    const int ns = fr->ns;
+    if (threadIdx.x < 64) {
+        all[threadIdx.x] = 0xffffu;
+        any[threadIdx.x] = 0u;
+    }
+    __syncthreads();
+    const size_t n = (size_t)fr->extW * fr->extH * ns;
+    const size_t stride = (size_t)gridDim.x * 256 / ns * ns;
+    size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (t < stride) {
+        const int si = (int)(t % ns);
+        uint32_t a = 0xffffu, o = 0u;
+        for (; t < n; t += stride) {
+            const uint32_t m = box_tests(fr, pixPattern, pos2d, t / ns, si);
+            a &= m;
+            o |= m;
         }
+        atomicAnd(&all[si], a);
+        atomicOr(&any[si], o);
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) rows[blockIdx.x * 64 + threadIdx.x] = all[threadIdx.x] | (any[threadIdx.x] << 16);
 }
-__global__ void __launch_bounds__(RH_FTHREADS) rh_filter_tiled(const FrameDev* __restrict__ fr,
-                                                       const float4* __restrict__ samples,
-                                                       const uint16_t* __restrict__ boxMask,
-                                                       const float* __restrict__ filterTab,
-                                                       const float* __restrict__ dither, float* __restrict__ channels,
-                                                       uchar4* __restrict__ rgba8, int tilesX, int ntiles) {
-    // LDS: halo records (RH_FT+2*xm)*(RH_FT+2*ym)*(8*ns+RH_FPAD) floats; the
-    // tail exchange reuses the first 320 floats.
-    extern __shared__ float lds[];
-    // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a
-    // contiguous run of tiles so neighbouring tiles share halos in its L2.
+
+// A pixel's box tests as bits by sample, for a frame shape where some vary:
+// 2*xm+1 words of the column tests (bit si: sample si lies within the box of
+// the pixel at -fx), then 2*ym+1 of the row tests.  One thread a pixel.
+__global__ void __launch_bounds__(256) rh_box_masks(const FrameDev* __restrict__ fr,
+                                                    const uchar4* __restrict__ pixPattern,
+                                                    const float* __restrict__ pos2d,
+                                                    uint2* __restrict__ masks) {
+    const int ns = fr->ns, nx = 2 * fr->shiftX + 1, ny = 2 * fr->shiftY + 1;
+    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= (size_t)fr->extW * fr->extH) return;
+    uint2* out = masks + q * (nx + ny);
+    for (int k = 0; k < nx + ny; ++k) out[k] = make_uint2(0u, 0u);
+    for (int si = 0; si < ns; ++si) {
+        const uint32_t m = box_tests(fr, pixPattern, pos2d, q, si);
+        for (int k = 0; k < nx + ny; ++k) {
+            const uint32_t b = (k < nx ? m >> k : m >> (8 + k - nx)) & 1u;
+            if (si < 32) out[k].x |= b << si;
+            else out[k].y |= b << (si - 32);
+        }
+    }
+}
+
+// The strip filter.  Each wave takes a strip of RH_FS_W x R display pixels and
+// walks down its halo rows: a row of RH_FS_W + 2*xm pixels' samples is staged in
+// LDS as 8 words a sample (Ci.rgb, z, Oi.rgb, 1), the next row's loads in
+// flight meanwhile, and every staged sample is added to the 2*YM+1 pixel rows
+// it contributes to.  A lane is one pixel column and one of the 8 words, so
+// each sum is taken by one lane in the reference's order (filter rows,
+// columns, samples): halo row hy gives row y its terms of fy = hy - y, rows
+// come in ascending order, and per row the columns and samples do.  The word
+// 1 sums the weights.
+//
+// Bound by vector issue (a multiplication and an addition a term: no
+// contraction; 134M wave instructions, 76% of the issue slots, at 1920x1080,
+// 4x4 samples, catmull-rom 3x3), then by HBM (each sample read once and its
+// halo).  So the per-sample tests are taken out of the loop: whether sample
+// si of a pixel lies in the box of the pixel at (-fx, -fy) is the same for
+// nearly every pixel of a frame shape (always for odd widths; for even ones
+// up to the rounding of positions at the box's edge), so the host makes one
+// list of the samples of a halo row with their weights from rh_box_classes,
+// without those whose test never holds, and in a group of four where some
+// test varies the weights are and-ed with the pixel's own tests
+// (rh_box_masks).  A sample that holds no surface is staged as zeros:
+// x + 0 * w is x, as the sums start at +0 and never become -0.  Both need
+// finite values: a wave that staged an infinity or NaN takes its pixels again
+// by filter_pixel, the reference's loop.
+//
+// 8 columns: 16 of two words a lane take 8% fewer instructions and leave 3
+// waves a SIMD instead of 4 (315 against 287 us at the frame above).  LOADS,
+// the samples a lane has in flight: a halo row of up to 32 samples a pixel in
+// one go at 5, of 64 at 10 (1075 to 958 us at 1024x1024, 8x8 samples).
+// Measured against 8x8-pixel tiles with their halo in LDS and the tests in
+// the loop, or (8x8 samples: a tile's halo does not fit) a thread a pixel
+// reading HBM: 633 to 287 us at the frame above, 1238 to 644 at 2048x2048,
+// 4x4, gaussian 2x2, 5297 to 958 at 1024x1024, 8x8, 254 to 118 at 256x256,
+// 8x8.
+#define RH_FS_W 8             // pixel columns of a strip
+// 64-word loads of a halo row's masks: at most 14 pixels of 14 words
+#define RH_FS_MASKS 4
+#define RH_FS_OUT 9           // words of a finished pixel: the 8 sums, the hit count
+
+template <int YM, int LOADS, bool VARIES, bool GAMMA>
+__global__ void __launch_bounds__(64) rh_filter_strip(const FrameDev* __restrict__ fr,
+                                                      const float4* __restrict__ samples,
+                                                      const uint2* __restrict__ boxMask,
+                                                      const float* __restrict__ entries,
+                                                      const uint32_t* __restrict__ groups, int ngroups,
+                                                      const uint2* __restrict__ always,
+                                                      const uchar4* __restrict__ pixPattern,
+                                                      const float* __restrict__ pos2d,
+                                                      const float* __restrict__ filterTab,
+                                                      const float* __restrict__ dither, float* __restrict__ channels,
+                                                      uchar4* __restrict__ rgba8, int tilesX, int ntiles, int R) {
+    constexpr int ROWS = 2 * YM + 1;      // pixel rows a halo row contributes to
+    constexpr int ENT = RH_FILTER_ENTRY(YM);
+    constexpr int FLUSH = 64 / RH_FS_W;        // pixel rows finished together
+    extern __shared__ float4 lds4[];
+    const int ns = fr->ns, xm = fr->shiftX;
+    const int HX = RH_FS_W + 2 * xm, S = 8 * (ns | 1), total = HX * ns;
+    constexpr int HW = LOADS > 5 ? 2 : 1; // 32-bit words of a pixel's sample bits
+    const int nwords = (total >> 5) + 4;
+    float* rec = reinterpret_cast<float*>(lds4);
+    float* outS = rec + HX * S;
+    uint32_t* hitw = reinterpret_cast<uint32_t*>(outS + 64 * RH_FS_OUT);
+    uint2* mk = reinterpret_cast<uint2*>(hitw + (nwords & ~1));
+    const int mw = 2 * xm + 1 + ROWS, mkWords = VARIES && boxMask ? HX * mw : 0;   // mask words of a halo row
+    // Workgroups are dealt round-robin to the 8 XCDs; each XCD gets a
+    // contiguous run of strips, so that neighbours share halos in its L2.
     // The grid is a multiple of 8 workgroups.
     const int per = gridDim.x >> 3;
     const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (tile >= ntiles) return;
-    const int ns = fr->ns, xm = fr->shiftX, ym = fr->shiftY;
-    const int extX0 = fr->extX0, extY0 = fr->extY0, extW = fr->extW, extH = fr->extH;
-    const int tx0 = fr->cropX0 + (tile % tilesX) * RH_FT, ty0 = fr->cropY0 + (tile / tilesX) * RH_FT;
-    const int HX = RH_FT + 2 * xm, HY = RH_FT + 2 * ym, NH = HX * HY;
-    const int S = 8 * ns + RH_FPAD;
-    const int tid = threadIdx.x;
+    const int lane = threadIdx.x;
+    const int extX0 = fr->extX0, extY0 = fr->extY0, extW = fr->extW;
+    const int x0 = fr->cropX0 + (tile % tilesX) * RH_FS_W, y0 = fr->cropY0 + (tile / tilesX) * R;
+    const int rows = min(R, fr->cropY1 - y0), steps = rows + 2 * YM;
+    const int col = lane % RH_FS_W, word = lane / RH_FS_W;
+    // A halo row's samples are contiguous.  A row reaching past the extended
+    // region (columns beyond the crop window, which no pixel reads) loads its
+    // last sample in their place.
+    const int rowMax = min(HX, extX0 + extW - (x0 - xm)) * ns;
+    const size_t q0 = (size_t)(y0 - YM - extY0) * extW + (x0 - xm - extX0);
+    const char* rowPtr = reinterpret_cast<const char*>(samples + 2 * q0 * ns);
+    const int maskMax = rowMax / ns * mw;
+    const size_t rowBytes = (size_t)extW * ns * 32;
+    const uint2* maskPtr = boxMask + (VARIES && boxMask ? q0 * mw : 0);
+    const uint32_t nsLo = ns >= 32 ? ~0u : (1u << ns) - 1u, nsHi = ns >= 64 ? ~0u : (ns > 32 ? (1u << (ns - 32)) - 1u : 0u);
 
-    // 1. Stage the halo's sample records (2 float4 per sample) and masks.
-    {
-        const int per_px = 2 * ns, total = NH * per_px;
-        const int dhp = RH_FTHREADS / per_px, dpart = RH_FTHREADS % per_px;
-        int hp = tid / per_px, part = tid % per_px;
-        int hy = hp / HX, hx = hp % HX;
-        for (int base = 0; base < total; base += RH_FTHREADS * RH_FU) {
-            float4 v[RH_FU];
-            uint32_t mk[RH_FU];
-            int dst[RH_FU];
+    float4 va[LOADS], vb[LOADS];
+    uint2 vm[RH_FS_MASKS];
+    int dst[LOADS];                 // where the lane's first samples go in rec
+    uint32_t src[LOADS];            // and their byte offsets in the row
 #pragma unroll
-            for (int u = 0; u < RH_FU; ++u) {
-                const int i = base + u * RH_FTHREADS + tid;
-                v[u] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(0xffffffffu));
-                mk[u] = 0;
-                dst[u] = -1;
-                if (i < total) {
-                    const int qx = tx0 - xm + hx, qy = ty0 - ym + hy;
-                    dst[u] = (hp * S + part * 4) * 2 + (part & 1);
-                    if (qx >= extX0 && qx < extX0 + extW && qy >= extY0 && qy < extY0 + extH) {
-                        const size_t q = (size_t)(qy - extY0) * extW + (qx - extX0);
-                        v[u] = samples[q * per_px + part];
-                        if (part & 1) mk[u] = boxMask[q * ns + (part >> 1)];
-                    }
-                }
-                part += dpart;
-                int adv = dhp;
-                if (part >= per_px) { part -= per_px; ++adv; }
-                hp += adv;
-                hx += adv;
-                while (hx >= HX) { hx -= HX; ++hy; }
+    for (int u = 0; u < LOADS; ++u) {
+        const int i = u * 64 + lane, px = i / ns;
+        dst[u] = px * S + (i - px * ns) * 8;
+        src[u] = (uint32_t)min(i, rowMax - 1) * 32u;
+    }
+    auto load = [&](int first) {
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) {
+            if (first + u * 64 >= total) break;        // uniform
+            const uint32_t at = first ? (uint32_t)min(first + u * 64 + lane, rowMax - 1) * 32u : src[u];
+            const float4* p = reinterpret_cast<const float4*>(rowPtr + at);
+            va[u] = p[0];
+            vb[u] = p[1];
+        }
+        if (VARIES && first == 0)
+#pragma unroll
+            for (int u = 0; u < RH_FS_MASKS; ++u)
+                if (u * 64 + lane < mkWords) vm[u] = maskPtr[min(u * 64 + lane, maskMax - 1)];
+    };
+    float nonFinite = 0.0f;               // becomes NaN
+    bool allHit = true;
+    auto store = [&](int first) {
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) {
+            const int i = first + u * 64 + lane;
+            if (first + u * 64 >= total) break;        // uniform
+            const bool hit = __float_as_uint(vb[u].w) != 0xffffffffu;
+            const unsigned long long hm = __ballot(hit);
+            if (lane == 0) {
+                hitw[(first >> 5) + 2 * u] = (uint32_t)hm;
+                hitw[(first >> 5) + 2 * u + 1] = (uint32_t)(hm >> 32);
             }
-#pragma unroll
-            for (int u = 0; u < RH_FU; ++u) {
-                if (dst[u] < 0) continue;
-                float* d = lds + (dst[u] >> 1);
-                d[0] = v[u].x;
-                d[1] = v[u].y;
-                d[2] = v[u].z;
-                d[3] = (dst[u] & 1) ? __uint_as_float(mk[u] | ((__float_as_uint(v[u].w) != 0xffffffffu) ? 0x80000000u : 0u))
-                                    : v[u].w;
+            float4 a = va[u], b = vb[u];
+            if (hm != ~0ull) {
+                allHit = allHit && !__ballot(!hit && i < total);
+                if (!hit) a = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (!hit) b = a;
+            }
+            b.w = 1.0f;
+            nonFinite = fmaf(a.x, 0.f, nonFinite); nonFinite = fmaf(a.y, 0.f, nonFinite);
+            nonFinite = fmaf(a.z, 0.f, nonFinite); nonFinite = fmaf(a.w, 0.f, nonFinite);
+            nonFinite = fmaf(b.x, 0.f, nonFinite); nonFinite = fmaf(b.y, 0.f, nonFinite);
+            nonFinite = fmaf(b.z, 0.f, nonFinite);
+            if (i < total) {
+                int at = dst[u];
+                if (first) {
+                    const int px = i / ns;
+                    at = px * S + (i - px * ns) * 8;
+                }
+                float4* d = reinterpret_cast<float4*>(rec + at);
+                d[0] = a;
+                d[1] = b;
             }
         }
+        if (VARIES && first == 0)
+#pragma unroll
+            for (int u = 0; u < RH_FS_MASKS; ++u)
+                if (u * 64 + lane < mkWords) mk[u * 64 + lane] = vm[u];
+    };
+
+    float acc[ROWS];
+    int cnt[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        cnt[r] = 0;
+        acc[r] = 0.0f;
     }
-    __syncthreads();
-    // 2. Weighted sums, one lane per pixel per wave's channels.
-    const int lane = tid & 63, part = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lx = lane & (RH_FT - 1), ly = lane / RH_FT;
-    const int x = tx0 + lx, y = ty0 + ly;
-    const bool valid = x < fr->cropX1 && y < fr->cropY1;
-    float gTot = 0.0f;
-    int count = 0;
-    float acc[2] = {0.0f, 0.0f};
-    if (valid) {
-        // record words: Ci.rgb, z, Oi.rgb, mask
-        if (part == 0) filter_taps<2, true>(lds, filterTab, ns, xm, ym, HX, S, lx, ly, 7, acc, gTot, count);
-        else if (part == 1) filter_taps<2, false>(lds + 2, filterTab, ns, xm, ym, HX, S, lx, ly, 5, acc, gTot, count);
-        else if (part == 2) filter_taps<2, false>(lds + 4, filterTab, ns, xm, ym, HX, S, lx, ly, 3, acc, gTot, count);
-        else filter_taps<1, false>(lds + 6, filterTab, ns, xm, ym, HX, S, lx, ly, 1, acc, gTot, count);
+    int allIn[ROWS];                      // the count where every sample holds a surface
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        allIn[r] = 0;
+        for (int fx = 0; fx <= 2 * xm; ++fx) allIn[r] += __popc(always[fx * ROWS + r].x) + __popc(always[fx * ROWS + r].y);
     }
-    __syncthreads();                  // the halo records are no longer read
-    // waves 1..3 hand their sums to wave 0: Ci.b, z, Oi.r, Oi.g, Oi.b
-    if (part == 1) {
-        lds[lane * 5 + 0] = acc[0];
-        lds[lane * 5 + 1] = acc[1];
-    } else if (part == 2) {
-        lds[lane * 5 + 2] = acc[0];
-        lds[lane * 5 + 3] = acc[1];
-    } else if (part == 3) {
-        lds[lane * 5 + 4] = acc[0];
+    load(0);
+    for (int step = 0; step < steps; ++step) {
+        // 1. this halo row into LDS, the next row's first loads issued
+        allHit = true;
+        store(0);
+        for (int first = LOADS * 64; first < total; first += LOADS * 64) {
+            load(first);
+            store(first);
+        }
+        rowPtr += rowBytes;
+        if (VARIES) maskPtr += (size_t)(boxMask ? extW * mw : 0);
+        if (step + 1 < steps) load(0);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // 2. its terms, four samples at a time: the next four's LDS reads and
+        // the weights after them are in flight meanwhile
+        const float* base = rec + col * S + word;
+        float e[3][4 * ENT], d[2][4];
+        auto weights = [&](int g, float* w) {
+#pragma unroll
+            for (int k = 0; k < 4 * ENT; ++k) w[k] = entries[(size_t)g * (4 * ENT) + k];
+        };
+        auto values = [&](const float* w, float* v) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = base[__float_as_int(w[q * ENT])];
+        };
+        auto add = [&](int g, const float* w, const float* v) {
+            const uint32_t info = VARIES ? groups[g] : 0u;
+            if (VARIES && (info >> 31)) {
+                // some test of the four varies: weights and-ed with the pixel's tests
+                const int fx = (int)(info >> 24) & 7;
+                const uint2* m = mk + (col + fx) * mw;
+                const uint2 mx = m[fx];
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    const uint2 my = m[2 * xm + 1 + r];
+                    const uint32_t lo = mx.x & my.x, hi = HW > 1 ? mx.y & my.y : 0u;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const uint32_t si = (info >> (6 * q)) & 63u;
+                        const uint32_t h = HW > 1 && si >= 32u ? hi : lo;
+                        const int keep = __builtin_amdgcn_sbfe((int)h, si & 31u, 1u);   // all ones: in the box
+                        const float gq = __int_as_float(__float_as_int(w[q * ENT + 1 + r]) & keep);
+                        acc[r] = acc[r] + v[q] * gq;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int r = 0; r < ROWS; ++r) acc[r] = acc[r] + v[q] * w[q * ENT + 1 + r];
+            }
+        };
+        weights(0, e[0]);
+        weights(1, e[1]);
+        values(e[0], d[0]);
+        // (the list is a multiple of two groups and has two more behind it)
+        for (int g = 0; g < ngroups; g += 2) {
+            weights(g + 2, e[2]);
+            values(e[1], d[1]);
+            add(g, e[0], d[0]);
+#pragma unroll
+            for (int k = 0; k < 4 * ENT; ++k) e[0][k] = e[2][k];
+            weights(g + 3, e[2]);
+            values(e[0], d[0]);
+            add(g + 1, e[1], d[1]);
+#pragma unroll
+            for (int k = 0; k < 4 * ENT; ++k) e[1][k] = e[2][k];
+        }
+        // the surface samples in the box of each pixel row
+        if (!VARIES && allHit) {
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) cnt[r] += allIn[r];
+        } else {
+            for (int fx = 0; fx <= 2 * xm; ++fx) {
+                const int at = (col + fx) * ns, w = at >> 5, sh = at & 31;
+                uint32_t lo = __builtin_amdgcn_alignbit(hitw[w + 1], hitw[w], sh) & nsLo;
+                uint32_t hi = HW > 1 ? __builtin_amdgcn_alignbit(hitw[w + 2], hitw[w + 1], sh) & nsHi : 0u;
+                const uint2* m = mk + (col + fx) * mw;
+                const bool own = VARIES && boxMask;
+                if (own) {
+                    lo &= m[fx].x;
+                    hi &= m[fx].y;
+                }
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    const uint2 t = own ? m[2 * xm + 1 + r] : always[fx * ROWS + r];
+                    cnt[r] += __popc(lo & t.x);
+                    if (HW > 1) cnt[r] += __popc(hi & t.y);
+                }
+            }
+        }
+        // 3. the pixel row that is complete: y = hy - YM
+        const int done = step - 2 * YM;
+        if (done >= 0) {
+            float* o = outS + ((done % FLUSH) * RH_FS_W + col) * RH_FS_OUT;
+            o[word] = acc[ROWS - 1];
+            if (word == 0) o[8] = __int_as_float(cnt[ROWS - 1]);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (done % FLUSH == FLUSH - 1 || done == rows - 1) {
+                const int r0 = done - done % FLUSH, y = y0 + r0 + lane / RH_FS_W, x = x0 + lane % RH_FS_W;
+                if (r0 + lane / RH_FS_W <= done && x < fr->cropX1) {
+                    const float* v = outS + lane * RH_FS_OUT;
+                    const float full[7] = {v[0], v[1], v[2], v[4], v[5], v[6], v[3]};
+                    const size_t t = (size_t)(y - fr->cropY0) * (fr->cropX1 - fr->cropX0) + (x - fr->cropX0);
+                    finish_pixel<GAMMA>(fr, full, v[7], __float_as_int(v[8]), ns, t, dither, channels, rgba8);
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int r = ROWS - 1; r > 0; --r) {
+            cnt[r] = cnt[r - 1];
+            acc[r] = acc[r - 1];
+        }
+        cnt[0] = 0;
+        acc[0] = 0.0f;
     }
-    __syncthreads();
-    if (part == 0 && valid) {
-        const float full[7] = {acc[0], acc[1], lds[lane * 5 + 0], lds[lane * 5 + 2], lds[lane * 5 + 3],
-                               lds[lane * 5 + 4], lds[lane * 5 + 1]};
-        const size_t t = (size_t)(y - fr->cropY0) * (fr->cropX1 - fr->cropX0) + (x - fr->cropX0);
-        finish_pixel(fr, full, gTot, count, ns, t, dither, channels, rgba8);
+    if (__ballot(nonFinite != 0.0f)) {
+        for (int p = lane; p < rows * RH_FS_W; p += 64) {
+            const int x = x0 + p % RH_FS_W, y = y0 + p / RH_FS_W;
+            if (x < fr->cropX1)
+                filter_pixel<GAMMA>(fr, samples, pixPattern, pos2d, filterTab, dither, channels, rgba8, x, y);
+        }
     }
 }
 
@@ -3323,40 +3487,62 @@ extern "C" hipError_t rh_launch_reduce_counters(hipStream_t st, const uint32_t* 
                        counters);
     return hipGetLastError();
 }
-// LDS bytes of one tiled-filter workgroup, or 0 if the tiled kernel cannot
-// take this frame shape (mask bits or LDS size exceeded).
-extern "C" size_t rh_filter_tile_lds(int ns, int xm, int ym) {
-    if (2 * xm + 1 > 8 || 2 * ym + 1 > 8) return 0;
-    const size_t bytes = (size_t)(RH_FT + 2 * xm) * (RH_FT + 2 * ym) * (8 * ns + RH_FPAD) * sizeof(float);
-    return bytes <= 64 * 1024 ? bytes : 0;
+extern "C" hipError_t rh_launch_box_classes(hipStream_t st, const FrameDev* fr, int workgroups,
+                                            const uchar4* pixPattern, const float* pos2d, uint32_t* rows) {
+    hipLaunchKernelGGL(rh_box_classes, dim3(workgroups), dim3(256), 0, st, fr, pixPattern, pos2d, rows);
+    return hipGetLastError();
 }
 
-extern "C" hipError_t rh_launch_box_masks(hipStream_t st, const FrameDev* fr, size_t nsamples,
-                                          const uchar4* pixPattern, const float* pos2d, uint16_t* masks) {
-    if (nsamples == 0) return hipSuccess;
-    hipLaunchKernelGGL(rh_box_masks, dim3((unsigned)((nsamples + 255) / 256)), dim3(256), 0, st, fr, pixPattern,
+extern "C" hipError_t rh_launch_box_masks(hipStream_t st, const FrameDev* fr, size_t npixels,
+                                          const uchar4* pixPattern, const float* pos2d, uint2* masks) {
+    if (npixels == 0) return hipSuccess;
+    hipLaunchKernelGGL(rh_box_masks, dim3((unsigned)((npixels + 255) / 256)), dim3(256), 0, st, fr, pixPattern,
                        pos2d, masks);
     return hipGetLastError();
 }
 
-// boxMask: the frame shape's masks from rh_launch_box_masks, or null when
-// rh_filter_tile_lds is 0 for it (then the general kernel runs).
+template <int YM, int LOADS>
+static void launch_filter_t(hipStream_t st, const FrameDev* fr, int width, int height, int ns, int xm,
+                            const float4* samples, const uint2* boxMask, const FilterDev& fp,
+                            const uchar4* pixPattern, const float* pos2d, const float* filterTab, const float* dither,
+                            float* channels, uchar4* rgba8, bool gamma) {
+    const int tilesX = (width + RH_FS_W - 1) / RH_FS_W;
+    // Rows a strip: the halo costs (R + 2*YM) / R, so as many as leave the
+    // device 4096 waves, 16 a CU (512x512, 4x4 samples: 60 us at 4096, 77 at
+    // 2048, 134 at 1024); half of that where most tests vary, as a row costs
+    // more there (317x211, 3x3 samples: 37 us at 4096, 31 at 2048).
+    const size_t waves = 2 * fp.nvary > fp.ngroups ? 2048 : 4096;
+    int R = 32;
+    while (R > 1 && (size_t)tilesX * ((height + R - 1) / R) < waves) R >>= 1;
+    const int ntiles = tilesX * ((height + R - 1) / R);
+    const size_t HX = RH_FS_W + 2 * xm, total = HX * ns;
+    const size_t lds = (HX * 8 * (ns | 1) + 64 * RH_FS_OUT) * sizeof(float) + ((total / 32 + 4) & ~size_t(1)) * 4 +
+                       (boxMask ? HX * (2 * xm + 1 + 2 * YM + 1) * 8 : 0);
+    auto* k = gamma ? &rh_filter_strip<YM, LOADS, true, true>
+                    : (boxMask ? &rh_filter_strip<YM, LOADS, true, false> : &rh_filter_strip<YM, LOADS, false, false>);
+    hipLaunchKernelGGL(k, dim3((ntiles + 7) / 8 * 8), dim3(64), lds, st, fr, samples, boxMask, fp.entries, fp.groups,
+                       fp.ngroups, fp.always, pixPattern, pos2d, filterTab, dither, channels, rgba8, tilesX, ntiles,
+                       R);
+}
+
+template <int YM>
+static auto filter_form(int ns) {
+    return ns > 32 ? &launch_filter_t<YM, 10> : &launch_filter_t<YM, 5>;
+}
+
+// fp: the frame shape's filter list; boxMask: its box tests when some vary,
+// else null; gamma: the frame's gamma is not 1.  A pixel's sample bits are two
+// words and its box tests 7 columns and rows: at most 64 samples a pixel and
+// 3 pixels of halo a side, the limits of a frame shape.
 extern "C" hipError_t rh_launch_filter(hipStream_t st, const FrameDev* fr, int width, int height, int ns, int xm,
-                                       int ym, const float4* samples, const uint16_t* boxMask,
+                                       int ym, const float4* samples, const uint2* boxMask, const FilterDev* fp,
                                        const uchar4* pixPattern, const float* pos2d, const float* filterTab,
-                                       const float* dither, float* channels, uchar4* rgba8) {
+                                       const float* dither, float* channels, uchar4* rgba8, int gamma) {
     const int npix = width * height;
     if (npix <= 0) return hipSuccess;
-    const size_t lds = boxMask ? rh_filter_tile_lds(ns, xm, ym) : 0;
-    if (lds) {
-        const int tilesX = (width + RH_FT - 1) / RH_FT, tilesY = (height + RH_FT - 1) / RH_FT;
-        const int ntiles = tilesX * tilesY;
-        const int per = (ntiles + 7) / 8;
-        hipLaunchKernelGGL(rh_filter_tiled, dim3(8 * per), dim3(RH_FTHREADS), lds, st, fr, samples, boxMask, filterTab,
-                           dither, channels, rgba8, tilesX, ntiles);
-    } else {
-        hipLaunchKernelGGL(rh_filter, dim3((npix + 255) / 256), dim3(256), 0, st, fr, samples, pixPattern, pos2d,
-                           filterTab, dither, channels, rgba8);
-    }
+    if (ns > 64 || xm > 3 || ym > 3) return hipErrorInvalidValue;
+    auto* f = ym == 0 ? filter_form<0>(ns) : (ym == 1 ? filter_form<1>(ns) : (ym == 2 ? filter_form<2>(ns) : filter_form<3>(ns)));
+    f(st, fr, width, height, ns, xm, samples, boxMask, *fp, pixPattern, pos2d, filterTab, dither, channels, rgba8,
+      gamma != 0);
     return hipGetLastError();
 }
