@@ -291,9 +291,21 @@ bool make_shape(const rh_options& o, Shape& s, std::string& err) {
         s.blockH = 1;
     }
     // Tasks: split each owned region into at most 4 x 4 near-equal parts of
-    // at least 4 blocks per side.
-    const int ntx = std::max(1, std::min(4, o.bucket_x / (4 * s.blockW)));
-    const int nty = std::max(1, std::min(4, o.bucket_y / (4 * s.blockH)));
+    // at least 4 blocks per side.  Wide blocks (few samples a pixel) take 2 a
+    // side, about 8x8 pixels: a task's whole list is staged and matched for
+    // each of its blocks, so a bucket-sized task of 16 4x4-pixel blocks spends
+    // its time on micropolygons elsewhere in the bucket (sampler at 2x2
+    // samples: 258 to 184 us at 637x475, 1098 to 921 at 1920x1080; 2x2-pixel
+    // blocks gain 0 to 10% in the sampler and lose more in binning).  The
+    // motion and lens samplers run one workgroup a task and keep the larger
+    // tasks, as do frames of so many buckets that their task count would
+    // matter (the no-allocation form holds counters per task).
+    const bool wide = o.shutter_open == o.shutter_close && !s.dof && s.buckets.size() <= 16384;
+    auto parts = [&](int bucket, int block) {
+        const int side = wide ? std::max(2 * block, std::min(8, 4 * block)) : 4 * block;
+        return std::max(1, std::min(4, bucket / side));
+    };
+    const int ntx = parts(o.bucket_x, s.blockW), nty = parts(o.bucket_y, s.blockH);
     s.tasks.clear();
     s.taskStart.assign(1, 0);
     for (size_t k = 0; k < s.buckets.size(); ++k) {

@@ -163,8 +163,9 @@ struct rh_ctx {
     DBuf dLongWork;                       // the long-list combine's work arrays (grown on demand)
     bool transparent = false;             // some posted surface has Os < 1
     bool anyMatte = false;                // some posted surface is a matte (RH_MATTE)
-    // work items: one per task (grid and per-bucket forms), cost-split (batched)
-    DBuf dItemsStatic, dItems, dItemCount, dQueue, dRows;
+    // work items: one per task (per-bucket form, probes), the static grid's, cost-split (batched)
+    DBuf dItemsStatic, dItemsGrid, dItems, dItemCount, dQueue, dRows;
+    int gridItems = 0;                    // items of the static grid (dItemsGrid)
     // occlusion culling: bucket trees, depth pyramids, (surface, bucket) tests, probe results
     DBuf dCullTrees, dCullPyr, dCullBounds, dCullRanges, dCullStart, dCullPairMax, dProbeOut;
     DBuf dProbeItems, dProbeTasks, dProbeCut, dProbeB, dProbeC;
@@ -196,7 +197,7 @@ struct rh_ctx {
                        &dGrids, &dParams,
                        &dPrims, &dCandStart, &dCandGrid, &dCapStart, &dMprec, &dMpbound, &dLists,
                        &dListCount, &dSamples, &dChannels, &dRgba, &dCounters, &dBucketRefs,
-                       &dHitData, &dHitNext, &dHitCtl, &dHitShards, &dHitHeads, &dDeepList, &dFrontDepth, &dLongWork, &dItemsStatic, &dItems,
+                       &dHitData, &dHitNext, &dHitCtl, &dHitShards, &dHitHeads, &dDeepList, &dFrontDepth, &dLongWork, &dItemsStatic, &dItemsGrid, &dItems,
                        &dItemCount, &dQueue, &dRows, &dSegBucket, &dSegCounts, &dMprecMB, &dCullTrees, &dCullPyr,
                        &dCullBounds, &dCullRanges, &dCullStart, &dCullPairMax, &dProbeOut, &dProbeItems,
                        &dProbeTasks, &dProbeCut, &dProbeB, &dProbeC};
@@ -346,6 +347,25 @@ hipError_t scratch_address(void** out) {
     return hipSuccess;
 }
 }  // namespace
+
+// The static grid's work items: the tasks, cut into items of 8 or 4 blocks (4:
+// one a wave) while the frame has fewer than 4096 items, 4 rounds of the 1024
+// workgroups the device holds: a small frame's sampler is as slow as its
+// longest workgroup (64x64: 118 to 34 us; 256x256: 112 to 95), and an item's
+// list is staged once per item, so a frame that fills the device keeps whole
+// tasks (512x512 with 8192 items: 318 to 332 us).
+static std::vector<uint2> grid_items(const std::vector<uint2>& tasks, int blocks) {
+    int per = 16;
+    while (per > 4 && blocks / per < 4096) per >>= 1;
+    if (per == 16) return tasks;
+    std::vector<uint2> out;
+    for (const uint2& t : tasks) {
+        const int n = (int)(t.y >> 16);
+        for (int b = 0; b < n; b += per)
+            out.push_back(make_uint2(t.x, (uint32_t)b | ((uint32_t)std::min(per, n - b) << 16)));
+    }
+    return out;
+}
 
 // The strip filter's lists, from the box tests of the frame shape's sample
 // positions: per filter column an entry for each sample that lies in the box
@@ -536,6 +556,8 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
             total += nblk;
         }
         c->maxItems = std::max(total, 1);
+        const std::vector<uint2> cut = grid_items(it, total);
+        c->gridItems = (int)cut.size();
         int cus = 0, dev = 0, occ = 0;
         if ((e = hipGetDevice(&dev)) == hipSuccess)
             e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -546,9 +568,10 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
         }
         c->persistentGrid = std::max(1, cus * best);
         const int unit = 8 * 16;
-        const int staticGrid = ((int)s.tasks.size() + unit - 1) / unit * unit;
+        const int staticGrid = (c->gridItems + unit - 1) / unit * unit;
         c->maxRows = std::max(staticGrid, c->persistentGrid);
         if (e == hipSuccess) e = upload(c->dItemsStatic, it, c->st);
+        if (e == hipSuccess) e = upload(c->dItemsGrid, cut, c->st);
         if (e == hipSuccess) e = c->dItems.ensure((size_t)c->maxItems * sizeof(uint2));
         if (e == hipSuccess) e = c->dItemCount.ensure(16);
         if (e == hipSuccess) e = c->dQueue.ensure(16);
@@ -853,7 +876,9 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
         rows = c->persistentGrid;
     } else {
         const int unit = 8 * 16;
-        rows = (nt + unit - 1) / unit * unit;
+        a.items = c->dItemsGrid.as<uint2>();
+        a.nStatic = c->gridItems;
+        rows = (c->gridItems + unit - 1) / unit * unit;
         ENQ(rh_launch_sample(c->st, variant, rows, &a));
     }
     if (timed) ENQ(hipEventRecord(c->ev[5], c->st));
@@ -949,7 +974,10 @@ static hipError_t enqueue_depth_pass(rh_ctx* c, bool sample) {
         const DofTables dt = c->dof();
         return rh_launch_sample_dof(c->st, &a, nt, &dt);
     }
-    return rh_launch_sample(c->st, 0, nt, &a);
+    const int unit = 8 * 16;
+    a.items = c->dItemsGrid.as<uint2>();
+    a.nStatic = c->gridItems;
+    return rh_launch_sample(c->st, 0, (c->gridItems + unit - 1) / unit * unit, &a);
 }
 
 // The schedule aqsis's occlusion culling gives (RenderSurface,
@@ -1212,7 +1240,8 @@ rh_status rh_render_device_noalloc(rh_ctx* c) {
     if (!c->scheduled) return fail(RH_ERR_STATE, "rh_render must run before rh_render_device_noalloc");
     if (!c->scratch) return fail(RH_ERR_STATE, "no scratch memory on this context's device");
     const int nt = (int)c->shape.tasks.size();
-    const size_t rows = (c->sched.motion || c->shape.dof) ? (size_t)nt : (size_t)((nt + 127) / 128 * 128);
+    const size_t rows = (c->sched.motion || c->shape.dof) ? (size_t)nt
+                                                          : (size_t)((std::max(nt, c->gridItems) + 127) / 128 * 128);
     if (kScratchRowsOffset + rows * 5 * sizeof(uint32_t) > RH_NOALLOC_SCRATCH_BYTES)
         return fail(RH_ERR_CAPACITY, "the frame has " + std::to_string(nt) + " sampling tasks; the no-allocation "
                                      "form holds the counters of at most " +
@@ -1505,7 +1534,7 @@ uint64_t rh_internal_device_bytes(const rh_ctx* c) {
                          &c->dListCount, &c->dSamples, &c->dChannels, &c->dRgba, &c->dCounters,
                          &c->dBucketRefs, &c->dHitData, &c->dHitNext, &c->dHitCtl, &c->dHitShards, &c->dHitHeads,
                          &c->dDeepList, &c->dFrontDepth,
-                         &c->dItemsStatic, &c->dItems, &c->dItemCount, &c->dQueue, &c->dRows, &c->dMprecMB,
+                         &c->dItemsStatic, &c->dItemsGrid, &c->dItems, &c->dItemCount, &c->dQueue, &c->dRows, &c->dMprecMB,
                          &c->dCullTrees, &c->dCullPyr, &c->dCullBounds, &c->dCullRanges, &c->dCullStart,
                          &c->dCullPairMax, &c->dProbeOut, &c->dProbeItems, &c->dProbeTasks, &c->dProbeCut,
                          &c->dProbeB, &c->dProbeC, &c->dShuffled, &c->dLens, &c->dPixDof, &c->dDofCells,
