@@ -182,6 +182,22 @@ struct DofTables {
     const float4* cells;
 };
 
+// A display request's format: its Quantize settings, and the channels of a
+// pixel it takes, in order (n of them, 4 bits each).
+struct DisplayFormat {
+    float one, min, max, dither;
+    int n;
+    uint32_t channels;
+};
+// RH_DSPY_* (include/aqsis_hider.h)
+#define RH_DSPY_FLOAT32_D 1
+#define RH_DSPY_UNSIGNED32_D 2
+#define RH_DSPY_SIGNED32_D 3
+#define RH_DSPY_UNSIGNED16_D 4
+#define RH_DSPY_SIGNED16_D 5
+#define RH_DSPY_UNSIGNED8_D 6
+#define RH_DSPY_SIGNED8_D 7
+
 // The strip filter's list (rh_filter_strip): the samples of a halo row that
 // add to a pixel, in the reference's order (filter columns, samples), in
 // groups of four of one column; ngroups is even, and two more groups follow.

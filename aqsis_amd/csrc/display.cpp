@@ -104,13 +104,4 @@ int mode_channels(int mode) {
     return ((mode & RH_MODE_A) ? 1 : 0) + ((mode & RH_MODE_RGB) ? 3 : 0) + ((mode & RH_MODE_Z) ? 1 : 0);
 }
 
-int format_request(const float* q, int mode, const float* ch, double s, int type, unsigned char* dst) {
-    unsigned char* p = dst;
-    if (mode & RH_MODE_A) p = put_value(q, ch[6], s, type, p);
-    if (mode & RH_MODE_RGB)
-        for (int k = 0; k < 3; ++k) p = put_value(q, ch[k], s, type, p);
-    if (mode & RH_MODE_Z) p = put_value(q, ch[7], s, type, p);
-    return (int)(p - dst);
-}
-
 }  // namespace rh

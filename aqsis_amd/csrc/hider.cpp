@@ -42,6 +42,8 @@ extern "C" hipError_t rh_launch_combine(hipStream_t, const FrameDev*, size_t, co
                                         const GridDev*, int, float4*, float*);
 extern "C" hipError_t rh_launch_reduce_counters(hipStream_t, const uint32_t*, int, const uint32_t*, int,
                                                 unsigned long long*);
+extern "C" hipError_t rh_launch_format_display(hipStream_t, int, const DisplayFormat*, const float*, const float*,
+                                               size_t, void*);
 extern "C" hipError_t rh_launch_box_classes(hipStream_t, const FrameDev*, int, const uchar4*, const float*, uint32_t*);
 extern "C" hipError_t rh_launch_box_masks(hipStream_t, const FrameDev*, size_t, const uchar4*, const float*,
                                           uint2*);
@@ -55,6 +57,10 @@ extern "C" hipError_t rh_launch_cull_probes_max(hipStream_t, const FrameDev*, co
                                                 const int4*, int, const float4*, float*);
 
 static_assert(rh::GRID_MOTION == RH_GRID_MOTION, "motion grid flag differs between host and device");
+static_assert(RH_DSPY_FLOAT32 == RH_DSPY_FLOAT32_D && RH_DSPY_UNSIGNED32 == RH_DSPY_UNSIGNED32_D &&
+              RH_DSPY_SIGNED32 == RH_DSPY_SIGNED32_D && RH_DSPY_UNSIGNED16 == RH_DSPY_UNSIGNED16_D &&
+              RH_DSPY_SIGNED16 == RH_DSPY_SIGNED16_D && RH_DSPY_UNSIGNED8 == RH_DSPY_UNSIGNED8_D &&
+              RH_DSPY_SIGNED8 == RH_DSPY_SIGNED8_D, "display value types differ");
 static_assert(RH_MATTE == RH_DEV_MATTE && RH_MATTE_ALPHA == RH_DEV_MATTE_ALPHA, "matte values differ");
 static_assert(RH_DEPTH_MIDPOINT == RH_DEV_DEPTH_MIDPOINT && RH_DEPTH_MAX == RH_DEV_DEPTH_MAX &&
                   RH_DEPTH_AVERAGE == RH_DEV_DEPTH_AVERAGE, "depth filter values differ");
@@ -152,7 +158,9 @@ struct rh_ctx {
     // the strip filter's list (FilterDev)
     bool boxVaries = false;
     int filtGroups = 0, filtVary = 0;
-    DBuf dFiltEntries, dFiltGroups, dFiltAlways;
+    size_t filtAlwaysAt = 0, filtGroupsAt = 0;   // words into dFiltList
+    std::vector<uint32_t> filtHost;
+    DBuf dFiltList;
     // schedule
     DBuf dGrids, dParams, dPrims, dCandStart, dCandGrid, dCapStart, dSegBucket, dSegCounts;
     // per frame
@@ -160,6 +168,7 @@ struct rh_ctx {
     DBuf dMprecMB;                        // motion-frame micropolygon records
     // transparent hits: arena of (u, v, depth, id) and (link, surface) pairs
     DBuf dHitData, dHitNext, dHitCtl, dHitShards, dHitHeads, dDeepList, dFrontDepth;
+    DBuf dFormat, dDrawsReq;              // a display request's values; its dither draws
     DBuf dLongWork;                       // the long-list combine's work arrays (grown on demand)
     bool transparent = false;             // some posted surface has Os < 1
     bool anyMatte = false;                // some posted surface is a matte (RH_MATTE)
@@ -193,11 +202,11 @@ struct rh_ctx {
     }
     template <typename F> void each_buffer(F f) {
         DBuf* all[] = {&dFrame, &dBuckets, &dTasks, &dPos2d, &dPos1d, &dPix, &dDither, &dFilter, &dBoxMask,
-                       &dFiltEntries, &dFiltGroups, &dFiltAlways, &dShuffled, &dLens, &dPixDof, &dDofCells,
+                       &dFiltList, &dShuffled, &dLens, &dPixDof, &dDofCells,
                        &dGrids, &dParams,
                        &dPrims, &dCandStart, &dCandGrid, &dCapStart, &dMprec, &dMpbound, &dLists,
                        &dListCount, &dSamples, &dChannels, &dRgba, &dCounters, &dBucketRefs,
-                       &dHitData, &dHitNext, &dHitCtl, &dHitShards, &dHitHeads, &dDeepList, &dFrontDepth, &dLongWork, &dItemsStatic, &dItemsGrid, &dItems,
+                       &dHitData, &dHitNext, &dHitCtl, &dHitShards, &dHitHeads, &dDeepList, &dFrontDepth, &dLongWork, &dFormat, &dDrawsReq, &dItemsStatic, &dItemsGrid, &dItems,
                        &dItemCount, &dQueue, &dRows, &dSegBucket, &dSegCounts, &dMprecMB, &dCullTrees, &dCullPyr,
                        &dCullBounds, &dCullRanges, &dCullStart, &dCullPairMax, &dProbeOut, &dProbeItems,
                        &dProbeTasks, &dProbeCut, &dProbeB, &dProbeC};
@@ -375,14 +384,16 @@ static hipError_t filter_lists(rh_ctx* c) {
     const rh::Shape& s = c->shape;
     const int ns = s.ns, xm = s.shiftX, ym = s.shiftY, rows = 2 * ym + 1, ent = RH_FILTER_ENTRY(ym);
     const size_t nsamp = (size_t)s.extW * s.extH * ns;
-    const int wgs = (int)std::min<size_t>(512, nsamp / 256 + 1);
+    // one workgroup's row of classes takes the room of 8 samples: the sample
+    // buffer, not yet in use, holds them
+    const int wgs = (int)std::min<size_t>(512, nsamp / 8192 + 1);
     std::vector<uint32_t> cls((size_t)wgs * 64);
-    hipError_t e = c->dItems.ensure(cls.size() * sizeof(uint32_t));   // scratch until the work items are set up
+    hipError_t e = c->dSamples.cap < cls.size() * sizeof(uint32_t) ? c->dSamples.ensure(cls.size() * sizeof(uint32_t)) : hipSuccess;
     if (e == hipSuccess)
         e = rh_launch_box_classes(c->st, c->dFrame.as<FrameDev>(), wgs, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
-                                  c->dItems.as<uint32_t>());
+                                  c->dSamples.as<uint32_t>());
     if (e == hipSuccess)
-        e = hipMemcpyAsync(cls.data(), c->dItems.p, cls.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st);
+        e = hipMemcpyAsync(cls.data(), c->dSamples.p, cls.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st);
     if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     if (e != hipSuccess) return e;
     std::vector<uint32_t> all(ns, 0xffffu), any(ns, 0u);
@@ -435,9 +446,14 @@ static hipError_t filter_lists(rh_ctx* c) {
     c->filtVary = (int)std::count_if(groups.begin(), groups.end(), [](uint32_t g) { return (g >> 31) != 0; });
     fill();
     fill();
-    if ((e = upload(c->dFiltEntries, entries, c->st)) != hipSuccess || (e = upload(c->dFiltGroups, groups, c->st)) != hipSuccess ||
-        (e = upload(c->dFiltAlways, always, c->st)) != hipSuccess)
-        return e;
+    // one device copy: entries, always, groups
+    c->filtHost.resize(entries.size() + 2 * always.size() + groups.size());
+    c->filtAlwaysAt = entries.size();
+    c->filtGroupsAt = entries.size() + 2 * always.size();
+    std::memcpy(c->filtHost.data(), entries.data(), entries.size() * sizeof(float));
+    std::memcpy(c->filtHost.data() + c->filtAlwaysAt, always.data(), always.size() * sizeof(always[0]));
+    std::memcpy(c->filtHost.data() + c->filtGroupsAt, groups.data(), groups.size() * sizeof(uint32_t));
+    if ((e = upload(c->dFiltList, c->filtHost, c->st)) != hipSuccess) return e;
     if (c->boxVaries) {
         const size_t npix = (size_t)s.extW * s.extH;
         if ((e = c->dBoxMask.ensure(npix * (2 * xm + 1 + rows) * 8)) != hipSuccess) return e;
@@ -445,7 +461,7 @@ static hipError_t filter_lists(rh_ctx* c) {
                                      c->dBoxMask.as<uint2>())) != hipSuccess)
             return e;
     }
-    return hipStreamSynchronize(c->st);   // the lists' host copies end here
+    return hipSuccess;
 }
 
 extern "C" {
@@ -775,8 +791,9 @@ static FrameCtl context_ctl(rh_ctx* c) {
 // The filter + expose + quantise stage of a frame.
 static hipError_t enqueue_filter(rh_ctx* c) {
     const rh::Shape& s = c->shape;
-    const FilterDev fp{c->dFiltEntries.as<float>(), c->dFiltGroups.as<uint32_t>(), c->filtGroups, c->filtVary,
-                       c->dFiltAlways.as<uint2>()};
+    const uint32_t* list = c->dFiltList.as<uint32_t>();
+    const FilterDev fp{reinterpret_cast<const float*>(list), list + c->filtGroupsAt, c->filtGroups, c->filtVary,
+                       reinterpret_cast<const uint2*>(list + c->filtAlwaysAt)};
     return rh_launch_filter(c->st, c->dFrame.as<FrameDev>(), s.width(), s.height(), s.ns, s.shiftX, s.shiftY,
                             c->dSamples.as<float4>(), c->boxVaries ? c->dBoxMask.as<uint2>() : nullptr,
                             &fp, c->dPix.as<uchar4>(), c->dPos2d.as<float>(), c->dFilter.as<float>(),
@@ -1384,23 +1401,35 @@ rh_status rh_format_display(const rh_options* opt, const float* channels, const 
     return RH_OK;
 }
 
-// The frame's display values of `type`, width x height x 4 values.
-static rh_status display_values(rh_ctx* c, int32_t type, std::vector<unsigned char>& out) {
+// The rendered frame's pixels in a display request's format, as values of
+// `type`, into out.  draws: the request's dither draws on the host when they
+// are not display 0's (which the device holds).
+static rh_status format_frame(rh_ctx* c, const DisplayFormat& f, int32_t type, const float* draws, void* out) {
     const rh::Shape& s = c->shape;
-    const size_t npix = (size_t)s.width() * s.height();
-    const int vb = rh::display_type_bytes(type);
-    if (vb == 0) return fail(RH_ERR_INVALID, "unknown display value type " + std::to_string(type));
-    out.resize(npix * 4 * vb);
+    const size_t npix = (size_t)s.width() * s.height(), bytes = npix * f.n * rh::display_type_bytes(type);
+    const float* dither = c->dDither.as<float>();
+    if (f.one != 0.0f && draws) {
+        HIP_TRY(c->dDrawsReq.ensure(npix * sizeof(float)));
+        HIP_TRY(hipMemcpyAsync(c->dDrawsReq.p, draws, npix * sizeof(float), hipMemcpyHostToDevice, c->st));
+        dither = c->dDrawsReq.as<float>();
+    }
+    HIP_TRY(c->dFormat.ensure(bytes));
+    HIP_TRY(rh_launch_format_display(c->st, type, &f, c->dChannels.as<float>(), dither, npix, c->dFormat.p));
+    HIP_TRY(hipMemcpyAsync(out, c->dFormat.p, bytes, hipMemcpyDeviceToHost, c->st));
+    HIP_TRY(hipStreamSynchronize(c->st));
+    return RH_OK;
+}
+
+// The frame's display values of `type`, width x height x 4 values.
+static rh_status display_values(rh_ctx* c, int32_t type, void* out) {
+    const rh::Shape& s = c->shape;
     if (type == RH_DSPY_UNSIGNED8 && rh::display_type(s.o) == RH_DSPY_UNSIGNED8) {
-        // the device quantised these already
-        HIP_TRY(hipMemcpy(out.data(), c->dRgba.p, npix * 4, hipMemcpyDeviceToHost));
+        // the filter quantised these already
+        HIP_TRY(hipMemcpy(out, c->dRgba.p, (size_t)s.width() * s.height() * 4, hipMemcpyDeviceToHost));
         return RH_OK;
     }
-    std::vector<float> ch(npix * 9);
-    HIP_TRY(hipMemcpy(ch.data(), c->dChannels.p, ch.size() * sizeof(float), hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < npix; ++i)
-        rh::format_pixel(s.o, &ch[i * 9], (double)c->plan.dither[i], type, &out[i * 4 * vb]);
-    return RH_OK;
+    const DisplayFormat f{s.o.quantize_one, s.o.quantize_min, s.o.quantize_max, s.o.quantize_dither, 4, 0x6210u};
+    return format_frame(c, f, type, nullptr, out);
 }
 
 rh_status rh_select_format(float one, float min, float max, int32_t* type) {
@@ -1420,23 +1449,22 @@ rh_status rh_read_display_request(rh_ctx* c, int32_t mode, const float* quantize
         return fail(RH_ERR_INVALID, "display index outside the frame's display requests");
     const int vb = rh::display_type_bytes(type);
     if (vb == 0) return fail(RH_ERR_INVALID, "unknown display value type " + std::to_string(type));
+    DisplayFormat f{quantize[0], quantize[1], quantize[2], quantize[3], 0, 0u};
+    auto add = [&](uint32_t channel) { f.channels |= channel << (4 * f.n++); };
+    if (mode & RH_MODE_A) add(6);
+    if (mode & RH_MODE_RGB)
+        for (uint32_t k = 0; k < 3; ++k) add(k);
+    if (mode & RH_MODE_Z) add(7);
     const size_t npix = (size_t)s.width() * s.height();
-    std::vector<float> ch(npix * 9);
-    HIP_TRY(hipMemcpy(ch.data(), c->dChannels.p, ch.size() * sizeof(float), hipMemcpyDeviceToHost));
-    const float* d = &c->plan.ditherAll[(size_t)index * npix];
-    unsigned char* dst = static_cast<unsigned char*>(out);
-    for (size_t i = 0; i < npix; ++i) dst += rh::format_request(quantize, mode, &ch[i * 9], (double)d[i], type, dst);
-    return RH_OK;
+    return format_frame(c, f, type, index ? &c->plan.ditherAll[(size_t)index * npix] : nullptr, out);
 }
 
 rh_status rh_read_display(rh_ctx* c, int32_t type, void* out) {
     if (!c || !out) return fail(RH_ERR_INVALID, "bad arguments");
     if (!c->rendered) return fail(RH_ERR_STATE, "no rendered frame");
-    std::vector<unsigned char> v;
-    rh_status r = display_values(c, type, v);
-    if (r != RH_OK) return r;
-    std::memcpy(out, v.data(), v.size());
-    return RH_OK;
+    if (rh::display_type_bytes(type) == 0)
+        return fail(RH_ERR_INVALID, "unknown display value type " + std::to_string(type));
+    return display_values(c, type, out);
 }
 
 rh_status rh_display_as(rh_ctx* c, rh_dspy_data_fn data, void* image, int32_t scanline_order, int32_t type) {
@@ -1444,10 +1472,11 @@ rh_status rh_display_as(rh_ctx* c, rh_dspy_data_fn data, void* image, int32_t sc
     if (!c->rendered) return fail(RH_ERR_STATE, "no rendered frame");
     const rh::Shape& s = c->shape;
     const int W = s.width();
-    std::vector<unsigned char> img;
-    rh_status r = display_values(c, type, img);
-    if (r != RH_OK) return r;
     const size_t entry = 4 * (size_t)rh::display_type_bytes(type);
+    if (entry == 0) return fail(RH_ERR_INVALID, "unknown display value type " + std::to_string(type));
+    std::vector<unsigned char> img((size_t)W * s.height() * entry);
+    rh_status r = display_values(c, type, img.data());
+    if (r != RH_OK) return r;
     // a pixel (x, y) of the crop window, in raster coordinates
     auto at = [&](int x, int y) { return &img[((size_t)(y - s.cropY0) * W + (x - s.cropX0)) * entry]; };
     std::vector<unsigned char> bucket, rows;
@@ -1528,7 +1557,7 @@ void rh_internal_trim_pool(uint64_t keep) { release_pool_memory(keep); }
 
 uint64_t rh_internal_device_bytes(const rh_ctx* c) {
     const DBuf* all[] = {&c->dFrame, &c->dBuckets, &c->dTasks, &c->dPos2d, &c->dPos1d, &c->dPix, &c->dDither,
-                         &c->dFilter, &c->dBoxMask, &c->dFiltEntries, &c->dFiltGroups, &c->dFiltAlways,
+                         &c->dFilter, &c->dBoxMask, &c->dFiltList,
                          &c->dGrids, &c->dParams, &c->dPrims, &c->dCandStart,
                          &c->dCandGrid, &c->dCapStart, &c->dSegBucket, &c->dSegCounts, &c->dMprec, &c->dMpbound, &c->dLists,
                          &c->dListCount, &c->dSamples, &c->dChannels, &c->dRgba, &c->dCounters,
@@ -1538,7 +1567,7 @@ uint64_t rh_internal_device_bytes(const rh_ctx* c) {
                          &c->dCullTrees, &c->dCullPyr, &c->dCullBounds, &c->dCullRanges, &c->dCullStart,
                          &c->dCullPairMax, &c->dProbeOut, &c->dProbeItems, &c->dProbeTasks, &c->dProbeCut,
                          &c->dProbeB, &c->dProbeC, &c->dShuffled, &c->dLens, &c->dPixDof, &c->dDofCells,
-                         &c->dLongWork};
+                         &c->dLongWork, &c->dFormat, &c->dDrawsReq};
     uint64_t total = 0;
     for (const DBuf* b : all) total += b->cap;
     return total;

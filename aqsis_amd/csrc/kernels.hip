@@ -2748,6 +2748,43 @@ __device__ __forceinline__ void filter_pixel(const FrameDev* __restrict__ fr, co
     finish_pixel<GAMMA>(fr, acc, gTot, count, ns, t, dither, channels, rgba8);
 }
 
+// A display request's values of each pixel (FormatBucketForDisplay,
+// ddmanager.cpp:1045-1118): the channels `f` names, quantised when f.one != 0,
+// stored as T with x86-64's conversions (a NaN or a value outside the 32-bit
+// range becomes INT_MIN, narrower types keep its low bits; the 32-bit types
+// clamp in double first).  Bound by the copy of the result to the host: for a
+// 512x512 depth image 1 MB instead of the 9.4 MB of channels, and no host
+// loop over the pixels (read-back 1.25 to 0.1 ms).
+template <int TYPE, typename T>
+__device__ __forceinline__ T display_value(const DisplayFormat& f, float v, double draw) {
+    if (TYPE == RH_DSPY_FLOAT32_D && f.one == 0.0f) return (T)v;
+    double value = (double)v;
+    if (f.one != 0.0f) {
+        const double x = 0.0f + value * (double)(f.one - 0.0f) + ((double)f.dither * draw);
+        value = (double)(lfloor_d(x - 0.5) + 1);
+        value = value < (double)f.min ? (double)f.min : (value > (double)f.max ? (double)f.max : value);
+    }
+    if (TYPE == RH_DSPY_FLOAT32_D) return (T)(float)value;
+    if (TYPE == RH_DSPY_UNSIGNED32_D) {
+        value = value < 0.0 ? 0.0 : (value > 4294967295.0 ? 4294967295.0 : value);
+        return value != value ? (T)0 : (T)(uint32_t)value;
+    }
+    if (TYPE == RH_DSPY_SIGNED32_D) value = value < -2147483648.0 ? -2147483648.0 : (value > 2147483647.0 ? 2147483647.0 : value);
+    const int32_t i = (value >= -2147483648.0 && value < 2147483648.0) ? (int32_t)value : INT_MIN;
+    return (T)(uint32_t)i;
+}
+
+template <int TYPE, typename T>
+__global__ void __launch_bounds__(256) rh_format_display(const DisplayFormat f, const float* __restrict__ channels,
+                                                         const float* __restrict__ dither, size_t npix,
+                                                         T* __restrict__ out) {
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= npix) return;
+    const double draw = f.one != 0.0f ? (double)dither[t] : 0.0;
+    for (int k = 0; k < f.n; ++k)
+        out[t * f.n + k] = display_value<TYPE, T>(f, channels[t * 9 + ((f.channels >> (4 * k)) & 15u)], draw);
+}
+
 // The box tests of one sample of the extended region: bit (fx + xm) says that
 // the sample of pixel qx lies inside the filter box of pixel qx - fx
 // (|position - pixel centre| <= ceil(width)/2, bucketprocessor.cpp:600-612,
@@ -3487,6 +3524,25 @@ extern "C" hipError_t rh_launch_reduce_counters(hipStream_t st, const uint32_t* 
                        counters);
     return hipGetLastError();
 }
+// npix pixels' values of type `type` (RH_DSPY_*) into out.
+extern "C" hipError_t rh_launch_format_display(hipStream_t st, int type, const DisplayFormat* f, const float* channels,
+                                               const float* dither, size_t npix, void* out) {
+    if (npix == 0) return hipSuccess;
+    const dim3 grid((unsigned)((npix + 255) / 256)), wg(256);
+#define RH_FORMAT(TYPE, T)                                                                                       \
+    hipLaunchKernelGGL((rh_format_display<TYPE, T>), grid, wg, 0, st, *f, channels, dither, npix, static_cast<T*>(out))
+    switch (type) {
+    case RH_DSPY_FLOAT32_D: RH_FORMAT(RH_DSPY_FLOAT32_D, float); break;
+    case RH_DSPY_UNSIGNED32_D: RH_FORMAT(RH_DSPY_UNSIGNED32_D, uint32_t); break;
+    case RH_DSPY_SIGNED32_D: RH_FORMAT(RH_DSPY_SIGNED32_D, uint32_t); break;
+    case RH_DSPY_UNSIGNED16_D: case RH_DSPY_SIGNED16_D: RH_FORMAT(RH_DSPY_UNSIGNED16_D, uint16_t); break;
+    case RH_DSPY_UNSIGNED8_D: case RH_DSPY_SIGNED8_D: RH_FORMAT(RH_DSPY_UNSIGNED8_D, uint8_t); break;
+    default: return hipErrorInvalidValue;
+    }
+#undef RH_FORMAT
+    return hipGetLastError();
+}
+
 extern "C" hipError_t rh_launch_box_classes(hipStream_t st, const FrameDev* fr, int workgroups,
                                             const uchar4* pixPattern, const float* pos2d, uint32_t* rows) {
     hipLaunchKernelGGL(rh_box_classes, dim3(workgroups), dim3(256), 0, st, fr, pixPattern, pos2d, rows);
