@@ -297,6 +297,46 @@ PlanKey plan_key(const rh::Shape& s) {
             s.shiftX, s.shiftY, s.nx, s.ny, s.o.jitter ? 1 : 0, s.o.num_displays};
 }
 
+// Box-test classes of recent frame shapes (filter_lists), a word a sample:
+// they follow from the sample positions and the filter's box, and asking the
+// device for them is a wait in a context's set-up (0.1 to 0.25 ms).
+struct ClassCache {
+    std::mutex m;
+    std::list<std::pair<std::pair<PlanKey, std::array<float, 2>>, std::vector<uint32_t>>> lru;   // front: most recent
+};
+ClassCache& class_cache() {
+    static ClassCache cc;
+    return cc;
+}
+constexpr size_t kClassCacheShapes = 64;
+
+std::pair<PlanKey, std::array<float, 2>> class_key(const rh::Shape& s) {
+    return {plan_key(s), {s.xfwo2, s.yfwo2}};
+}
+
+bool recent_classes(const rh::Shape& s, std::vector<uint32_t>& out) {
+    ClassCache& cc = class_cache();
+    const auto key = class_key(s);
+    std::lock_guard<std::mutex> lk(cc.m);
+    for (auto it = cc.lru.begin(); it != cc.lru.end(); ++it)
+        if (it->first == key) {
+            cc.lru.splice(cc.lru.begin(), cc.lru, it);
+            out = it->second;
+            return true;
+        }
+    return false;
+}
+
+void keep_classes(const rh::Shape& s, const std::vector<uint32_t>& cls) {
+    ClassCache& cc = class_cache();
+    const auto key = class_key(s);
+    std::lock_guard<std::mutex> lk(cc.m);
+    for (const auto& e : cc.lru)
+        if (e.first == key) return;       // another thread had them too
+    cc.lru.emplace_front(key, cls);
+    if (cc.lru.size() > kClassCacheShapes) cc.lru.pop_back();
+}
+
 void cached_plan(const rh::Shape& s, rh::Plan& out) {
     const PlanKey key = plan_key(s);
     PlanCache& pc = plan_cache();
@@ -384,24 +424,35 @@ static hipError_t filter_lists(rh_ctx* c) {
     const rh::Shape& s = c->shape;
     const int ns = s.ns, xm = s.shiftX, ym = s.shiftY, rows = 2 * ym + 1, ent = RH_FILTER_ENTRY(ym);
     const size_t nsamp = (size_t)s.extW * s.extH * ns;
-    // one workgroup's row of classes takes the room of 8 samples: the sample
-    // buffer, not yet in use, holds them
-    const int wgs = (int)std::min<size_t>(512, nsamp / 8192 + 1);
-    std::vector<uint32_t> cls((size_t)wgs * 64);
-    hipError_t e = c->dSamples.cap < cls.size() * sizeof(uint32_t) ? c->dSamples.ensure(cls.size() * sizeof(uint32_t)) : hipSuccess;
-    if (e == hipSuccess)
-        e = rh_launch_box_classes(c->st, c->dFrame.as<FrameDev>(), wgs, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
-                                  c->dSamples.as<uint32_t>());
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(cls.data(), c->dSamples.p, cls.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, c->st);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
-    if (e != hipSuccess) return e;
-    std::vector<uint32_t> all(ns, 0xffffu), any(ns, 0u);
-    for (int w = 0; w < wgs; ++w)
+    hipError_t e;
+    std::vector<uint32_t> cls(ns);
+    if (!recent_classes(s, cls)) {
+        // one workgroup's row of classes takes the room of 8 samples: the
+        // sample buffer, not yet in use, holds them
+        const int wgs = (int)std::min<size_t>(512, nsamp / 8192 + 1);
+        std::vector<uint32_t> rowsOf((size_t)wgs * 64);
+        const size_t bytes = rowsOf.size() * sizeof(uint32_t);
+        if ((e = c->dSamples.ensure(std::max(bytes, c->dSamples.cap))) != hipSuccess ||
+            (e = rh_launch_box_classes(c->st, c->dFrame.as<FrameDev>(), wgs, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
+                                       c->dSamples.as<uint32_t>())) != hipSuccess ||
+            (e = hipMemcpyAsync(rowsOf.data(), c->dSamples.p, bytes, hipMemcpyDeviceToHost, c->st)) != hipSuccess ||
+            (e = hipStreamSynchronize(c->st)) != hipSuccess)
+            return e;
         for (int si = 0; si < ns; ++si) {
-            all[si] &= cls[(size_t)w * 64 + si] & 0xffffu;
-            any[si] |= cls[(size_t)w * 64 + si] >> 16;
+            uint32_t a = 0xffffu, o = 0u;
+            for (int w = 0; w < wgs; ++w) {
+                a &= rowsOf[(size_t)w * 64 + si] & 0xffffu;
+                o |= rowsOf[(size_t)w * 64 + si] >> 16;
+            }
+            cls[si] = a | (o << 16);
         }
+        keep_classes(s, cls);
+    }
+    std::vector<uint32_t> all(ns), any(ns);
+    for (int si = 0; si < ns; ++si) {
+        all[si] = cls[si] & 0xffffu;
+        any[si] = cls[si] >> 16;
+    }
     std::vector<float> entries;
     std::vector<uint32_t> groups;
     std::vector<unsigned long long> always((size_t)(2 * xm + 1) * rows, 0ull);
@@ -455,9 +506,9 @@ static hipError_t filter_lists(rh_ctx* c) {
     std::memcpy(c->filtHost.data() + c->filtGroupsAt, groups.data(), groups.size() * sizeof(uint32_t));
     if ((e = upload(c->dFiltList, c->filtHost, c->st)) != hipSuccess) return e;
     if (c->boxVaries) {
-        const size_t npix = (size_t)s.extW * s.extH;
-        if ((e = c->dBoxMask.ensure(npix * (2 * xm + 1 + rows) * 8)) != hipSuccess) return e;
-        if ((e = rh_launch_box_masks(c->st, c->dFrame.as<FrameDev>(), npix, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
+        const size_t nwords = (size_t)s.extW * s.extH * (2 * xm + 1 + rows);
+        if ((e = c->dBoxMask.ensure(nwords * sizeof(uint2))) != hipSuccess) return e;
+        if ((e = rh_launch_box_masks(c->st, c->dFrame.as<FrameDev>(), nwords, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
                                      c->dBoxMask.as<uint2>())) != hipSuccess)
             return e;
     }

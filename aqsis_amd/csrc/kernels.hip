@@ -2846,24 +2846,28 @@ __global__ void __launch_bounds__(256) rh_box_classes(const FrameDev* __restrict
 
 // A pixel's box tests as bits by sample, for a frame shape where some vary:
 // 2*xm+1 words of the column tests (bit si: sample si lies within the box of
-// the pixel at -fx), then 2*ym+1 of the row tests.  One thread a pixel.
+// the pixel at -fx), then 2*ym+1 of the row tests.  One thread a word.
 __global__ void __launch_bounds__(256) rh_box_masks(const FrameDev* __restrict__ fr,
                                                     const uchar4* __restrict__ pixPattern,
-                                                    const float* __restrict__ pos2d,
-                                                    uint2* __restrict__ masks) {
-    const int ns = fr->ns, nx = 2 * fr->shiftX + 1, ny = 2 * fr->shiftY + 1;
-    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (size_t)fr->extW * fr->extH) return;
-    uint2* out = masks + q * (nx + ny);
-    for (int k = 0; k < nx + ny; ++k) out[k] = make_uint2(0u, 0u);
+                                                    const float* __restrict__ pos2d, uint2* __restrict__ masks) {
+    const int ns = fr->ns, nx = 2 * fr->shiftX + 1, nw = nx + 2 * fr->shiftY + 1, extW = fr->extW;
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t q = t / nw;
+    if (q >= (size_t)extW * fr->extH) return;
+    const int k = (int)(t - q * nw);
+    const bool row = k >= nx;
+    const int p = row ? fr->extY0 + (int)(q / extW) : fr->extX0 + (int)(q % extW);
+    const float cent = (p - (row ? k - nx - fr->shiftY : k - fr->shiftX)) + 0.5f;
+    const float half = row ? fr->yfwo2 : fr->xfwo2;
+    const float* pos = pos2d + 2 * (size_t)pixPattern[q].x * ns + (row ? 1 : 0);
+    uint2 m = make_uint2(0u, 0u);
     for (int si = 0; si < ns; ++si) {
-        const uint32_t m = box_tests(fr, pixPattern, pos2d, q, si);
-        for (int k = 0; k < nx + ny; ++k) {
-            const uint32_t b = (k < nx ? m >> k : m >> (8 + k - nx)) & 1u;
-            if (si < 32) out[k].x |= b << si;
-            else out[k].y |= b << (si - 32);
-        }
+        const float v = ((float)p + pos[2 * si]) - cent;
+        const uint32_t b = v >= -half && v <= half ? 1u : 0u;
+        if (si < 32) m.x |= b << si;
+        else m.y |= b << (si - 32);
     }
+    masks[t] = m;
 }
 
 // The strip filter.  Each wave takes a strip of RH_FS_W x R display pixels and
@@ -3549,10 +3553,10 @@ extern "C" hipError_t rh_launch_box_classes(hipStream_t st, const FrameDev* fr, 
     return hipGetLastError();
 }
 
-extern "C" hipError_t rh_launch_box_masks(hipStream_t st, const FrameDev* fr, size_t npixels,
+extern "C" hipError_t rh_launch_box_masks(hipStream_t st, const FrameDev* fr, size_t nwords,
                                           const uchar4* pixPattern, const float* pos2d, uint2* masks) {
-    if (npixels == 0) return hipSuccess;
-    hipLaunchKernelGGL(rh_box_masks, dim3((unsigned)((npixels + 255) / 256)), dim3(256), 0, st, fr, pixPattern,
+    if (nwords == 0) return hipSuccess;
+    hipLaunchKernelGGL(rh_box_masks, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, st, fr, pixPattern,
                        pos2d, masks);
     return hipGetLastError();
 }
