@@ -73,6 +73,12 @@
 #define SPH_IDENT_D 17
 #define SPH_TABLES_D 18
 
+// Words of the batched form's plan: [0] its items, then the items of each
+// cost class and those handed out (33 each).
+#define RH_PLAN_HIST 32
+#define RH_PLAN_NEXT 96
+#define RH_PLAN_WORDS 132
+
 struct FrameDev {
     float camToRaster[16];
     int cropX0, cropX1, cropY0, cropY1;

@@ -32,7 +32,7 @@ extern "C" hipError_t rh_launch_sample_dof(hipStream_t, const SampleLaunch*, int
 extern "C" hipError_t rh_sample_occupancy(int, int*);
 extern "C" hipError_t rh_launch_plan_items(hipStream_t, const FrameDev*, const TaskDev*, int, const uint32_t*,
                                            uint32_t, int, uint2*, uint32_t*, uint32_t*);
-extern "C" hipError_t rh_launch_frame_begin(hipStream_t, unsigned long long*, uint32_t*, uint32_t*);
+extern "C" hipError_t rh_launch_frame_begin(hipStream_t, unsigned long long*, uint32_t*, uint32_t*, uint32_t*);
 extern "C" hipError_t rh_launch_combine_long(hipStream_t, const FrameDev*, size_t, const uint2*,
                                              const unsigned long long*, uint32_t*, const float4*, const uint2*,
                                              const PrimDev*, const float*, int, int, const GridDev*, int, float4*,
@@ -640,7 +640,7 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
         if (e == hipSuccess) e = upload(c->dItemsStatic, it, c->st);
         if (e == hipSuccess) e = upload(c->dItemsGrid, cut, c->st);
         if (e == hipSuccess) e = c->dItems.ensure((size_t)c->maxItems * sizeof(uint2));
-        if (e == hipSuccess) e = c->dItemCount.ensure(16);
+        if (e == hipSuccess) e = c->dItemCount.ensure(RH_PLAN_WORDS * sizeof(uint32_t));
         if (e == hipSuccess) e = c->dQueue.ensure(16);
         if (e == hipSuccess) e = c->dRows.ensure((size_t)c->maxRows * 5 * sizeof(uint32_t));
     }
@@ -885,7 +885,7 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
     hipError_t e;
 #define ENQ(x) do { if ((e = (x)) != hipSuccess) return e; } while (0)
     if (timed) ENQ(hipEventRecord(c->ev[0], c->st));
-    ENQ(rh_launch_frame_begin(c->st, k.counters, k.hitCtl, c->dHitShards.as<uint32_t>()));
+    ENQ(rh_launch_frame_begin(c->st, k.counters, k.hitCtl, c->dHitShards.as<uint32_t>(), c->dItemCount.as<uint32_t>()));
     ENQ(rh_launch_dice(c->st, f, c->dGrids.as<GridDev>(), (int)S.grids.size(), c->dPrims.as<PrimDev>(),
                        c->dParams.as<float>(), c->dMprec.as<float>(), c->dMpbound.as<float4>(),
                        S.motion ? c->dMprecMB.as<float4>() : nullptr));
@@ -1018,7 +1018,7 @@ static hipError_t enqueue_depth_pass(rh_ctx* c, bool sample) {
     const FrameDev* f = c->dFrame.as<FrameDev>();
     hipError_t e;
     if ((e = rh_launch_frame_begin(c->st, c->dCounters.as<unsigned long long>(), c->dHitCtl.as<uint32_t>(),
-                                   c->dHitShards.as<uint32_t>())) != hipSuccess)
+                                   c->dHitShards.as<uint32_t>(), c->dItemCount.as<uint32_t>())) != hipSuccess)
         return e;
     if ((e = rh_launch_dice(c->st, f, c->dGrids.as<GridDev>(), (int)S.grids.size(), c->dPrims.as<PrimDev>(),
                             c->dParams.as<float>(), c->dMprec.as<float>(), c->dMpbound.as<float4>(),

@@ -2366,65 +2366,94 @@ rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buc
 // ---------------------------------------------------------------------------
 // Batched form: work items ordered by cost
 // ---------------------------------------------------------------------------
-// One workgroup.  A task's cost is (list length + 16) x blocks; a task is cut
+// A task's cost is (list length + 16) x blocks; a task is cut
 // into k items of near-equal block ranges, at least enough that no item
 // needs more than one pass (itemBlocks blocks), and more while an item would
 // cost over splitCost (down to one block per item).  Items are written in
 // descending order of log2(cost), so the persistent sampler takes the
 // largest first; the order inside a class is unspecified (results do not
-// depend on it).  Also resets the work queue.
-__global__ void __launch_bounds__(1024) rh_plan_items(const FrameDev* __restrict__ fr,
-                                                      const TaskDev* __restrict__ tasks, int ntasks,
-                                                      const uint32_t* __restrict__ listCount, uint32_t splitCost,
-                                                      int itemBlocks, uint2* __restrict__ items,
-                                                      uint32_t* __restrict__ itemCount,
-                                                      uint32_t* __restrict__ queueHead) {
-    __shared__ uint32_t hist[33], offs[33];
-    const int tid = threadIdx.x;
+// depend on it).  Two passes over the tasks, one thread each: the items per
+// class, then each workgroup takes its share of every class's range (latency
+// bound: a single workgroup walking the tasks took 92 us for 32,640 of them
+// and 187 for 65,536, the two passes take 11 and 14).
+// ctl: RH_PLAN_HIST.. items per class, RH_PLAN_NEXT.. items handed out, both
+// cleared by rh_frame_begin; [0] the number of items.
+struct PlanTask {
+    int nblk, per, nitems, bin;
+};
+
+__device__ __forceinline__ PlanTask plan_task(const FrameDev* __restrict__ fr, const TaskDev T, uint32_t listCount,
+                                              uint32_t splitCost, int itemBlocks) {
     const int bw = fr->blockW, bh = fr->blockH;
-    if (tid < 33) hist[tid] = 0;
+    PlanTask p;
+    p.nblk = ((T.x1 - T.x0 + bw - 1) / bw) * ((T.y1 - T.y0 + bh - 1) / bh);
+    const unsigned long long cost = (unsigned long long)(listCount + 16u) * (unsigned)p.nblk;
+    int k = (p.nblk + itemBlocks - 1) / itemBlocks;
+    while (k < p.nblk && cost / (unsigned long long)k > splitCost) k = (2 * k < p.nblk) ? 2 * k : p.nblk;
+    // items of `per` blocks; the last may be shorter, so count them
+    p.per = (p.nblk + k - 1) / k;
+    p.nitems = (p.nblk + p.per - 1) / p.per;
+    unsigned long long c = cost / (unsigned long long)p.nitems;
+    if (c > 0xffffffffull) c = 0xffffffffull;
+    p.bin = 32 - __clz((uint32_t)c | 1u);   // 1..32
+    return p;
+}
+
+__global__ void __launch_bounds__(256) rh_plan_count(const FrameDev* __restrict__ fr, const TaskDev* __restrict__ tasks,
+                                                     int ntasks, const uint32_t* __restrict__ listCount,
+                                                     uint32_t splitCost, int itemBlocks, uint32_t* __restrict__ ctl) {
+    __shared__ uint32_t hist[33];
+    if (threadIdx.x < 33) hist[threadIdx.x] = 0;
     __syncthreads();
-    for (int pass = 0; pass < 2; ++pass) {
-        for (int t = tid; t < ntasks; t += 1024) {
-            const TaskDev T = tasks[t];
-            const int nblk = ((T.x1 - T.x0 + bw - 1) / bw) * ((T.y1 - T.y0 + bh - 1) / bh);
-            const unsigned long long cost = (unsigned long long)(listCount[t] + 16u) * (unsigned)nblk;
-            int k = (nblk + itemBlocks - 1) / itemBlocks;
-            while (k < nblk && cost / (unsigned long long)k > splitCost) k = (2 * k < nblk) ? 2 * k : nblk;
-            // items of `per` blocks; the last may be shorter, so count them
-            const int per = (nblk + k - 1) / k;
-            const int nitems = (nblk + per - 1) / per;
-            unsigned long long c = cost / (unsigned long long)nitems;
-            if (c > 0xffffffffull) c = 0xffffffffull;
-            const int bin = 32 - __clz((uint32_t)c | 1u);   // 1..32
-            if (pass == 0) {
-                atomicAdd(&hist[bin], (uint32_t)nitems);
-            } else {
-                for (int b0 = 0; b0 < nblk; b0 += per) {
-                    const int nb = (nblk - b0) < per ? (nblk - b0) : per;
-                    const uint32_t slot = atomicAdd(&offs[bin], 1u);
-                    items[slot] = make_uint2((uint32_t)t, (uint32_t)b0 | ((uint32_t)nb << 16));
-                }
-            }
-        }
-        __syncthreads();
-        if (pass == 0 && tid == 0) {
-            uint32_t run = 0;
-            for (int b = 32; b >= 0; --b) {
-                offs[b] = run;
-                run += hist[b];
-            }
-            itemCount[0] = run;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < ntasks) {
+        const PlanTask p = plan_task(fr, tasks[t], listCount[t], splitCost, itemBlocks);
+        atomicAdd(&hist[p.bin], (uint32_t)p.nitems);
+    }
+    __syncthreads();
+    if (threadIdx.x < 33 && hist[threadIdx.x]) atomicAdd(&ctl[RH_PLAN_HIST + threadIdx.x], hist[threadIdx.x]);
+}
+
+__global__ void __launch_bounds__(256) rh_plan_items(const FrameDev* __restrict__ fr, const TaskDev* __restrict__ tasks,
+                                                     int ntasks, const uint32_t* __restrict__ listCount,
+                                                     uint32_t splitCost, int itemBlocks, uint2* __restrict__ items,
+                                                     uint32_t* __restrict__ ctl, uint32_t* __restrict__ queueHead) {
+    __shared__ uint32_t mine[33], base[33];
+    const int tid = threadIdx.x;
+    if (tid < 33) mine[tid] = 0;
+    __syncthreads();
+    const int t = blockIdx.x * 256 + tid;
+    PlanTask p = {0, 1, 0, 0};
+    uint32_t slot = 0;
+    if (t < ntasks) {
+        p = plan_task(fr, tasks[t], listCount[t], splitCost, itemBlocks);
+        slot = atomicAdd(&mine[p.bin], (uint32_t)p.nitems);
+    }
+    __syncthreads();
+    if (tid < 33) {
+        // the class starts after the costlier ones
+        uint32_t start = 0;
+        for (int b = 32; b > tid; --b) start += ctl[RH_PLAN_HIST + b];
+        base[tid] = start + (mine[tid] ? atomicAdd(&ctl[RH_PLAN_NEXT + tid], mine[tid]) : 0u);
+        if (blockIdx.x == 0 && tid == 0) {
+            ctl[0] = start + ctl[RH_PLAN_HIST];
             queueHead[0] = 0;
         }
-        __syncthreads();
+    }
+    __syncthreads();
+    if (t >= ntasks) return;
+    slot += base[p.bin];
+    for (int b0 = 0; b0 < p.nblk; b0 += p.per) {
+        const int nb = (p.nblk - b0) < p.per ? (p.nblk - b0) : p.per;
+        items[slot++] = make_uint2((uint32_t)t, (uint32_t)b0 | ((uint32_t)nb << 16));
     }
 }
 
 // Clears the frame's counters (graph-safe: a kernel, not a memset).
 __global__ void rh_frame_begin(unsigned long long* __restrict__ counters, uint32_t* __restrict__ hitCtl,
-                               uint32_t* __restrict__ hitShards) {
+                               uint32_t* __restrict__ hitShards, uint32_t* __restrict__ planCtl) {
     const int t = threadIdx.x;
+    for (int k = t; k < RH_PLAN_WORDS; k += 64) planCtl[k] = 0u;
     if (t < RH_HIT_SHARDS) hitShards[t * RH_HIT_SHARD_WORDS] = 0u;
     if (t < RH_NCOUNTERS) counters[t] = 0ull;
     if (t < RH_HITCTL_WORDS) hitCtl[t] = 0u;
@@ -3463,9 +3492,11 @@ extern "C" hipError_t rh_sample_occupancy(int variant, int* blocksPerCU) {
 
 extern "C" hipError_t rh_launch_plan_items(hipStream_t st, const FrameDev* fr, const TaskDev* tasks, int ntasks,
                                            const uint32_t* listCount, uint32_t splitCost, int itemBlocks,
-                                           uint2* items, uint32_t* itemCount, uint32_t* queueHead) {
-    hipLaunchKernelGGL(rh_plan_items, dim3(1), dim3(1024), 0, st, fr, tasks, ntasks, listCount, splitCost,
-                       itemBlocks, items, itemCount, queueHead);
+                                           uint2* items, uint32_t* ctl, uint32_t* queueHead) {
+    const dim3 grid((unsigned)std::max(1, (ntasks + 255) / 256)), wg(256);
+    hipLaunchKernelGGL(rh_plan_count, grid, wg, 0, st, fr, tasks, ntasks, listCount, splitCost, itemBlocks, ctl);
+    hipLaunchKernelGGL(rh_plan_items, grid, wg, 0, st, fr, tasks, ntasks, listCount, splitCost, itemBlocks, items, ctl,
+                       queueHead);
     return hipGetLastError();
 }
 
@@ -3516,8 +3547,8 @@ extern "C" hipError_t rh_launch_combine_long(hipStream_t st, const FrameDev* fr,
 }
 
 extern "C" hipError_t rh_launch_frame_begin(hipStream_t st, unsigned long long* counters, uint32_t* hitCtl,
-                                            uint32_t* hitShards) {
-    hipLaunchKernelGGL(rh_frame_begin, dim3(1), dim3(64), 0, st, counters, hitCtl, hitShards);
+                                            uint32_t* hitShards, uint32_t* planCtl) {
+    hipLaunchKernelGGL(rh_frame_begin, dim3(1), dim3(64), 0, st, counters, hitCtl, hitShards, planCtl);
     return hipGetLastError();
 }
 
