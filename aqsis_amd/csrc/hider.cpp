@@ -28,7 +28,7 @@ extern "C" hipError_t rh_launch_bin(hipStream_t, const FrameDev*, const BucketDe
                                     const unsigned long long*, const float4*, uint32_t*, uint32_t*, uint32_t*,
                                     uint32_t*, unsigned long long*, int, int, const float4*);
 extern "C" hipError_t rh_launch_sample(hipStream_t, int, int, const SampleLaunch*);
-extern "C" hipError_t rh_launch_sample_dof(hipStream_t, const SampleLaunch*, int, const DofTables*);
+extern "C" hipError_t rh_launch_sample_dof(hipStream_t, const SampleLaunch*, int, int, const DofTables*);
 extern "C" hipError_t rh_sample_occupancy(int, int*);
 extern "C" hipError_t rh_launch_plan_items(hipStream_t, const FrameDev*, const TaskDev*, int, const uint32_t*,
                                            uint32_t, int, uint2*, uint32_t*, uint32_t*);
@@ -175,6 +175,7 @@ struct rh_ctx {
     // work items: one per task (per-bucket form, probes), the static grid's, cost-split (batched)
     DBuf dItemsStatic, dItemsGrid, dItems, dItemCount, dQueue, dRows;
     int gridItems = 0;                    // items of the static grid (dItemsGrid)
+    int dofSplit = 1;                     // lens sampler: workgroups sharing a task's passes
     // occlusion culling: bucket trees, depth pyramids, (surface, bucket) tests, probe results
     DBuf dCullTrees, dCullPyr, dCullBounds, dCullRanges, dCullStart, dCullPairMax, dProbeOut;
     DBuf dProbeItems, dProbeTasks, dProbeCut, dProbeB, dProbeC;
@@ -637,6 +638,14 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
         const int unit = 8 * 16;
         const int staticGrid = (c->gridItems + unit - 1) / unit * unit;
         c->maxRows = std::max(staticGrid, c->persistentGrid);
+        if (s.dof) {
+            // Each pass (4 lens cells of a tile) stages the task's list by
+            // itself, so the passes of a frame with few tasks are spread over
+            // workgroups until the device (5 a CU) has a few rounds of them.
+            const int nt = (int)s.tasks.size();
+            while (c->dofSplit < (s.ns + 3) / 4 && (c->dofSplit + 1) * nt <= 4096) ++c->dofSplit;
+            c->maxRows = std::max(c->maxRows, nt * c->dofSplit);
+        }
         if (e == hipSuccess) e = upload(c->dItemsStatic, it, c->st);
         if (e == hipSuccess) e = upload(c->dItemsGrid, cut, c->st);
         if (e == hipSuccess) e = c->dItems.ensure((size_t)c->maxItems * sizeof(uint2));
@@ -923,8 +932,8 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
     } else if (s.dof) {
         // Depth of field: the lens form of the sampler, whatever the layout.
         const DofTables dt = c->dof();
-        ENQ(rh_launch_sample_dof(c->st, &a, nt, &dt));
-        rows = nt;
+        ENQ(rh_launch_sample_dof(c->st, &a, nt, c->dofSplit, &dt));
+        rows = nt * c->dofSplit;
     } else if (tu.mode == RH_MODE_PLAIN) {
         // One launch per bucket, in bucket order.
         for (int b = 0; b < nb; ++b) {
@@ -1040,7 +1049,7 @@ static hipError_t enqueue_depth_pass(rh_ctx* c, bool sample) {
     if (S.motion) return rh_launch_sample_mb(c->st, &a, nt, c->dMprecMB.as<float4>());
     if (s.dof) {
         const DofTables dt = c->dof();
-        return rh_launch_sample_dof(c->st, &a, nt, &dt);
+        return rh_launch_sample_dof(c->st, &a, nt, c->dofSplit, &dt);
     }
     const int unit = 8 * 16;
     a.items = c->dItemsGrid.as<uint2>();
@@ -1164,7 +1173,7 @@ static rh_status cull_schedule(rh_ctx* c, const rh::Forest& forest) {
                     HIP_TRY(rh_launch_sample_mb(c->st, &a, ni, c->dMprecMB.as<float4>()));
                 } else if (s.dof) {
                     const DofTables dt = c->dof();
-                    HIP_TRY(rh_launch_sample_dof(c->st, &a, ni, &dt));
+                    HIP_TRY(rh_launch_sample_dof(c->st, &a, ni, 1, &dt));
                 } else {
                     HIP_TRY(rh_launch_sample(c->st, 0, ni, &a));
                 }
@@ -1308,7 +1317,7 @@ rh_status rh_render_device_noalloc(rh_ctx* c) {
     if (!c->scheduled) return fail(RH_ERR_STATE, "rh_render must run before rh_render_device_noalloc");
     if (!c->scratch) return fail(RH_ERR_STATE, "no scratch memory on this context's device");
     const int nt = (int)c->shape.tasks.size();
-    const size_t rows = (c->sched.motion || c->shape.dof) ? (size_t)nt
+    const size_t rows = (c->sched.motion || c->shape.dof) ? (size_t)nt * (c->sched.motion ? 1 : c->dofSplit)
                                                           : (size_t)((std::max(nt, c->gridItems) + 127) / 128 * 128);
     if (kScratchRowsOffset + rows * 5 * sizeof(uint32_t) > RH_NOALLOC_SCRATCH_BYTES)
         return fail(RH_ERR_CAPACITY, "the frame has " + std::to_string(nt) + " sampling tasks; the no-allocation "

@@ -2113,13 +2113,17 @@ __device__ __forceinline__ bool dof_quad_hit(const float* qx, const float* qy, c
 // Contains2D and the LOD range are order-free; then each lane, in list
 // order: occlusion skip, SPL_bound_hits, dofSampleInBound (micropolygon.cpp:
 // 1531-1550) against the micropolygon's bound, the moved-quad hit test and
-// StoreSample.  One workgroup of four waves per task.  STORE: StoreSample's
-// mode (RH_STORE_*).
+// StoreSample.  Four waves, `split` workgroups a task, each taking some of the
+// passes of four blocks.  Bound by vector issue, half of it the moved-quad
+// test; at 317x211, 3x3 samples: 1087 us with tasks of 16x4 pixels (half the
+// lanes without a pixel), one workgroup a task and bound tests of a 64-bit
+// shift a lane each, 470 us now.  STORE: StoreSample's mode (RH_STORE_*).
 template <int STORE>
 __global__ void __launch_bounds__(RH_DOF_WAVES * 64)
 rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets, const TaskDev* __restrict__ tasks,
-              int itemBase, const unsigned long long* __restrict__ capStart, const uint32_t* __restrict__ listCount,
-              const uint32_t* __restrict__ lists, const float4* __restrict__ mprec4, const GridDev* __restrict__ grids,
+              int itemBase, int split, const unsigned long long* __restrict__ capStart,
+              const uint32_t* __restrict__ listCount, const uint32_t* __restrict__ lists,
+              const float4* __restrict__ mprec4, const GridDev* __restrict__ grids,
               const PrimDev* __restrict__ prims, const float* __restrict__ pos2d, const float* __restrict__ pos1d,
               const uchar4* __restrict__ pixPattern, const uint8_t* __restrict__ shuffled,
               const float2* __restrict__ lensTab, const uint8_t* __restrict__ pixDof, const float4* __restrict__ cells,
@@ -2135,21 +2139,23 @@ rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buc
     __shared__ uint32_t wsum[RH_DOF_WAVES][5];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ns = fr->ns;
-    const int task = taskList ? (int)taskList[itemBase + blockIdx.x] : itemBase + (int)blockIdx.x;
+    // `split` workgroups share a task's passes
+    const int item = itemBase + (int)(blockIdx.x / (uint32_t)split), share = (int)(blockIdx.x % (uint32_t)split);
+    const int task = taskList ? (int)taskList[item] : item;
     const TaskDev T = tasks[task];
     const BucketDev B = buckets[T.bucket];
     constexpr bool cullH = STORE != RH_STORE_LIST_ALL, midS = STORE == RH_STORE_MIDPOINT;
     const int tilesX = (T.x1 - T.x0 + 7) >> 3, tilesY = (T.y1 - T.y0 + 7) >> 3;
     const int nblk = tilesX * tilesY * ns;
     const uint32_t* L = lists + capStart[task];
-    const uint32_t n = list_cut(L, listCount[task], itemCut ? itemCut[itemBase + blockIdx.x] : idCut);
+    const uint32_t n = list_cut(L, listCount[task], itemCut ? itemCut[item] : idCut);
     const unsigned long long rowRep = 0x0101010101010101ull;   // bit 8r of every row r
     const int lx = lane & 7, ly = lane >> 3;
     uint32_t nTest = 0, nBound = 0, nHit = 0, nIn = 0, nIn2 = 0;
     HitArena arena = hit_arena(fr->hitCapacity, hitCtl, hitShards, blockIdx.x + wave * (RH_HIT_SHARDS / RH_DOF_WAVES));
 
     // every wave runs the same number of passes (the staging barriers)
-    for (int p0 = 0; p0 < nblk; p0 += RH_DOF_WAVES) {
+    for (int p0 = share * RH_DOF_WAVES; p0 < nblk; p0 += split * RH_DOF_WAVES) {
         const int blk = p0 + wave;
         const bool has = blk < nblk;                     // uniform across the wave
         const int tile = has ? blk / ns : 0, cell = has ? blk - tile * ns : 0;
@@ -2256,15 +2262,36 @@ rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buc
             for (int i0 = 0; i0 < nm; i0 += 64) {
                 const int ni = (nm - i0) < 64 ? (nm - i0) : 64;
                 // (2) order-free: the lane's sample in the micropolygon's
-                // window, inside its shifted bound, LOD in range
-                unsigned long long pb = 0ull;
-                for (int i = 0; i < ni; ++i) {
-                    const unsigned long long mm = matM[wave][i0 + i];
-                    const float4 sb = matB[wave][i0 + i];
-                    const bool inB = !(sx < sb.x) & !(sx > sb.y) & !(sy < sb.z) & !(sy > sb.w);
-                    const bool in = ((mm >> lane) & 1ull) != 0ull && inB;
-                    pb |= (unsigned long long)in << i;
-                }
+                // window, inside its shifted bound, LOD in range; four at a
+                // time, broadcast reads first, then branch-free tests (the
+                // first micropolygon ends in the high bit; reads past ni stay
+                // inside the arrays and their bits are shifted out)
+                uint32_t ph = 0u, pl = 0u;
+                auto test4 = [&](int i, uint32_t acc) -> uint32_t {
+                    unsigned long long mm[4];
+                    float4 sb[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        mm[q] = matM[wave][i0 + i + q];
+                        sb[q] = matB[wave][i0 + i + q];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const bool inB = !(sx < sb[q].x) & !(sx > sb[q].y) & !(sy < sb[q].z) & !(sy > sb[q].w);
+                        const bool in = __builtin_amdgcn_inverse_ballot_w64(mm[q]) & inB;
+                        acc = acc + acc + (uint32_t)in;
+                    }
+                    return acc;
+                };
+                const int ni4 = (ni + 3) & ~3;
+                const int n0 = ni4 < 32 ? ni4 : 32, n1 = ni4 - n0;
+                for (int i = 0; i < n0; i += 4) ph = test4(i, ph);
+                for (int i = 32; i < ni4; i += 4) pl = test4(i, pl);
+                ph = ph << (32 - n0);
+                pl = n1 > 0 ? pl << (32 - n1) : 0u;
+                unsigned long long pb = ((unsigned long long)__builtin_bitreverse32(pl) << 32) |
+                                        (unsigned long long)__builtin_bitreverse32(ph);
+                pb &= lanes_below(ni);
                 // (3) ordered: each lane its own candidates in list order
                 while (__ballot(pb != 0ull)) {
                     bool hit = false;
@@ -3456,13 +3483,16 @@ extern "C" hipError_t rh_launch_sample_mb(hipStream_t st, const SampleLaunch* a,
     return hipGetLastError();
 }
 
-// The depth-of-field form of the sampler: one workgroup per task, tasks
-// [a->itemBase, a->itemBase + ntasks).
-extern "C" hipError_t rh_launch_sample_dof(hipStream_t st, const SampleLaunch* a, int ntasks, const DofTables* t) {
+// The depth-of-field form of the sampler, tasks [a->itemBase, a->itemBase +
+// ntasks).
+// `split` workgroups (1 or more) share a task's passes.
+extern "C" hipError_t rh_launch_sample_dof(hipStream_t st, const SampleLaunch* a, int ntasks, int split,
+                                           const DofTables* t) {
     if (ntasks <= 0) return hipSuccess;
+    if (split < 1) return hipErrorInvalidValue;
 #define RH_LAUNCH_DOF(STORE)                                                                                       \
-    hipLaunchKernelGGL((rh_sample_dof<STORE>), dim3(ntasks), dim3(RH_DOF_WAVES * 64), 0, st, a->fr, a->buckets,     \
-                       a->tasks, a->itemBase, a->capStart, a->listCount, a->lists,                                   \
+    hipLaunchKernelGGL((rh_sample_dof<STORE>), dim3(ntasks * split), dim3(RH_DOF_WAVES * 64), 0, st, a->fr, a->buckets, \
+                       a->tasks, a->itemBase, split, a->capStart, a->listCount, a->lists,                                   \
                        reinterpret_cast<const float4*>(a->mprec), a->grids, a->prims, a->pos2d, a->pos1d,           \
                        a->pixPattern, t->shuffled, t->lens, t->pixDof, t->cells, a->samples, a->hitData, a->hitNext, \
                        a->hitCtl, a->hitShards, a->hitHeads, a->frontDepth, a->rowCounts, a->rowBase, a->idCut, a->itemCut, \
