@@ -54,6 +54,8 @@
 // stored hits, point-in-polygon hits, second Newton steps), 5 tasks whose
 // list overflowed, 6 micropolygon-bucket references, 7 and 8 unused.
 #define RH_NCOUNTERS 9
+// A context's pinned block: the counters, then the first hit control words.
+#define RH_HOST_HITCTL 4
 // Hit-list entries (its occluding hit included) the combine kernels sort in
 // LDS; a sample with more transparent hits goes to the long-list pass.
 #define RH_MAX_HITS 64
@@ -203,6 +205,9 @@ struct DisplayFormat {
 #define RH_DSPY_SIGNED16_D 5
 #define RH_DSPY_UNSIGNED8_D 6
 #define RH_DSPY_SIGNED8_D 7
+
+// Bytes a read-back workgroup copies.
+#define RH_READ_WG_BYTES 65536
 
 // The strip filter's list (rh_filter_strip): the samples of a halo row that
 // add to a pixel, in the reference's order (filter columns, samples), in

@@ -57,6 +57,17 @@ struct WorkPool {
 
     void run(int n, int threads, const std::function<void(int)>& f) {
         std::lock_guard<std::mutex> one(runMutex);
+        run_locked(n, threads, f);
+    }
+
+    bool run_if_free(int n, int threads, const std::function<void(int)>& f) {
+        std::unique_lock<std::mutex> one(runMutex, std::try_to_lock);
+        if (!one.owns_lock()) return false;
+        run_locked(n, threads, f);
+        return true;
+    }
+
+    void run_locked(int n, int threads, const std::function<void(int)>& f) {
         const int helpers = std::min(threads, n) - 1;
         {
             std::unique_lock<std::mutex> lk(m);
@@ -110,6 +121,8 @@ static void run_parallel(int n, int threads, const std::function<void(int)>& fn)
     }
     work_pool().run(n, threads, fn);
 }
+
+bool run_if_free(int n, int threads, const std::function<void(int)>& fn) { return work_pool().run_if_free(n, threads, fn); }
 
 // ---------------------------------------------------------------------------
 // Frame shape

@@ -4,6 +4,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <functional>
 #include <memory>
 #include <string>
 #include <vector>
@@ -206,6 +207,10 @@ inline bool hits_listed(const rh_options& o, const rh_prim& q) {
     if (!cullable_hits(o)) return true;
     return !(q.Os[0] >= 1.0f && q.Os[1] >= 1.0f && q.Os[2] >= 1.0f) && q.matte != RH_MATTE_ALPHA;
 }
+
+// run_parallel's loop on up to `threads` threads of the process's worker pool,
+// the caller taking part; false, with nothing run, when the pool is busy with another loop.
+bool run_if_free(int n, int threads, const std::function<void(int)>& fn);
 
 // build_forest + simulate without occlusion culling.
 bool make_schedule(const Shape& s, const rh_prim* prims, int n, Schedule& out, std::string& err,

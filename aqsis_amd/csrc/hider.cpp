@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <chrono>
 #include <cstdint>
 #include <mutex>
@@ -41,7 +42,8 @@ extern "C" hipError_t rh_launch_combine(hipStream_t, const FrameDev*, size_t, co
                                         uint32_t*, const float4*, const uint2*, const PrimDev*, const float*, int, int,
                                         const GridDev*, int, float4*, float*);
 extern "C" hipError_t rh_launch_reduce_counters(hipStream_t, const uint32_t*, int, const uint32_t*, int,
-                                                unsigned long long*);
+                                                unsigned long long*, const uint32_t*, unsigned long long*);
+extern "C" hipError_t rh_launch_read_back(hipStream_t, const void*, void*, size_t, int, uint32_t*, uint32_t*, uint32_t);
 extern "C" hipError_t rh_launch_format_display(hipStream_t, int, const DisplayFormat*, const float*, const float*,
                                                size_t, void*);
 extern "C" hipError_t rh_launch_box_classes(hipStream_t, const FrameDev*, int, const uchar4*, const float*, uint32_t*);
@@ -131,6 +133,157 @@ template <typename T> hipError_t upload(DBuf& b, const std::vector<T>& v, hipStr
     return hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st);
 }
 
+// Pinned host memory of the process's contexts: a block of counters per
+// context, which the device writes at the end of a frame, and a few lanes
+// through which results are read back.  Taken from the driver when first
+// needed, handed back when the last context is destroyed; at most kLanes
+// lanes, a read that finds none free takes a plain copy.
+constexpr size_t kCtlBytes = 256, kSlabBytes = 64 << 10;
+constexpr int kLanes = 4;
+constexpr size_t kLaneBytes = 16 << 20;   // a 2048x2048 frame's 8-bit image
+constexpr int kLanePieces = kLaneBytes / RH_READ_WG_BYTES;
+
+struct ReadLane {
+    int dev = 0;
+    uint32_t seq = 0;                     // of its last use: what a piece's flag is set to
+    unsigned char* p = nullptr;           // kLaneBytes, then a flag per piece
+    unsigned char* dp = nullptr;          // the device's address of p
+    uint32_t* done = nullptr;             // device: workgroups of each piece that are through
+    volatile uint32_t* flags() const { return reinterpret_cast<volatile uint32_t*>(p + kLaneBytes); }
+};
+
+struct PinnedPool {
+    std::mutex m;
+    int contexts = 0;
+    std::vector<void*> slabs, freeCtl;
+    std::vector<ReadLane*> lanes, freeLanes;
+
+    static PinnedPool& get() {
+        static PinnedPool* p = new PinnedPool();   // kept until the process ends
+        return *p;
+    }
+    // A context's counter block; null when the driver has no pinned memory.
+    void* take_ctl() {
+        std::lock_guard<std::mutex> lk(m);
+        if (freeCtl.empty()) {
+            void* s = nullptr;
+            if (hipHostMalloc(&s, kSlabBytes, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
+            slabs.push_back(s);
+            for (size_t o = 0; o < kSlabBytes; o += kCtlBytes) freeCtl.push_back(static_cast<unsigned char*>(s) + o);
+        }
+        void* p = freeCtl.back();
+        freeCtl.pop_back();
+        ++contexts;
+        return p;
+    }
+    void give_ctl(void* p) {
+        std::lock_guard<std::mutex> lk(m);
+        freeCtl.push_back(p);
+        if (--contexts > 0) return;
+        for (void* s : slabs) (void)hipHostFree(s);
+        slabs.clear();
+        freeCtl.clear();
+        for (ReadLane* l : freeLanes) drop(l);
+        freeLanes.clear();
+    }
+    ReadLane* take_lane(int dev) {
+        std::lock_guard<std::mutex> lk(m);
+        for (size_t i = 0; i < freeLanes.size(); ++i)
+            if (freeLanes[i]->dev == dev) {
+                ReadLane* l = freeLanes[i];
+                freeLanes.erase(freeLanes.begin() + (long)i);
+                return l;
+            }
+        if ((int)lanes.size() >= kLanes) return nullptr;
+        ReadLane* l = new (std::nothrow) ReadLane();
+        if (!l) return nullptr;
+        l->dev = dev;
+        lanes.push_back(l);
+        const size_t flagBytes = kLanePieces * sizeof(uint32_t);
+        if (hipHostMalloc(reinterpret_cast<void**>(&l->p), kLaneBytes + flagBytes,
+                          hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess ||
+            hipHostGetDevicePointer(reinterpret_cast<void**>(&l->dp), l->p, 0) != hipSuccess ||
+            hipMalloc(reinterpret_cast<void**>(&l->done), flagBytes) != hipSuccess ||
+            hipMemset(l->done, 0, flagBytes) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGetLastError();
+            drop(l);
+            return nullptr;
+        }
+        std::memset(l->p + kLaneBytes, 0, flagBytes);
+        return l;
+    }
+    void give_lane(ReadLane* l) {
+        std::lock_guard<std::mutex> lk(m);
+        if (contexts > 0) freeLanes.push_back(l);
+        else drop(l);
+    }
+
+private:
+    void drop(ReadLane* l) {
+        if (l->done) (void)hipFree(l->done);
+        if (l->p) (void)hipHostFree(l->p);
+        lanes.erase(std::find(lanes.begin(), lanes.end(), l));
+        delete l;
+    }
+};
+
+// Copy a result from the device, on its context's stream.  A plain copy into
+// pageable memory costs about 15 us and runs at 17 GB/s (one thread copies
+// out of the runtime's staging memory), an asynchronous copy of a piece 30
+// us; so a kernel writes the result into a lane and sets a flag after each
+// piece, and up to 8 of the worker pool's threads copy the pieces on as they
+// arrive: 0.26 MB 127 to 33 us, 2.4 MB 141 to 90, 8.3 MB 485 to 280 (30
+// GB/s), 16.8 MB 966 to 460.
+// dst may be any host memory; src a context's buffer (read to a multiple of 16 bytes).
+constexpr size_t kReadPlain = 64 << 10;   // bytes below which the plain copy stays
+
+hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    ReadLane* lane = bytes >= kReadPlain ? PinnedPool::get().take_lane(dev) : nullptr;
+    if (!lane) {
+        e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
+        return e == hipSuccess ? hipStreamSynchronize(st) : e;
+    }
+    for (size_t from = 0; from < bytes && e == hipSuccess; from += kLaneBytes) {
+        const size_t len = std::min(kLaneBytes, bytes - from);
+        unsigned char* to = static_cast<unsigned char*>(dst) + from;
+        // up to 16 pieces of whole workgroups, 256 KB at least
+        size_t piece = std::max<size_t>(256 << 10, (len + 15) / 16);
+        piece = (piece + RH_READ_WG_BYTES - 1) / RH_READ_WG_BYTES * RH_READ_WG_BYTES;
+        const int n = (int)((len + piece - 1) / piece);
+        const uint32_t seq = ++lane->seq;
+        e = rh_launch_read_back(st, static_cast<const unsigned char*>(src) + from, lane->dp, len, (int)(piece / RH_READ_WG_BYTES),
+                                lane->done, reinterpret_cast<uint32_t*>(lane->dp + kLaneBytes), seq);
+        if (e != hipSuccess) break;
+        std::atomic<bool> lost{false};
+        auto take = [&](int i) {
+            const size_t at = (size_t)i * piece;
+            for (uint32_t spin = 0; lane->flags()[i] != seq; ++spin) {
+                // a stream that is through without the flag has failed
+                if ((spin & 0xfff) == 0xfff && hipStreamQuery(st) != hipErrorNotReady && lane->flags()[i] != seq) {
+                    lost = true;
+                    return;
+                }
+                __builtin_ia32_pause();
+            }
+            std::atomic_thread_fence(std::memory_order_acquire);
+            std::memcpy(to + at, lane->p + at, std::min(piece, len - at));
+        };
+        if (n == 1 || !rh::run_if_free(n, 8, take))
+            for (int i = 0; i < n; ++i) take(i);
+        // nothing may still be writing to the lane when it is used again
+        e = hipStreamSynchronize(st);
+        if (e == hipSuccess && lost) e = hipErrorUnknown;
+    }
+    PinnedPool::get().give_lane(lane);
+    return e;
+}
+
 double ms_since(std::chrono::steady_clock::time_point t0) {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
@@ -191,6 +344,9 @@ struct rh_ctx {
         graph = nullptr;
     }
     void* scratch = nullptr;              // this device's scratch array (rh_render_device_noalloc)
+    // pinned: a frame's counters and hit control words as its last kernels leave them
+    unsigned long long* hostCtl = nullptr;
+    unsigned long long* hostCtlDev = nullptr;   // the device's address of it
     FrameDev frame;                       // host copy of dFrame
     rh_stats stats;
     DofTables dof() const {
@@ -220,6 +376,7 @@ struct rh_ctx {
         for (auto& e : ev)
             if (e) (void)hipEventDestroy(e);
         if (st) (void)hipStreamDestroy(st);
+        if (hostCtl) PinnedPool::get().give_ctl(hostCtl);
     }
 };
 
@@ -533,6 +690,11 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
     keep_pool_memory();
     hipError_t e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
     c->each_buffer([c](DBuf& b) { b.st = c->st; });
+    if (e == hipSuccess) {
+        c->hostCtl = static_cast<unsigned long long*>(PinnedPool::get().take_ctl());
+        if (!c->hostCtl) { delete c; return fail(RH_ERR_NOMEM, "no pinned host memory"); }
+        e = hipHostGetDevicePointer(reinterpret_cast<void**>(&c->hostCtlDev), c->hostCtl, 0);
+    }
     for (int i = 0; i < 6 && e == hipSuccess; ++i) e = hipEventCreate(&c->ev[i]);
     if (e != hipSuccess) { delete c; return fail(RH_ERR_DEVICE, std::string("stream/event creation: ") + hipGetErrorString(e)); }
 
@@ -968,7 +1130,8 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
                               c->dSamples.as<float4>(),
                               c->dFrontDepth.as<float>()));
     if (timed) ENQ(hipEventRecord(c->ev[3], c->st));
-    ENQ(rh_launch_reduce_counters(c->st, k.rows, rows, c->dBucketRefs.as<uint32_t>(), nb, k.counters));
+    ENQ(rh_launch_reduce_counters(c->st, k.rows, rows, c->dBucketRefs.as<uint32_t>(), nb, k.counters, k.hitCtl,
+                                  c->hostCtlDev));
     ENQ(enqueue_filter(c));
     if (timed) ENQ(hipEventRecord(c->ev[4], c->st));
 #undef ENQ
@@ -1209,6 +1372,13 @@ static rh_status cull_schedule(rh_ctx* c, const rh::Forest& forest) {
 
 static rh_status finish_frame(rh_ctx* c, const unsigned long long* cnt, bool staged);
 
+// A completed frame's counters and hit control words.
+static void read_ctl(const rh_ctx* c, unsigned long long* cnt, uint32_t* hc) {
+    const volatile unsigned long long* h = c->hostCtl;
+    for (int i = 0; i < RH_NCOUNTERS; ++i) cnt[i] = i < 7 ? h[i] : 0ull;
+    for (int i = 0; i < RH_HOST_HITCTL; ++i) hc[i] = (uint32_t)h[RH_NCOUNTERS + i];
+}
+
 // One frame on the resident inputs.  The batched form replays its frame
 // graph unless `eager` asks for the same launches issued one by one with a
 // timestamp between the stages.
@@ -1246,9 +1416,8 @@ static rh_status render_frame(rh_ctx* c, bool eager) {
             HIP_TRY(enqueue_frame(c, true, context_ctl(c)));
         }
         HIP_TRY(hipEventSynchronize(c->ev[4]));
-        HIP_TRY(hipMemcpy(cnt, c->dCounters.p, sizeof(cnt), hipMemcpyDeviceToHost));
-        uint32_t hc[4];
-        HIP_TRY(hipMemcpy(hc, c->dHitCtl.p, sizeof(hc), hipMemcpyDeviceToHost));
+        uint32_t hc[RH_HOST_HITCTL];
+        read_ctl(c, cnt, hc);
         if (hc[0] > 0) {
             // The arena ran out: redo the frame with room for every hit.
             if (attempt >= 2) return fail(RH_ERR_CAPACITY, "transparent-hit arena kept overflowing");
@@ -1330,9 +1499,8 @@ rh_status rh_render_device_noalloc(rh_ctx* c) {
     HIP_TRY(enqueue_frame(c, true, k, true));
     HIP_TRY(hipEventSynchronize(c->ev[4]));
     unsigned long long cnt[RH_NCOUNTERS];
-    uint32_t hc[4];
-    HIP_TRY(hipMemcpy(cnt, k.counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(hc, k.hitCtl, sizeof(hc), hipMemcpyDeviceToHost));
+    uint32_t hc[RH_HOST_HITCTL];
+    read_ctl(c, cnt, hc);
     if (hc[0] > 0)
         return fail(RH_ERR_CAPACITY, "the frame needs " + std::to_string((uint64_t)c->frame.hitCapacity + hc[0]) +
                                          " transparent-hit entries and the "
@@ -1429,15 +1597,14 @@ rh_status rh_frame_size(const rh_ctx* c, int32_t* w, int32_t* h, int32_t* ew, in
 rh_status rh_read_channels(rh_ctx* c, float* out) {
     if (!c || !out) return fail(RH_ERR_INVALID, "bad arguments");
     if (!c->rendered) return fail(RH_ERR_STATE, "no rendered frame");
-    HIP_TRY(hipMemcpy(out, c->dChannels.p, (size_t)c->shape.width() * c->shape.height() * 9 * sizeof(float),
-                      hipMemcpyDeviceToHost));
+    HIP_TRY(read_back(out, c->dChannels.p, (size_t)c->shape.width() * c->shape.height() * 9 * sizeof(float), c->st));
     return RH_OK;
 }
 
 rh_status rh_read_rgba8(rh_ctx* c, uint8_t* out) {
     if (!c || !out) return fail(RH_ERR_INVALID, "bad arguments");
     if (!c->rendered) return fail(RH_ERR_STATE, "no rendered frame");
-    HIP_TRY(hipMemcpy(out, c->dRgba.p, (size_t)c->shape.width() * c->shape.height() * 4, hipMemcpyDeviceToHost));
+    HIP_TRY(read_back(out, c->dRgba.p, (size_t)c->shape.width() * c->shape.height() * 4, c->st));
     return RH_OK;
 }
 
@@ -1475,8 +1642,7 @@ static rh_status format_frame(rh_ctx* c, const DisplayFormat& f, int32_t type, c
     }
     HIP_TRY(c->dFormat.ensure(bytes));
     HIP_TRY(rh_launch_format_display(c->st, type, &f, c->dChannels.as<float>(), dither, npix, c->dFormat.p));
-    HIP_TRY(hipMemcpyAsync(out, c->dFormat.p, bytes, hipMemcpyDeviceToHost, c->st));
-    HIP_TRY(hipStreamSynchronize(c->st));
+    HIP_TRY(read_back(out, c->dFormat.p, bytes, c->st));
     return RH_OK;
 }
 
@@ -1485,7 +1651,7 @@ static rh_status display_values(rh_ctx* c, int32_t type, void* out) {
     const rh::Shape& s = c->shape;
     if (type == RH_DSPY_UNSIGNED8 && rh::display_type(s.o) == RH_DSPY_UNSIGNED8) {
         // the filter quantised these already
-        HIP_TRY(hipMemcpy(out, c->dRgba.p, (size_t)s.width() * s.height() * 4, hipMemcpyDeviceToHost));
+        HIP_TRY(read_back(out, c->dRgba.p, (size_t)s.width() * s.height() * 4, c->st));
         return RH_OK;
     }
     const DisplayFormat f{s.o.quantize_one, s.o.quantize_min, s.o.quantize_max, s.o.quantize_dither, 4, 0x6210u};

@@ -664,11 +664,16 @@ __global__ void __launch_bounds__(256) rh_bin_write(const FrameDev* __restrict__
 }
 
 // Frame counters from the sampling rows and per-bucket rows: counters[0..4] the
-// hider's SPL counts, counters[6] the micropolygon-bucket references.
+// hider's SPL counts, counters[6] the micropolygon-bucket references.  `host`:
+// the counters and the first hit control words once more, in pinned host
+// memory (hostCtl of a context), so that the host reads them after the frame
+// without a copy (two blocking copies took 25 us of every frame).
 // One workgroup.
 __global__ void __launch_bounds__(1024) rh_reduce_counters(const uint32_t* __restrict__ rowCounts, int nrows,
                                                            const uint32_t* __restrict__ bucketRefs, int nbuckets,
-                                                           unsigned long long* __restrict__ counters) {
+                                                           unsigned long long* __restrict__ counters,
+                                                           const uint32_t* __restrict__ hitCtl,
+                                                           unsigned long long* __restrict__ host) {
     __shared__ unsigned long long part[6][32];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     unsigned long long acc[6] = {0, 0, 0, 0, 0, 0};
@@ -685,7 +690,13 @@ __global__ void __launch_bounds__(1024) rh_reduce_counters(const uint32_t* __res
         unsigned long long v = 0;
         for (int w = 0; w < 16; ++w) v += part[tid][w];
         counters[tid < 5 ? tid : 6] = v;
+        host[tid < 5 ? tid : 6] = v;
+    } else if (tid < 6 + RH_HOST_HITCTL) {
+        host[RH_NCOUNTERS + tid - 6] = hitCtl[tid - 6];
+    } else if (tid == 6 + RH_HOST_HITCTL) {
+        host[5] = counters[5];            // counted while the lists were built
     }
+    __threadfence_system();
 }
 
 // ---------------------------------------------------------------------------
@@ -2804,6 +2815,40 @@ __device__ __forceinline__ void filter_pixel(const FrameDev* __restrict__ fr, co
     finish_pixel<GAMMA>(fr, acc, gTot, count, ns, t, dither, channels, rgba8);
 }
 
+// Read-back: `bytes` bytes (rounded up to 16) of a result into pinned host
+// memory, RH_READ_WG_BYTES a workgroup; the last workgroup of each piece of
+// `per` sets the piece's flag in host memory to `seq` (and its device counter
+// back to 0), after every store of the piece is visible to the host.
+__global__ void __launch_bounds__(256) rh_read_back(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t bytes,
+                                                    int per, uint32_t* __restrict__ done,
+                                                    volatile uint32_t* __restrict__ flags, uint32_t seq) {
+    const size_t n = (bytes + 15) / 16, base = (size_t)blockIdx.x * (RH_READ_WG_BYTES / 16);
+    uint4 v[4];
+    for (int k = 0; k < RH_READ_WG_BYTES / 16 / 256; k += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const size_t i = base + (size_t)(k + u) * 256 + threadIdx.x;
+            if (i < n) v[u] = src[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const size_t i = base + (size_t)(k + u) * 256 + threadIdx.x;
+            if (i < n) dst[i] = v[u];
+        }
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int piece = (int)blockIdx.x / per;
+        const int wgs = min(per, (int)gridDim.x - piece * per);
+        if (atomicAdd(&done[piece], 1u) == (uint32_t)wgs - 1u) {
+            done[piece] = 0u;
+            __threadfence_system();
+            flags[piece] = seq;
+        }
+    }
+}
+
 // A display request's values of each pixel (FormatBucketForDisplay,
 // ddmanager.cpp:1045-1118): the channels `f` names, quantised when f.one != 0,
 // stored as T with x86-64's conversions (a NaN or a value outside the 32-bit
@@ -3584,11 +3629,21 @@ extern "C" hipError_t rh_launch_frame_begin(hipStream_t st, unsigned long long* 
 
 extern "C" hipError_t rh_launch_reduce_counters(hipStream_t st, const uint32_t* taskCounts, int ntasks,
                                                 const uint32_t* bucketRefs, int nbuckets,
-                                                unsigned long long* counters) {
+                                                unsigned long long* counters, const uint32_t* hitCtl,
+                                                unsigned long long* host) {
     hipLaunchKernelGGL(rh_reduce_counters, dim3(1), dim3(1024), 0, st, taskCounts, ntasks, bucketRefs, nbuckets,
-                       counters);
+                       counters, hitCtl, host);
     return hipGetLastError();
 }
+extern "C" hipError_t rh_launch_read_back(hipStream_t st, const void* src, void* dst, size_t bytes, int per,
+                                          uint32_t* done, uint32_t* flags, uint32_t seq) {
+    if (bytes == 0 || per < 1) return hipErrorInvalidValue;
+    const unsigned wgs = (unsigned)((bytes + RH_READ_WG_BYTES - 1) / RH_READ_WG_BYTES);
+    hipLaunchKernelGGL(rh_read_back, dim3(wgs), dim3(256), 0, st, static_cast<const uint4*>(src),
+                       static_cast<uint4*>(dst), bytes, per, done, flags, seq);
+    return hipGetLastError();
+}
+
 // npix pixels' values of type `type` (RH_DSPY_*) into out.
 extern "C" hipError_t rh_launch_format_display(hipStream_t st, int type, const DisplayFormat* f, const float* channels,
                                                const float* dither, size_t npix, void* out) {

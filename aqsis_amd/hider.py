@@ -178,12 +178,12 @@ class Hider:
         _check(lib().rh_render_stages(self._ctx))
 
     def channels(self):
-        out = np.zeros((self.height, self.width, 9), np.float32)
+        out = np.empty((self.height, self.width, 9), np.float32)
         _check(lib().rh_read_channels(self._ctx, _ptr(out)))
         return out
 
     def rgba8(self):
-        out = np.zeros((self.height, self.width, 4), np.uint8)
+        out = np.empty((self.height, self.width, 4), np.uint8)
         _check(lib().rh_read_rgba8(self._ctx, _ptr(out)))
         return out
 
@@ -192,7 +192,7 @@ class Hider:
         FormatBucketForDisplay gives them, of RH_DSPY_* `type` (default the
         type the Quantize settings select) (rh_read_display)."""
         t = self.display_type if type is None else (DSPY[type] if isinstance(type, str) else int(type))
-        out = np.zeros((self.height, self.width, 4), DSPY_DTYPE[t])
+        out = np.empty((self.height, self.width, 4), DSPY_DTYPE[t])
         _check(lib().rh_read_display(self._ctx, t, _ptr(out)))
         return out
 
@@ -213,7 +213,7 @@ class Hider:
         else:
             t = DSPY[type] if isinstance(type, str) else int(type)
         k = (1 if m & MODE_A else 0) + (3 if m & MODE_RGB else 0) + (1 if m & MODE_Z else 0)
-        out = np.zeros((self.height, self.width, max(k, 1)), DSPY_DTYPE.get(t, np.uint8))
+        out = np.empty((self.height, self.width, max(k, 1)), DSPY_DTYPE.get(t, np.uint8))
         _check(lib().rh_read_display_request(self._ctx, m, _ptr(q), index, t, _ptr(out)))
         return out
 
@@ -255,9 +255,9 @@ class Hider:
 
     def samples(self):
         n = self.ext_width * self.ext_height * self.spp
-        ids = np.zeros(n, np.uint32)
-        depth = np.zeros(n, np.float32)
-        rgbaz = np.zeros((n, 7), np.float32)
+        ids = np.empty(n, np.uint32)
+        depth = np.empty(n, np.float32)
+        rgbaz = np.empty((n, 7), np.float32)
         _check(lib().rh_read_samples(self._ctx, _ptr(ids), _ptr(depth), _ptr(rgbaz)))
         return ids, depth, rgbaz
 
