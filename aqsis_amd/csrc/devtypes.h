@@ -34,14 +34,12 @@
 //  [0..7]   raster x, y of the four vertices in grid order
 //           (iu,iv), (iu+1,iv), (iu,iv+1), (iu+1,iv+1)
 //  [8..11]  vertex depths z0..z3 (camera z, grid order)
-//  [12..15] bound min x, max x, min y, max y
-//  [16]     bound min z
-//  [17]     flags (int bits): vertex-order code (bits 0..7), degenerate (8),
+//  [12]     flags (int bits): vertex-order code (bits 0..7), degenerate (8),
 //           linear, i.e. one Newton step (9), opaque: Oi >= (1,1,1)
 //           component-wise, color.h:432-435 (10)
-//  [18]     grid index (int bits)  [19] surface (int bits)
-#define RH_MPREC_FLOATS 20
-#define RH_MPREC_GRID 18
+//  [13]     grid index (int bits)  [14] surface (int bits)  [15] unused
+#define RH_MPREC_FLOATS 16
+#define RH_MPREC_GRID 13
 // Motion-frame micropolygon record, in floats:
 //  [0..11]  key 0: x, y, z of the four vertices in grid order
 //  [12..23] key 1 (a static micropolygon repeats key 0)

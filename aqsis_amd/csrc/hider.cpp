@@ -965,7 +965,7 @@ static rh_status upload_schedule(rh_ctx* c) {
     HIP_TRY(upload(c->dSegBucket, S.segBucket, c->st));
     HIP_TRY(c->dSegCounts.ensure(S.candGrid.size() * 17 * sizeof(uint32_t)));
     HIP_TRY(upload(c->dCapStart, cap, c->st));
-    HIP_TRY(c->dMprec.ensure(S.micropolygons * RH_MPREC_FLOATS * sizeof(float)));
+    if (!S.motion) HIP_TRY(c->dMprec.ensure(S.micropolygons * RH_MPREC_FLOATS * sizeof(float)));
     HIP_TRY(c->dMpbound.ensure(S.micropolygons * sizeof(float4)));
     HIP_TRY(c->dLists.ensure((size_t)S.capStart.back() * sizeof(uint32_t)));
     if (S.motion) HIP_TRY(c->dMprecMB.ensure(S.micropolygons * RH_MPREC_MB_FLOATS * sizeof(float)));
@@ -1813,8 +1813,8 @@ static uint64_t frame_bytes(const rh::Shape& s) {
 static uint64_t footprint_bytes(const rh::Shape& s, const rh::Schedule& S, const rh_prim* prims, int32_t n) {
     uint64_t bytes = frame_bytes(s) + S.grids.size() * sizeof(GridDev) + S.paramFloats * 4 +
                      (uint64_t)n * sizeof(PrimDev) + S.candGrid.size() * (4 + 4 + 17 * 4) +
-                     S.micropolygons * (RH_MPREC_FLOATS * 4 + 16) + S.capStart.back() * 4 +
-                     (S.motion ? S.micropolygons * RH_MPREC_MB_FLOATS * 4 : 0);
+                     S.micropolygons * ((S.motion ? RH_MPREC_MB_FLOATS : RH_MPREC_FLOATS) * 4 + 16) +
+                     S.capStart.back() * 4;
     bool transparent = false;
     for (int32_t i = 0; i < n; ++i)
         if (rh::hits_listed(s.o, prims[i])) transparent = true;

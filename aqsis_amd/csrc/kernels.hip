@@ -253,13 +253,23 @@ __device__ __forceinline__ int key_param_floats(int type, int cu, int cv) {
                                   : (type == RH_PRIM_BICUBIC ? 48 : 12);
 }
 
+// MB: a frame with moving micropolygons (the records the motion sampler reads
+// instead of the static ones).  Bound by the latency of a grid's chain (its
+// parameters, the forward differences) and by HBM writes, so by the grids a CU
+// holds and the bytes a micropolygon takes: without key 1's vertices in LDS 7
+// workgroups a CU instead of 5, and 64 bytes of record instead of 80 (the
+// sampler finds the bound and the least depth from the vertices again, the
+// same comparisons).  1920x1080 patches 272 -> 213 us, 2048x2048 of 4x4-vertex
+// patches 1850 -> 1438 us, and the static sampler, which reads the shorter
+// records, 1613 -> 1578 and 5900 -> 5870 us.
+template <bool MB>
 __global__ void __launch_bounds__(256) rh_dice_bust(const FrameDev* __restrict__ fr, const GridDev* __restrict__ grids,
                                                     const PrimDev* __restrict__ prims,
                                                     const float* __restrict__ params,
                                                     float* __restrict__ mprec, float4* __restrict__ mpbound,
                                                     float4* __restrict__ mprecMB) {
     __shared__ float4 V[RH_MAX_GRID_VERTS];
-    __shared__ float4 V1[RH_MAX_GRID_VERTS];
+    __shared__ float4 V1[MB ? RH_MAX_GRID_VERTS : 1];
     __shared__ float rows[4 * RH_MAX_GRID_ROWS * 3];
     const int tid = threadIdx.x;
     const GridDev G = grids[blockIdx.x];
@@ -267,7 +277,7 @@ __global__ void __launch_bounds__(256) rh_dice_bust(const FrameDev* __restrict__
     const float* prm = params + G.paramOff;
 
     const int type = G.type & ~RH_GRID_MOTION;
-    const bool motion = (G.type & RH_GRID_MOTION) != 0;
+    const bool motion = MB && (G.type & RH_GRID_MOTION) != 0;
     dice_points(type, cu, cv, prm, V, rows);
     __syncthreads();
     // Projection to hybrid raster space keeping camera z (micropolygon.cpp:723-731)
@@ -343,15 +353,14 @@ __global__ void __launch_bounds__(256) rh_dice_bust(const FrameDev* __restrict__
         // occluding hits as an opaque one's (bucketprocessor.cpp:1490-1491)
         const PrimDev& Pr = prims[G.prim];
         const bool opaque = (Pr.Oi[0] >= 1.0f && Pr.Oi[1] >= 1.0f && Pr.Oi[2] >= 1.0f) || Pr.matte == RH_DEV_MATTE_ALPHA;
-        float4* out = reinterpret_cast<float4*>(mprec + (size_t)(G.mpBase + m) * RH_MPREC_FLOATS);
         const uint32_t flags = (uint32_t)(code & 0xff) | (degen ? 1u << 8 : 0u) | (linear ? 1u << 9 : 0u) |
                                (opaque ? 1u << 10 : 0u);
-        out[0] = make_float4(P[0].x, P[0].y, P[1].x, P[1].y);
-        out[1] = make_float4(P[2].x, P[2].y, P[3].x, P[3].y);
-        out[2] = make_float4(P[0].z, P[1].z, P[2].z, P[3].z);
-        out[3] = make_float4(bminx, bmaxx, bminy, bmaxy);
-        out[4] = make_float4(bminz, __uint_as_float(flags), __int_as_float((int)blockIdx.x), __int_as_float(G.prim));
-        if (!mprecMB) {
+        if (!MB) {
+            float4* out = reinterpret_cast<float4*>(mprec + (size_t)(G.mpBase + m) * RH_MPREC_FLOATS);
+            out[0] = make_float4(P[0].x, P[0].y, P[1].x, P[1].y);
+            out[1] = make_float4(P[2].x, P[2].y, P[3].x, P[3].y);
+            out[2] = make_float4(P[0].z, P[1].z, P[2].z, P[3].z);
+            out[3] = make_float4(__uint_as_float(flags), __int_as_float((int)blockIdx.x), __int_as_float(G.prim), 0.0f);
             if (fr->dofOn) {
                 // AddMPG grows the bound by the larger circle of confusion at
                 // its two depths (imagebuffer.cpp:519-530); binning reads it
@@ -752,9 +761,20 @@ __device__ __forceinline__ float pick4(int i, float a0, float a1, float a2, floa
     return i == 0 ? a0 : (i == 1 ? a1 : (i == 2 ? a2 : a3));
 }
 
+// CalculateBound (micropolygon.cpp:1663-1673) of a compact record's vertices:
+// (min x, max x, min y, max y), and the least depth; A, B, C, D are vertices
+// 0, 1, 3, 2.
+__device__ __forceinline__ float4 record_bound(const float4 a, const float4 b) {
+    return make_float4(fmin_ref(fmin_ref(fmin_ref(a.x, a.z), b.z), b.x), fmax_ref(fmax_ref(fmax_ref(a.x, a.z), b.z), b.x),
+                       fmin_ref(fmin_ref(fmin_ref(a.y, a.w), b.w), b.y), fmax_ref(fmax_ref(fmax_ref(a.y, a.w), b.w), b.y));
+}
+__device__ __forceinline__ float record_minz(const float4 z) {
+    return fmin_ref(fmin_ref(fmin_ref(z.x, z.y), z.w), z.z);
+}
+
 __device__ __forceinline__ void expand_record(const float4* __restrict__ src, uint32_t id, float4* out) {
-    const float4 a = src[0], b = src[1], zz = src[2], bd = src[3], r4 = src[4];
-    const uint32_t fl = __float_as_uint(r4.y);
+    const float4 a = src[0], b = src[1], zz = src[2], r3 = src[3];
+    const uint32_t fl = __float_as_uint(r3.x);
     const int code = (int)(fl & 0xffu);
     const bool degen = (fl >> 8) & 1u;
     // the vertices in the order the code gives
@@ -793,8 +813,8 @@ __device__ __forceinline__ void expand_record(const float4* __restrict__ src, ui
     out[4] = zz;
     out[5] = make_float4(a.x, a.y, Ex, Ey);
     out[6] = make_float4(Fx, Fy, Gx, Gy);
-    out[7] = bd;
-    out[8] = make_float4(r4.x, __uint_as_float((fl >> 9) & 3u), r4.w, __uint_as_float(id));
+    out[7] = record_bound(a, b);
+    out[8] = make_float4(record_minz(zz), __uint_as_float((fl >> 9) & 3u), r3.z, __uint_as_float(id));
 }
 
 // Colour and opacity of a hit: InterpolateOutputs (micropolygon.cpp:
@@ -1269,8 +1289,7 @@ rh_sample(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets
             const size_t sidx = ((size_t)(py - fr->extY0) * fr->extW + (px - fr->extX0)) * ns + si;
             float4 a = make_float4(0.f, 0.f, 0.f, FLT_MAX), b = make_float4(0.f, 0.f, 0.f, __uint_as_float(win[k]));
             if (win[k] != 0xffffffffu) {
-                const float4 r8 = mprec4[(size_t)win[k] * (RH_MPREC_FLOATS / 4) + 4];
-                const PrimDev& P = prims[__float_as_uint(r8.w)];
+                const PrimDev& P = prims[__float_as_uint(mprec4[(size_t)win[k] * (RH_MPREC_FLOATS / 4) + 3].z)];
                 shade_hit(P, wu[k], wv[k], MID ? sD[k] : occlZ[k], win[k], a, b);
                 finish_occluding(fr, P, nh[k] > 0, depthOnly, occlZ[k], a, b);
             }
@@ -2202,7 +2221,8 @@ rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buc
             if (tid < cnt) {
                 const uint32_t id = L[c0 + tid];
                 const float4* src = mprec4 + (size_t)id * (RH_MPREC_FLOATS / 4);
-                const float4 a = src[0], b = src[1], zz = src[2], bd = src[3], r4 = src[4];
+                const float4 a = src[0], b = src[1], zz = src[2], r3 = src[3], bd = record_bound(a, b);
+                const float minz = record_minz(zz);
                 // CacheHitTestValues with DoF (micropolygon.cpp:1394-1421):
                 // each vertex's CoC, their component-wise least and largest
                 const float2 c0v = dof_coc(fr, zz.x), c1v = dof_coc(fr, zz.y), c2v = dof_coc(fr, zz.z),
@@ -2214,15 +2234,15 @@ rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buc
                 // the larger CoC at the bound's depths (CalculateBound's
                 // order: A, B, C = vertex 3, D = vertex 2)
                 const float bmaxz = fmax_ref(fmax_ref(fmax_ref(zz.x, zz.y), zz.w), zz.z);
-                const float2 cz0 = dof_coc(fr, r4.x), cz1 = dof_coc(fr, bmaxz);
+                const float2 cz0 = dof_coc(fr, minz), cz1 = dof_coc(fr, bmaxz);
                 float4* R = &recs[tid * 9];
                 R[0] = a; R[1] = b; R[2] = zz; R[3] = bd;
-                R[4] = make_float4(r4.x, r4.y, r4.w, __uint_as_float(id));
+                R[4] = make_float4(minz, r3.x, r3.z, __uint_as_float(id));
                 R[5] = make_float4(c0v.x, c0v.y, c1v.x, c1v.y);
                 R[6] = make_float4(c2v.x, c2v.y, c3v.x, c3v.y);
                 R[7] = make_float4(cminx, cminy, cmaxx, cmaxy);
                 R[8] = make_float4(fmax_ref(cz0.x, cz1.x), fmax_ref(cz0.y, cz1.y),
-                                   (bmaxz < fr->clipNear || r4.x > fr->clipFar) ? 1.0f : 0.0f, 0.0f);
+                                   (bmaxz < fr->clipNear || minz > fr->clipFar) ? 1.0f : 0.0f, 0.0f);
             }
             __syncthreads();
             if (!has) continue;
@@ -2372,8 +2392,7 @@ rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buc
         if (!live) continue;
         float4 A = make_float4(0.f, 0.f, 0.f, FLT_MAX), Bv = make_float4(0.f, 0.f, 0.f, __uint_as_float(win));
         if (win != 0xffffffffu) {
-            const float4 r4 = mprec4[(size_t)win * (RH_MPREC_FLOATS / 4) + 4];
-            const PrimDev& P = prims[__float_as_uint(r4.w)];
+            const PrimDev& P = prims[__float_as_uint(mprec4[(size_t)win * (RH_MPREC_FLOATS / 4) + 3].z)];
             shade_hit(P, wu, wv, sD, win, A, Bv);
             finish_occluding(fr, P, nh > 0, depthOnly, occlZ, A, Bv);
         }
@@ -3411,8 +3430,12 @@ extern "C" hipError_t rh_launch_dice(hipStream_t st, const FrameDev* fr, const G
                                      const PrimDev* prims, const float* params, float* mprec,
                                      float4* mpbound, float4* mprecMB) {
     if (ngrids <= 0) return hipSuccess;
-    hipLaunchKernelGGL(rh_dice_bust, dim3(ngrids), dim3(256), 0, st, fr, grids, prims, params, mprec,
-                       mpbound, mprecMB);
+    if (mprecMB)
+        hipLaunchKernelGGL(rh_dice_bust<true>, dim3(ngrids), dim3(256), 0, st, fr, grids, prims, params, mprec,
+                           mpbound, mprecMB);
+    else
+        hipLaunchKernelGGL(rh_dice_bust<false>, dim3(ngrids), dim3(256), 0, st, fr, grids, prims, params, mprec,
+                           mpbound, mprecMB);
     return hipGetLastError();
 }
 
