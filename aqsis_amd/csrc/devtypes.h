@@ -29,6 +29,10 @@
 // Largest grid: u*v <= 256 micropolygons gives at most 2 x 257 vertices.
 #define RH_MAX_GRID_VERTS 514
 #define RH_MAX_GRID_ROWS 257
+// The binning takes a grid's micropolygons 64 at a time, and keeps per segment
+// (bucket, candidate grid) a mask for each step and task of a square of tasks.
+#define RH_GRID_STEPS 4
+#define RH_SEG_MASKS(side) (RH_GRID_STEPS * ((side) <= 2 ? 4 : 16))
 // Micropolygon record, in floats (the sampler rebuilds edge equations and
 // the inverse-bilinear set-up from it when it stages a record):
 //  [0..7]   raster x, y of the four vertices in grid order

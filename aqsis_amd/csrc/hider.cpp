@@ -14,6 +14,7 @@
 #include <new>
 #include <string>
 #include <thread>
+#include <tuple>
 #include <vector>
 
 #include "../../include/aqsis_hider.h"
@@ -26,8 +27,8 @@ extern "C" hipError_t rh_launch_dice(hipStream_t, const FrameDev*, const GridDev
 extern "C" hipError_t rh_launch_sample_mb(hipStream_t, const SampleLaunch*, int, const float4*);
 extern "C" hipError_t rh_launch_bin(hipStream_t, const FrameDev*, const BucketDev*, int, const TaskDev*,
                                     const GridDev*, const uint32_t*, const uint32_t*, const uint32_t*, size_t,
-                                    const unsigned long long*, const float4*, uint32_t*, uint32_t*, uint32_t*,
-                                    uint32_t*, unsigned long long*, int, int, const float4*);
+                                    const unsigned long long*, const float4*, uint32_t*, unsigned long long*, uint32_t*,
+                                    uint32_t*, uint32_t*, unsigned long long*, int, int, const float4*);
 extern "C" hipError_t rh_launch_sample(hipStream_t, int, int, const SampleLaunch*);
 extern "C" hipError_t rh_launch_sample_dof(hipStream_t, const SampleLaunch*, int, int, const DofTables*);
 extern "C" hipError_t rh_sample_occupancy(int, int*);
@@ -315,7 +316,7 @@ struct rh_ctx {
     std::vector<uint32_t> filtHost;
     DBuf dFiltList;
     // schedule
-    DBuf dGrids, dParams, dPrims, dCandStart, dCandGrid, dCapStart, dSegBucket, dSegCounts;
+    DBuf dGrids, dParams, dPrims, dCandStart, dCandGrid, dCapStart, dSegBucket, dSegCounts, dSegMasks;
     // per frame
     DBuf dMprec, dMpbound, dLists, dListCount, dSamples, dChannels, dRgba, dCounters, dBucketRefs;
     DBuf dMprecMB;                        // motion-frame micropolygon records
@@ -364,7 +365,7 @@ struct rh_ctx {
                        &dPrims, &dCandStart, &dCandGrid, &dCapStart, &dMprec, &dMpbound, &dLists,
                        &dListCount, &dSamples, &dChannels, &dRgba, &dCounters, &dBucketRefs,
                        &dHitData, &dHitNext, &dHitCtl, &dHitShards, &dHitHeads, &dDeepList, &dFrontDepth, &dLongWork, &dFormat, &dDrawsReq, &dItemsStatic, &dItemsGrid, &dItems,
-                       &dItemCount, &dQueue, &dRows, &dSegBucket, &dSegCounts, &dMprecMB, &dCullTrees, &dCullPyr,
+                       &dItemCount, &dQueue, &dRows, &dSegBucket, &dSegCounts, &dSegMasks, &dMprecMB, &dCullTrees, &dCullPyr,
                        &dCullBounds, &dCullRanges, &dCullStart, &dCullPairMax, &dProbeOut, &dProbeItems,
                        &dProbeTasks, &dProbeCut, &dProbeB, &dProbeC};
         for (DBuf* b : all) f(*b);
@@ -574,6 +575,15 @@ static std::vector<uint2> grid_items(const std::vector<uint2>& tasks, int blocks
     return out;
 }
 
+// The columns and rows of a bucket's tasks, which are in row-major order: the
+// first row's length is the width.
+static std::pair<int, int> task_grid(const rh::Shape& s, size_t bucket) {
+    const int first = s.taskStart[bucket], n = s.taskStart[bucket + 1] - first;
+    int w = 0;
+    while (w < n && s.tasks[first + w].y0 == s.tasks[first].y0) ++w;
+    return {w, w > 0 ? n / w : 0};
+}
+
 // The strip filter's lists, from the box tests of the frame shape's sample
 // positions: per filter column an entry for each sample that lies in the box
 // of some pixel there, in sample order, with weight 0 in the rows where its
@@ -734,10 +744,7 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
         d.bx = s.bx0 + (int)(k % s.nbr); d.by = s.by0 + (int)(k / s.nbr);
         d.task0 = s.taskStart[k];
         d.ntask = s.taskStart[k + 1] - s.taskStart[k];
-        // tasks are in row-major order: the first row's length is the width
-        d.ntx = 0;
-        while (d.ntx < d.ntask && s.tasks[d.task0 + d.ntx].y0 == s.tasks[d.task0].y0) ++d.ntx;
-        d.nty = d.ntx > 0 ? d.ntask / d.ntx : 0;
+        std::tie(d.ntx, d.nty) = task_grid(s, k);
         c->binTaskSide = std::max(c->binTaskSide, std::max(d.ntx, d.nty));
         bk.push_back(d);
     }
@@ -964,6 +971,7 @@ static rh_status upload_schedule(rh_ctx* c) {
     HIP_TRY(upload(c->dCandGrid, S.candGrid, c->st));
     HIP_TRY(upload(c->dSegBucket, S.segBucket, c->st));
     HIP_TRY(c->dSegCounts.ensure(S.candGrid.size() * 17 * sizeof(uint32_t)));
+    HIP_TRY(c->dSegMasks.ensure(S.candGrid.size() * RH_SEG_MASKS(c->binTaskSide) * sizeof(unsigned long long)));
     HIP_TRY(upload(c->dCapStart, cap, c->st));
     if (!S.motion) HIP_TRY(c->dMprec.ensure(S.micropolygons * RH_MPREC_FLOATS * sizeof(float)));
     HIP_TRY(c->dMpbound.ensure(S.micropolygons * sizeof(float4)));
@@ -1064,7 +1072,8 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
     ENQ(rh_launch_bin(c->st, f, c->dBuckets.as<BucketDev>(), nb, c->dTasks.as<TaskDev>(), c->dGrids.as<GridDev>(),
                       c->dCandStart.as<uint32_t>(), c->dCandGrid.as<uint32_t>(), c->dSegBucket.as<uint32_t>(),
                       S.candGrid.size(), c->dCapStart.as<unsigned long long>(), c->dMpbound.as<float4>(),
-                      c->dSegCounts.as<uint32_t>(), c->dLists.as<uint32_t>(), c->dListCount.as<uint32_t>(),
+                      c->dSegCounts.as<uint32_t>(), c->dSegMasks.as<unsigned long long>(), c->dLists.as<uint32_t>(),
+                      c->dListCount.as<uint32_t>(),
                       c->dBucketRefs.as<uint32_t>(), k.counters, c->binTaskSide,
                       ((c->frame.bucketX & (c->frame.bucketX - 1)) == 0 && (c->frame.bucketY & (c->frame.bucketY - 1)) == 0) ? 1 : 0,
                       S.motion ? c->dMprecMB.as<float4>() : nullptr));
@@ -1199,7 +1208,8 @@ static hipError_t enqueue_depth_pass(rh_ctx* c, bool sample) {
     if ((e = rh_launch_bin(c->st, f, c->dBuckets.as<BucketDev>(), (int)s.buckets.size(), c->dTasks.as<TaskDev>(),
                            c->dGrids.as<GridDev>(), c->dCandStart.as<uint32_t>(), c->dCandGrid.as<uint32_t>(),
                            c->dSegBucket.as<uint32_t>(), S.candGrid.size(), c->dCapStart.as<unsigned long long>(),
-                           c->dMpbound.as<float4>(), c->dSegCounts.as<uint32_t>(), c->dLists.as<uint32_t>(),
+                           c->dMpbound.as<float4>(), c->dSegCounts.as<uint32_t>(), c->dSegMasks.as<unsigned long long>(),
+                           c->dLists.as<uint32_t>(),
                            c->dListCount.as<uint32_t>(), c->dBucketRefs.as<uint32_t>(),
                            c->dCounters.as<unsigned long long>(), c->binTaskSide,
                            ((c->frame.bucketX & (c->frame.bucketX - 1)) == 0 &&
@@ -1785,7 +1795,7 @@ uint64_t rh_internal_device_bytes(const rh_ctx* c) {
     const DBuf* all[] = {&c->dFrame, &c->dBuckets, &c->dTasks, &c->dPos2d, &c->dPos1d, &c->dPix, &c->dDither,
                          &c->dFilter, &c->dBoxMask, &c->dFiltList,
                          &c->dGrids, &c->dParams, &c->dPrims, &c->dCandStart,
-                         &c->dCandGrid, &c->dCapStart, &c->dSegBucket, &c->dSegCounts, &c->dMprec, &c->dMpbound, &c->dLists,
+                         &c->dCandGrid, &c->dCapStart, &c->dSegBucket, &c->dSegCounts, &c->dSegMasks, &c->dMprec, &c->dMpbound, &c->dLists,
                          &c->dListCount, &c->dSamples, &c->dChannels, &c->dRgba, &c->dCounters,
                          &c->dBucketRefs, &c->dHitData, &c->dHitNext, &c->dHitCtl, &c->dHitShards, &c->dHitHeads,
                          &c->dDeepList, &c->dFrontDepth,
@@ -1811,8 +1821,13 @@ static uint64_t frame_bytes(const rh::Shape& s) {
 
 // Device bytes of one frame of a scheduled scene.
 static uint64_t footprint_bytes(const rh::Shape& s, const rh::Schedule& S, const rh_prim* prims, int32_t n) {
+    int side = 1;
+    for (size_t k = 0; k < s.buckets.size(); ++k) {
+        const std::pair<int, int> n = task_grid(s, k);
+        side = std::max(side, std::max(n.first, n.second));
+    }
     uint64_t bytes = frame_bytes(s) + S.grids.size() * sizeof(GridDev) + S.paramFloats * 4 +
-                     (uint64_t)n * sizeof(PrimDev) + S.candGrid.size() * (4 + 4 + 17 * 4) +
+                     (uint64_t)n * sizeof(PrimDev) + S.candGrid.size() * (4 + 4 + 17 * 4 + RH_SEG_MASKS(side) * 8) +
                      S.micropolygons * ((S.motion ? RH_MPREC_MB_FLOATS : RH_MPREC_FLOATS) * 4 + 16) +
                      S.capStart.back() * 4;
     bool transparent = false;
