@@ -47,11 +47,13 @@
 // Motion-frame micropolygon record, in floats:
 //  [0..11]  key 0: x, y, z of the four vertices in grid order
 //  [12..23] key 1 (a static micropolygon repeats key 0)
-//  [24]     flags as above, plus RH_MB_MOVING  [25] grid index (int bits)
+//  [24]     flags as above, plus RH_MB_MOVING and its number of sub-bounds
+//           (from bit RH_MB_DIVISIONS)  [25] grid index (int bits)
 //  [26..27] key times  [28..31] static bound min x, max x, min y, max y
 #define RH_MPREC_MB_FLOATS 32
 #define RH_MPREC_MB_GRID 25
 #define RH_MB_MOVING (1u << 11)
+#define RH_MB_DIVISIONS 16
 // Device counters: 0..4 the hider's SPL counters (sample tests, bound hits,
 // stored hits, point-in-polygon hits, second Newton steps), 5 tasks whose
 // list overflowed, 6 micropolygon-bucket references, 7 and 8 unused.

@@ -398,19 +398,21 @@ __global__ void __launch_bounds__(256) rh_dice_bust(const FrameDev* __restrict__
         mb[5] = make_float4(K1[2].z, K1[3].x, K1[3].y, K1[3].z);
         const float t0 = motion ? prm1[key_param_floats(type, cu, cv)] : 0.0f;
         const float t1 = motion ? prm1[key_param_floats(type, cu, cv) + 1] : 0.0f;
-        mb[6] = make_float4(__uint_as_float(flags | (motion ? RH_MB_MOVING : 0u)), __int_as_float((int)blockIdx.x), t0, t1);
+        int divisions = 0;
         if (motion) {
             float kb[2][6];
             mb_key_bound(P, kb[0]);
             mb_key_bound(K1, kb[1]);
             mpbound[G.mpBase + m] = make_float4(fmin_ref(kb[0][0], kb[1][0]), fmax_ref(kb[0][3], kb[1][3]),
                                                 fmin_ref(kb[0][1], kb[1][1]), fmax_ref(kb[0][4], kb[1][4]));
-            const int divisions = mb_divisions(kb[0], P[0], K1[0], max(4, fr->nx * fr->ny));
+            divisions = mb_divisions(kb[0], P[0], K1[0], max(4, fr->nx * fr->ny));
             mb[7] = mb_hull(kb, divisions, t0, t1, fr->shutterOpen, fr->shutterClose);
         } else {
             mpbound[G.mpBase + m] = make_float4(bminx, bmaxx, bminy, bmaxy);
             mb[7] = make_float4(bminx, bmaxx, bminy, bmaxy);
         }
+        mb[6] = make_float4(__uint_as_float(flags | (motion ? RH_MB_MOVING | (uint32_t)divisions << RH_MB_DIVISIONS : 0u)),
+                            __int_as_float((int)blockIdx.x), t0, t1);
     }
 }
 
@@ -1446,13 +1448,74 @@ __device__ __forceinline__ MBHit quad_hit(const f3d p0, const f3d p1, const f3d 
 //     entries that visit the lane's sample; the lanes then take their own
 //     entries lowest bit first, so each sample sees its visits in order and a
 //     wave runs as many visit steps as its busiest lane has visits.
-#ifndef RH_MB_RECS
-#define RH_MB_RECS 128     // records staged per chunk (a multiple of 64)
-#endif
-#ifndef RH_MB_PAIRS
-#define RH_MB_PAIRS 1792   // (record, sub-bound) pairs per chunk at most
-#endif
-#define RH_MB_RING 128     // visit results held per wave
+// Bound by VALU (about half its time) and by the waits for the slowest wave
+// of a chunk.  256x256, 8x8 samples, 600 moving patches: 10420 us with every
+// sub-bound a pair and the visits found by searches of rank tables, 7980 with
+// the sub-bounds a task can meet and a list of visits, 6440 with longer chunks.
+// Records staged per chunk (a multiple of 64, at most 512) and (record,
+// sub-bound) pairs per chunk at most.  The waves meet after each chunk, whose
+// cost differs from block to block, so a chunk is as long as LDS allows: 128
+// records and 1792 pairs 7980 us, 256 and 1216 6540, 320 and 912 6440, 384 and
+// 608 6460 (two workgroups a CU of 8 waves, 192 and 192: 6710).
+#define RH_MB_RECS 320
+#define RH_MB_PAIRS 912
+#define RH_MB_RING 128     // visits and results held per wave
+#define RH_MB_STATIC 0xfe00u
+#define RH_MB_DIVS 64      // sub-bounds of a micropolygon at most
+#define RH_MB_IN 0x10000u
+#define RH_MB_LINEAR 0x20000u
+#define RH_MB_OPAQUE 0x40000u
+
+// The sub-bounds of a moving micropolygon that can meet pixels [x0, x1) x
+// [y0, y1), as divs holds them: d sub-bounds in all, of which those from the
+// second byte on, as many as the top byte says, the first of all among them.
+// A bound's side goes along a straight line with the step t of the shutter's
+// d: sub-bound b lies between t = b and b + 1, and can meet the pixels while
+// its upper sides are past x0 and y0 and its lower ones short of x1 and y1,
+// each a half-line of t.  What the kept ones visit is decided exactly
+// afterwards, so this only has to err outwards: by a hundredth of a step
+// and the rounding of the summed times (up to 64 additions) and by the rounding
+// of the sides in pixels.  The first sub-bound begins at key 0, wherever the shutter
+// opens, so it is kept unless they are the same time.  Values that leave the
+// range of the conversions, and times too coarse to tell steps apart, take
+// all.
+__device__ __forceinline__ uint32_t mb_sub_range(const float kb[2][6], int d, float T0, float T1, float open,
+                                                 float close, float x0, float x1, float y0, float y1) {
+    const uint32_t all = (uint32_t)d | (uint32_t)d << 24;
+    const float dt = (close - open) / d, inv = 1.0f / (T1 - T0);
+    const float m0 = (open - T0) * inv, dm = dt * inv;
+    float P = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 6; ++c)
+        if (c != 2 && c != 5) P = fmaxf(P, fabsf(kb[0][c])), P = fmaxf(P, fabsf(kb[1][c]));
+    const float reach = P * (1.0f + fabsf(m0) + d * dm);
+    bool sound = d > 1 && T1 > T0 && dt > 0.0f && reach < 1e9f;
+    const float eb = 0.01f + 3e-5f * (fabsf(open) + fabsf(close) + fabsf(T0) + fabsf(T1)) / dt;
+    const float ep = 1e-3f + 1e-5f * reach;
+    float lo = 0.0f, hi = (float)(d - 1);
+    // side c of the bound over t: A + t S; `up`: it has to be past e, else short of it
+    auto side = [&](int c, bool up, float e) {
+        const float s = kb[1][c] - kb[0][c];
+        const float S = s * dm, rest = e - (kb[0][c] + m0 * s);
+        sound = sound && rest == rest && S == S;
+        if (fabsf(S) * d < 1e-6f * fabsf(rest) || S == 0.0f) {
+            if (up ? rest > 0.0f : rest < 0.0f) hi = -1.0f;   // never, or (rest 0) always
+            return;
+        }
+        const float t = rest / S;
+        if (up == (S > 0.0f)) lo = fmaxf(lo, t - 1.0f - eb);
+        else hi = fminf(hi, t + eb);
+    };
+    side(3, true, x0 - ep);
+    side(0, false, x1 + ep);
+    side(4, true, y0 - ep);
+    side(1, false, y1 + ep);
+    if (!sound || !(eb < 64.0f)) return all;
+    const int b0 = (int)ceilf(fminf(lo, 64.0f)), b1 = hi < 0.0f ? -1 : (int)floorf(hi);
+    const int n = b1 >= b0 ? b1 - b0 + 1 : 0;
+    const uint32_t one = (open != T0 && (b0 > 0 || n == 0)) ? 1u : 0u;
+    return (uint32_t)d | (uint32_t)(b0 & 0xff) << 8 | one << 16 | ((uint32_t)n + one) << 24;
+}
 
 // Transpose of a 64 x 64 bit matrix held one row per lane (bit c of lane r's
 // word is element (r, c)): lane c returns column c.  Six rounds exchange
@@ -1472,25 +1535,8 @@ __device__ __forceinline__ unsigned long long transpose64(unsigned long long row
     return row;
 }
 
-// The position of the k-th (from 0) set bit of m, which has more than k.
-__device__ __forceinline__ int select_bit(unsigned long long m, int k) {
-    int pos = 0;
-    int c = __popc((uint32_t)m);
-    if (k >= c) { k -= c; m >>= 32; pos = 32; }
-    uint32_t w = (uint32_t)m;
-    c = __popc(w & 0xffffu);
-    if (k >= c) { k -= c; w >>= 16; pos += 16; }
-    c = __popc(w & 0xffu);
-    if (k >= c) { k -= c; w >>= 8; pos += 8; }
-    c = __popc(w & 0xfu);
-    if (k >= c) { k -= c; w >>= 4; pos += 4; }
-    c = __popc(w & 0x3u);
-    if (k >= c) { k -= c; w >>= 2; pos += 2; }
-    return pos + ((k >= (int)(w & 1u)) ? 1 : 0);
-}
-
 template <int NW, int STORE>
-__global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restrict__ fr,
+__global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __restrict__ fr,
                                                         const BucketDev* __restrict__ buckets,
                                                         const TaskDev* __restrict__ tasks, int ntasks,
                                                         const unsigned long long* __restrict__ capStart,
@@ -1510,11 +1556,13 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                                                         const uint32_t* __restrict__ taskList, int depthOnly) {
     __shared__ float4 recs[RH_MB_RECS * 8];
     __shared__ float kbs[RH_MB_RECS][12];          // key bounds, kb[k][c] at [k * 6 + c]
-    __shared__ float dts[RH_MB_RECS];
-    __shared__ int divs[RH_MB_RECS];
+    // sub-bounds | first taken << 8 | the first of all taken too << 16 | number taken << 24
+    __shared__ uint32_t divs[RH_MB_RECS];
+    // per number of sub-bounds d their time step, and their end times from d (d - 1) / 2 on
+    __shared__ float dts[RH_MB_DIVS + 1], times[RH_MB_DIVS * (RH_MB_DIVS + 1) / 2];
     __shared__ int offs[RH_MB_RECS + 1];
     __shared__ uint32_t ids[RH_MB_RECS];
-    // entries: (record | sub-bound << 8 (0xff: static) | index window << 16,
+    // entries: (record | sub-bound << 9 (RH_MB_STATIC: static) | index window << 16,
     // sub-sample x range, y range (lo | hi << 16), min z); the bound
     // (min x, max x, min y, max y); the times (time0, time1)
     __shared__ uint4 E0[RH_MB_PAIRS];
@@ -1523,11 +1571,12 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
     __shared__ uint16_t buf[NW][128];
     __shared__ float4 smp[NW][64];                 // the block's samples: x, y, time, LOD test
     __shared__ unsigned long long winLanes[65];
-    // per wave: the visit results ring, and per rank its first position and lanes
+    // per wave, rings over its visits: (lane, place in buf), and their results:
+    // entry | RH_MB_* << 16, then the depth (the entry's least one for a visit
+    // outside its quad) and the place in the quad
+    __shared__ uint16_t ringVis[NW][RH_MB_RING];
     __shared__ uint32_t ringCode[NW][RH_MB_RING];
     __shared__ float ringD[NW][RH_MB_RING], ringU[NW][RH_MB_RING], ringV[NW][RH_MB_RING];
-    __shared__ int rankStart[NW][65];
-    __shared__ unsigned long long rankLanes[NW][64];
     __shared__ uint32_t wtot[NW];
     __shared__ int nfitShared;
     __shared__ uint32_t wsum[NW][5];
@@ -1558,9 +1607,6 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
     const float timePerSample = fastShutter ? 0.0f : ns / (closetime - opentime);
     const int timeRanges = max(4, nx * ny);
     const float clipNear = fr->clipNear, clipFar = fr->clipFar;
-    // the task in sub-sample units of the bucket's sample region
-    const int tgx0 = (T.x0 - B.sx0) * nx, tgx1 = (T.x1 - B.sx0) * nx;
-    const int tgy0 = (T.y0 - B.sy0) * ny, tgy1 = (T.y1 - B.sy0) * ny;
     // a block's lanes of sub-sample index below k, and the rows of its lanes
     unsigned long long rowRep = 0ull;
     for (int r = 0; r < BH; ++r) rowRep |= 1ull << (r * BW);
@@ -1569,8 +1615,23 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
             const unsigned long long m = __ballot(laneOk && si < k);
             if (lane == 0) winLanes[k] = m;
         }
+    if (wave == 1) {
+        const int d = lane + 1;
+        const float dt = (closetime - opentime) / d;
+        dts[d] = dt;
+        float time = opentime + dt;
+        for (int b = 0; b < d; ++b) {
+            times[d * lane / 2 + b] = time;
+            time += dt;
+        }
+    }
 
     for (int p0 = 0; p0 < nbx * nby; p0 += NW) {
+        // the rows of this pass's blocks, and those in sub-sample units of the
+        // bucket's sample region
+        const int y0 = T.y0 + p0 / nbx * bh, y1 = min(T.y0 + (min(p0 + NW, nbx * nby) - 1) / nbx * bh + bh, T.y1);
+        const int tgx0 = (T.x0 - B.sx0) * nx, tgx1 = (T.x1 - B.sx0) * nx;
+        const int tgy0 = (y0 - B.sy0) * ny, tgy1 = (y1 - B.sy0) * ny;
         const int blk = p0 + wave;
         const bool has = blk < nbx * nby;       // uniform per wave
         const int bx = T.x0 + (blk % nbx) * bw, by = T.y0 + (blk / nbx) * bh;
@@ -1606,12 +1667,12 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                 if ((q & 7) == 0) ids[q / 8] = id;
             }
             __syncthreads();
-            // per record: key bounds, sub-bound count and time step
+            // per record: key bounds, and the sub-bounds that can meet the task
             if (tid < cnt) {
                 const float4* R = &recs[tid * 8];
-                const uint32_t flags = __float_as_uint(R[6].x);
-                int d = 1;
-                float dtv = 0.0f;
+                const float4 r6 = R[6];
+                const uint32_t flags = __float_as_uint(r6.x);
+                uint32_t dv = 1u | 1u << 24;
                 if (flags & RH_MB_MOVING) {
                     const float4 r0 = R[0], r1 = R[1], r2 = R[2], r3 = R[3], r4 = R[4], r5 = R[5];
                     const f3d K0[4] = {mk3(r0.x, r0.y, r0.z), mk3(r0.w, r1.x, r1.y), mk3(r1.z, r1.w, r2.x),
@@ -1626,11 +1687,10 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                         kbs[tid][c] = kb[0][c];
                         kbs[tid][6 + c] = kb[1][c];
                     }
-                    d = mb_divisions(kb[0], K0[0], K1[0], timeRanges);
-                    dtv = (closetime - opentime) / d;
+                    dv = mb_sub_range(kb, (int)((flags >> RH_MB_DIVISIONS) & 0xffu), r6.z, r6.w, opentime, closetime,
+                                      (float)T.x0, (float)T.x1, (float)y0, (float)y1);
                 }
-                divs[tid] = d;
-                dts[tid] = dtv;
+                divs[tid] = dv;
             }
             __syncthreads();
             // pair offsets, and the records whose pairs fit in one pass
@@ -1639,7 +1699,7 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                 int dk[PER], incl = 0;
 #pragma unroll
                 for (int j = 0; j < PER; ++j) {
-                    dk[j] = PER * lane + j < cnt ? divs[PER * lane + j] : 0;
+                    dk[j] = PER * lane + j < cnt ? (int)(divs[PER * lane + j] >> 24) : 0;
                     incl += dk[j];
                 }
                 for (int off = 1; off < 64; off <<= 1) {
@@ -1678,7 +1738,7 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                         if (offs[mid] <= p) lo = mid;
                         else hi = mid - 1;
                     }
-                    const int r = lo, b = p - offs[r];
+                    const int r = lo;
                     const float4* R = &recs[r * 8];
                     const float4 r6 = R[6];
                     const uint32_t flags = __float_as_uint(r6.x);
@@ -1701,7 +1761,7 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                             const int gx0 = max((sX - B.sx0) * nx + im, tgx0), gx1 = min((eX - 1 - B.sx0) * nx + em, tgx1);
                             const int gy0 = max((sY - B.sy0) * ny + in, tgy0), gy1 = min((eY - 1 - B.sy0) * ny + en, tgy1);
                             keep = gx0 < gx1 && gy0 < gy1;
-                            ea = (uint32_t)r | (0xffu << 8) | ((uint32_t)ns << 24);
+                            ea = (uint32_t)r | RH_MB_STATIC | ((uint32_t)ns << 24);
                             ex = (uint32_t)gx0 | ((uint32_t)gx1 << 16);
                             ey = (uint32_t)gy0 | ((uint32_t)gy1 << 16);
                             // CalculateBound's min z: min(min(min(A,B),C),D), A..D = P0,P1,P3,P2
@@ -1713,14 +1773,11 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                         const float* kb0 = &kbs[r][0];
                         const float* kb1 = &kbs[r][6];
                         const float T0 = r6.z, T1 = r6.w;
-                        const int d = divs[r];
-                        const float dt = dts[r];
-                        float time = opentime + dt, tp = 0.0f;
-                        for (int i = 0; i < b; ++i) {
-                            tp = time;
-                            time += dt;
-                        }
-                        const float tc = time;
+                        const uint32_t dv = divs[r];
+                        const int d = (int)(dv & 0xffu), one = (int)((dv >> 16) & 1u), k = p - offs[r];
+                        const int b = k < one ? 0 : (int)((dv >> 8) & 0xffu) + k - one;
+                        const float dt = dts[d];
+                        const float tc = times[d * (d - 1) / 2 + b], tp = b == 0 ? 0.0f : times[d * (d - 1) / 2 + b - 1];
                         const float mixc = (tc - T0) / (T1 - T0);
                         const float mixp = (tp - T0) / (T1 - T0);
                         float sb[6];
@@ -1754,7 +1811,7 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                                 const int gx0 = max((sX - B.sx0) * nx, tgx0), gx1 = min((eX - B.sx0) * nx, tgx1);
                                 const int gy0 = max((sY - B.sy0) * ny, tgy0), gy1 = min((eY - B.sy0) * ny, tgy1);
                                 keep = gx0 < gx1 && gy0 < gy1;
-                                ea = (uint32_t)r | ((uint32_t)b << 8) | ((uint32_t)indexT0 << 16) |
+                                ea = (uint32_t)r | ((uint32_t)b << 9) | ((uint32_t)indexT0 << 16) |
                                      ((uint32_t)idxEnd << 24);
                                 ex = (uint32_t)gx0 | ((uint32_t)gx1 << 16);
                                 ey = (uint32_t)gy0 | ((uint32_t)gy1 << 16);
@@ -1830,57 +1887,49 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                         }
                     }
                     const unsigned long long vm = transpose64(pass, lane);
-                    // Two passes over the visits of these entries.  A: every
-                    // visit's tests but the occlusion test, 64 visits a step
-                    // whichever samples they belong to, taken in rank-major
-                    // order (each lane's first visit, then each lane's
-                    // second, ...), results into a ring in LDS.  B: once a
-                    // rank is complete, each lane applies its visit of that
-                    // rank in order: occlusion test, counters, StoreSample.
+                    // Three steps over the visits of these entries, taken in
+                    // rank-major order (each lane's first visit, then each
+                    // lane's second, ...).  List: whole ranks, into a ring,
+                    // until 64 visits wait.  A: every visit's tests but the
+                    // occlusion test, 64 visits a step whichever samples they
+                    // belong to, results into a ring.  B: once a rank is
+                    // complete, each lane applies its visit of that rank in
+                    // order: occlusion test, counters, StoreSample.
                     const int cnt = __popcll(vm);
                     int maxc = cnt;
                     for (int off = 32; off > 0; off >>= 1) maxc = max(maxc, __shfl_xor(maxc, off));
-                    int total = 0;
-                    for (int r = 0; r < maxc; ++r) {
-                        const unsigned long long lm = __ballot(cnt > r);
-                        if (lane == 0) {
-                            rankStart[wave][r] = total;
-                            rankLanes[wave][r] = lm;
+                    unsigned long long rem = vm;
+                    int listed = 0, done = 0, rL = 0, rB = 0, startB = 0;
+                    while (rB < maxc) {
+                        while (rL < maxc && listed - done < 64) {
+                            const bool act = cnt > rL;
+                            const unsigned long long lm = __ballot(act);
+                            if (act) {
+                                const int q = __builtin_ctzll(rem);
+                                rem &= rem - 1ull;
+                                ringVis[wave][(listed + __popcll(lm & lanesBelow)) & (RH_MB_RING - 1)] =
+                                    (uint16_t)(lane | q << 6);
+                            }
+                            listed += __popcll(lm);
+                            ++rL;
                         }
-                        total += __popcll(lm);
-                    }
-                    if (lane == 0) rankStart[wave][maxc] = total;
-                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    const uint32_t vmLo = (uint32_t)vm, vmHi = (uint32_t)(vm >> 32);
-                    int done = 0, rB = 0;
-                    while (done < total) {
+                        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
                         // A: visits [done, done + 64)
                         {
                             const int p = done + lane;
-                            const bool pv = p < total;
-                            int rk = 0;
-                            {
-                                int lo = 0, hi = maxc - 1;
-                                while (lo < hi) {
-                                    const int mid = (lo + hi + 1) >> 1;
-                                    if (rankStart[wave][mid] <= p) lo = mid;
-                                    else hi = mid - 1;
-                                }
-                                rk = lo;
-                            }
-                            const int own = pv ? select_bit(rankLanes[wave][rk], p - rankStart[wave][rk]) : lane;
-                            const unsigned long long vmo =
-                                ((unsigned long long)(uint32_t)__shfl((int)vmHi, own) << 32) | (uint32_t)__shfl((int)vmLo, own);
-                            const float osx = __shfl(sx, own), osy = __shfl(sy, own), ost = __shfl(stime, own);
+                            const bool pv = p < listed;
                             uint32_t fl = 0;
                             float D = 0.f, u = 0.f, v = 0.f;
-                            int q = 0;
                             if (pv) {
-                                q = select_bit(vmo, rk);
-                                const int e = buf[wave][q];
-                                const uint32_t a = E0[e].x;
-                                const int r = (int)(a & 0xffu), b = (int)((a >> 8) & 0xffu);
+                                const uint32_t vis = ringVis[wave][p & (RH_MB_RING - 1)];
+                                const float4 sp = smp[wave][vis & 63u];
+                                const float osx = sp.x, osy = sp.y, ost = sp.z;
+                                const int e = buf[wave][vis >> 6];
+                                const uint4 h0 = E0[e];
+                                const uint32_t a = h0.x;
+                                D = __uint_as_float(h0.w);
+                                const int r = (int)(a & 0x1ffu);
                                 const float4* R = &recs[r * 8];
                                 const float4 r6 = R[6];
                                 const uint32_t flags = __float_as_uint(r6.x);
@@ -1891,7 +1940,7 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                                                    mk3(r1.z, r1.w, r2.x), mk3(r2.y, r2.z, r2.w)};
                                 bool tight = true;
                                 f3d pts[4] = {K0[0], K0[1], K0[2], K0[3]};
-                                if (b != 0xff) {
+                                if ((a & RH_MB_STATIC) != RH_MB_STATIC) {
                                     // CqMicroPolygonMotion::Sample: the key span of
                                     // the time, the tight bound and the vertices there
                                     const float* kb0 = &kbs[r][0];
@@ -1924,66 +1973,78 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                                     const f3d K1[4] = {mk3(r3.x, r3.y, r3.z), mk3(r3.w, r4.x, r4.y),
                                                        mk3(r4.z, r4.w, r5.x), mk3(r5.y, r5.z, r5.w)};
                                     // a key's vertices when the time is exact, else
-                                    // (1 - F) K0 + F K1; selected per component
+                                    // (1 - F) K0 + F K1
                                     const float F1 = 1.0f - Fraction;
-                                    const bool k1 = iIndex != 0;
 #pragma unroll
-                                    for (int k = 0; k < 4; ++k) {
-                                        const f3d mixed = mk3((F1 * K0[k].x) + (Fraction * K1[k].x),
-                                                              (F1 * K0[k].y) + (Fraction * K1[k].y),
-                                                              (F1 * K0[k].z) + (Fraction * K1[k].z));
-                                        pts[k].x = Exact ? (k1 ? K1[k].x : K0[k].x) : mixed.x;
-                                        pts[k].y = Exact ? (k1 ? K1[k].y : K0[k].y) : mixed.y;
-                                        pts[k].z = Exact ? (k1 ? K1[k].z : K0[k].z) : mixed.z;
+                                    for (int k = 0; k < 4; ++k)
+                                        pts[k] = mk3((F1 * K0[k].x) + (Fraction * K1[k].x),
+                                                     (F1 * K0[k].y) + (Fraction * K1[k].y),
+                                                     (F1 * K0[k].z) + (Fraction * K1[k].z));
+                                    if (Exact) {
+                                        const bool k1 = iIndex != 0;
+#pragma unroll
+                                        for (int k = 0; k < 4; ++k)
+                                            pts[k] = mk3(k1 ? K1[k].x : K0[k].x, k1 ? K1[k].y : K0[k].y,
+                                                         k1 ? K1[k].z : K0[k].z);
                                     }
                                 }
                                 if (tight) {
                                     const MBHit h = quad_hit(pts[0], pts[1], pts[2], pts[3], code, degen, osx, osy);
                                     if (h.in) {
-                                        fl = 2u | (h.linear ? 4u : 0u);
+                                        fl = RH_MB_IN | (h.linear ? RH_MB_LINEAR : 0u) |
+                                             ((flags >> 10) & 1u ? RH_MB_OPAQUE : 0u);
                                         D = h.D; u = h.u; v = h.v;
                                     }
                                 }
                                 const int slot = p & (RH_MB_RING - 1);
-                                ringCode[wave][slot] = (uint32_t)q | (fl << 8);
+                                ringCode[wave][slot] = (uint32_t)e | fl;
                                 ringD[wave][slot] = D;
-                                ringU[wave][slot] = u;
-                                ringV[wave][slot] = v;
+                                if (fl) {
+                                    ringU[wave][slot] = u;
+                                    ringV[wave][slot] = v;
+                                }
                             }
                         }
-                        done = min(done + 64, total);
+                        done = min(done + 64, listed);
                         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                         __builtin_amdgcn_wave_barrier();
                         // B: the ranks now complete, in order
-                        while (rB < maxc && rankStart[wave][rB + 1] <= done) {
+                        while (rB < maxc) {
                             const bool act = cnt > rB;
                             const unsigned long long lm = __ballot(act);
-                            bool hit = false, opaque = false;
-                            float D = 0.f, u = 0.f, v = 0.f;
-                            uint32_t hid = 0;
-                            int hgrid = 0;
+                            const int first = startB;
+                            if (first + __popcll(lm) > done) break;
+                            startB += __popcll(lm);
+                            ++rB;
+                            const int slot = (first + __popcll(lm & lanesBelow)) & (RH_MB_RING - 1);
+                            uint32_t rc = 0;
+                            float D = 0.f, mz = 0.f;
                             if (act) {
-                                const int slot = (rankStart[wave][rB] + __popcll(lm & lanesBelow)) & (RH_MB_RING - 1);
-                                const uint32_t rc = ringCode[wave][slot];
-                                const int e = buf[wave][rc & 0xffu];
-                                const uint4 h = E0[e];
-                                const float mz = __uint_as_float(h.w);
-                                const int r = (int)(h.x & 0xffu);
-                                const float4 r6 = recs[r * 8 + 6];
-                                opaque = (__float_as_uint(r6.x) >> 10) & 1u;
+                                rc = ringCode[wave][slot];
+                                D = ringD[wave][slot];
+                                mz = D;
+                            }
+                            const bool in = (rc & RH_MB_IN) != 0u;
+                            uint4 h = make_uint4(0u, 0u, 0u, 0u);
+                            if (in) {
+                                h = E0[rc & 0xffffu];
+                                mz = __uint_as_float(h.w);
+                            }
+                            const bool bound = act && !(cullH && mz > occlZ);
+                            nBound += bound ? 1u : 0u;
+                            if (!__ballot(bound && in)) continue;
+                            const int r = (int)(h.x & 0x1ffu);
+                            const bool opaque = (rc & RH_MB_OPAQUE) != 0u;
+                            bool hit = false;
+                            float u = 0.f, v = 0.f;
+                            uint32_t hid = 0;
+                            if (bound && in) {
+                                ++nIn;
+                                if (!(rc & RH_MB_LINEAR)) ++nIn2;
+                                u = ringU[wave][slot];
+                                v = ringV[wave][slot];
                                 hid = ids[r];
-                                hgrid = __float_as_int(r6.y);
-                                if (!(cullH && mz > occlZ)) {
-                                    ++nBound;
-                                    if (rc & 0x200u) {
-                                        ++nIn;
-                                        if (!(rc & 0x400u)) ++nIn2;
-                                        D = ringD[wave][slot];
-                                        u = ringU[wave][slot];
-                                        v = ringV[wave][slot];
-                                        hit = !cullH || !(occlZ <= D);
-                                    }
-                                }
+                                hit = !cullH || !(occlZ <= D);
                             }
                             // StoreSample (bucketprocessor.cpp:1471-1569); the
                             // midpoint case keeps the nearest opaque hit and
@@ -2009,12 +2070,11 @@ __global__ void __launch_bounds__(NW * 64) rh_sample_mb(const FrameDev* __restri
                                 const uint32_t slot = hit_entry(arena, am, lane);
                                 if (app && slot < RH_HIT_NOROOM) {
                                     hitData[slot] = make_float4(u, v, D, __uint_as_float(hid));
-                                    hitNext[slot] = make_uint2(head, (uint32_t)grids[hgrid].prim);
+                                    hitNext[slot] = make_uint2(head, (uint32_t)grids[__float_as_int(recs[r * 8 + 6].y)].prim);
                                     head = slot;
                                     ++nh;
                                 }
                             }
-                            ++rB;
                         }
                     }
                     // keep what the buffer holds past the first 64

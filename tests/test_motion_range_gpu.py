@@ -1,0 +1,43 @@
+"""The motion sampler's choice of the sub-bounds that can meet a task: keys at,
+inside and outside the shutter, shutters far from time zero, surfaces that move
+along one axis, both, hardly or far past the frame, and static ones among
+them; one to sixty-four samples; every output and counter the oracle's."""
+import numpy as np
+import pytest
+
+from aqsis_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shutter,keys", [((0.0, 1.0), (0.0, 1.0)), ((0.0, 1.0), (0.25, 0.7)), ((0.2, 0.5), (0.0, 1.0)),
+                                          ((1000.0, 1000.5), (1000.0, 1000.5)), ((0.0, 1.0), (0.5, 2.0))])
+@pytest.mark.parametrize("k", [(1, 1), (3, 2), (8, 8)])
+def test_sub_bounds(oracle, k, shutter, keys):
+    from aqsis_amd.hider import Hider
+    print(f"motion {k} shutter {shutter} keys {keys}", flush=True)
+    opts, prims = scenes.motion_scene(seed=3, n=60, res=(61, 47), size_px=14.0, samples=k, shift_sigma=0.2,
+                                      shutter=shutter, key_times=keys)
+    for i, p in enumerate(prims):
+        for j in range(16):
+            a, b = list(p.P[j]), list(p.P1[j])
+            dx, dy = b[0] - a[0], b[1] - a[1]
+            scale = [(1.0, 1.0), (1.0, 0.0), (0.0, 1.0), (1e-5, 1e-5), (40.0, 40.0)][i % 5]
+            p.P1[j][:] = [float(np.float32(a[0] + dx * scale[0])), float(np.float32(a[1] + dy * scale[1])), b[2]]
+        if i % 7 == 0:
+            p.nkeys = 1
+        if i % 3 == 0:
+            p.Os[:] = [1.0, 1.0, 1.0]
+    ref = oracle.render(opts, prims, occlusion_cull=True)
+    with Hider(opts) as h:
+        h.post_surfaces(prims)
+        h.render()
+        ids, depth, rgbaz = h.samples()
+        st = h.stats()
+        ch = h.channels()
+    assert np.array_equal(ids, ref["mp_id"])
+    assert np.array_equal(depth.view(np.uint32), ref["depth"].view(np.uint32))
+    assert np.array_equal(rgbaz.view(np.uint32), ref["rgbaz"].view(np.uint32))
+    assert np.array_equal(ch.view(np.uint32), ref["channels"].view(np.uint32))
+    for key in ("spl_count", "spl_bound_hits", "spl_hits"):
+        assert st[key] == ref["stats"][key], key
