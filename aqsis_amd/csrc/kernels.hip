@@ -2670,13 +2670,36 @@ __device__ __forceinline__ void combine_sample(const FrameDev* __restrict__ fr, 
     float col[3] = {0.0f, 0.0f, 0.0f}, opa[3] = {0.0f, 0.0f, 0.0f};
     float opaqueDepth0 = occlZ, opaqueDepth1 = FLT_MAX, maxOpaqueDepth = FLT_MAX;
     const float zt0 = fr->zThreshold[0], zt1 = fr->zThreshold[1], zt2 = fr->zThreshold[2];
+    // Bound by the latency of the list's links and of these loads: a hit's
+    // record and surface are loaded two steps ahead and its surface's colours
+    // one (the occluding hit's place loads a hit of the list instead, which is
+    // not used).  1024x1024 at 8x8 samples 2924 -> 2628 us, 256x256 motion 450
+    // -> 393 us.
+    float4 hNow, hNext;
+    uint32_t sNext;
+    PrimDev pNow;
+    {
+        const uint32_t x0 = x[n - 1] != 0xffffffffu ? x[n - 1] : e.x;
+        hNow = hitData[x0];
+        pNow = prims[hitNext[x0].y];
+        const uint32_t x1 = n > 1 && x[n - 2] != 0xffffffffu ? x[n - 2] : e.x;
+        hNext = hitData[x1];
+        sNext = hitNext[x1].y;
+    }
     for (int q = n - 1; q >= 0; --q) {
         float4 hA = oA, hB = oB;
         bool matte = occMatte;
+        const float4 h = hNow;
+        const PrimDev P = pNow;
+        hNow = hNext;
+        if (q > 0) pNow = prims[sNext];
+        if (q > 1) {
+            const uint32_t x2 = x[q - 2] != 0xffffffffu ? x[q - 2] : e.x;
+            hNext = hitData[x2];
+            sNext = hitNext[x2].y;
+        }
         if (x[q] != 0xffffffffu) {
             // InterpolateOutputs of the hit's surface at its (u, v)
-            const float4 h = hitData[x[q]];
-            const PrimDev& P = prims[hitNext[x[q]].y];
             shade_hit(P, h.x, h.y, h.z, __float_as_uint(h.w), hA, hB);
             matte = FULL && occ.mprec && P.matte == RH_DEV_MATTE;
         }
