@@ -1451,14 +1451,18 @@ __device__ __forceinline__ MBHit quad_hit(const f3d p0, const f3d p1, const f3d 
 // Bound by VALU (about half its time) and by the waits for the slowest wave
 // of a chunk.  256x256, 8x8 samples, 600 moving patches: 10420 us with every
 // sub-bound a pair and the visits found by searches of rank tables, 7980 with
-// the sub-bounds a task can meet and a list of visits, 6440 with longer chunks.
+// the sub-bounds a task can meet and a list of visits, 6440 with longer chunks,
+// 6200 with padded records.
 // Records staged per chunk (a multiple of 64, at most 512) and (record,
 // sub-bound) pairs per chunk at most.  The waves meet after each chunk, whose
 // cost differs from block to block, so a chunk is as long as LDS allows: 128
 // records and 1792 pairs 7980 us, 256 and 1216 6540, 320 and 912 6440, 384 and
-// 608 6460 (two workgroups a CU of 8 waves, 192 and 192: 6710).
+// 608 6460 (two workgroups a CU of 8 waves, 192 and 192: 6710).  With a part
+// of padding a record, which takes the lanes' reads of one part of different
+// records off the same banks, 320 and 784 6200, 256 and 1104 6430.
 #define RH_MB_RECS 320
-#define RH_MB_PAIRS 912
+#define RH_MB_PAIRS 784
+#define RH_MB_STRIDE 9      // float4s of a staged record: one more than it has, off the same banks
 #define RH_MB_RING 128     // visits and results held per wave
 #define RH_MB_STATIC 0xfe00u
 #define RH_MB_DIVS 64      // sub-bounds of a micropolygon at most
@@ -1554,7 +1558,7 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
                                                         uint32_t* __restrict__ rowCounts, int rowBase, int taskBase,
                                                         uint32_t idCut, const uint32_t* __restrict__ itemCut,
                                                         const uint32_t* __restrict__ taskList, int depthOnly) {
-    __shared__ float4 recs[RH_MB_RECS * 8];
+    __shared__ float4 recs[RH_MB_RECS * RH_MB_STRIDE];
     __shared__ float kbs[RH_MB_RECS][12];          // key bounds, kb[k][c] at [k * 6 + c]
     // sub-bounds | first taken << 8 | the first of all taken too << 16 | number taken << 24
     __shared__ uint32_t divs[RH_MB_RECS];
@@ -1663,13 +1667,13 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
             __syncthreads();
             for (int q = tid; q < cnt * 8; q += NW * 64) {
                 const uint32_t id = L[c0 + q / 8];
-                recs[q] = mprecMB[(size_t)id * 8 + (q & 7)];
+                recs[q / 8 * RH_MB_STRIDE + (q & 7)] = mprecMB[(size_t)id * 8 + (q & 7)];
                 if ((q & 7) == 0) ids[q / 8] = id;
             }
             __syncthreads();
             // per record: key bounds, and the sub-bounds that can meet the task
             if (tid < cnt) {
-                const float4* R = &recs[tid * 8];
+                const float4* R = &recs[tid * RH_MB_STRIDE];
                 const float4 r6 = R[6];
                 const uint32_t flags = __float_as_uint(r6.x);
                 uint32_t dv = 1u | 1u << 24;
@@ -1739,7 +1743,7 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
                         else hi = mid - 1;
                     }
                     const int r = lo;
-                    const float4* R = &recs[r * 8];
+                    const float4* R = &recs[r * RH_MB_STRIDE];
                     const float4 r6 = R[6];
                     const uint32_t flags = __float_as_uint(r6.x);
                     if (!(flags & RH_MB_MOVING)) {
@@ -1930,7 +1934,7 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
                                 const uint32_t a = h0.x;
                                 D = __uint_as_float(h0.w);
                                 const int r = (int)(a & 0x1ffu);
-                                const float4* R = &recs[r * 8];
+                                const float4* R = &recs[r * RH_MB_STRIDE];
                                 const float4 r6 = R[6];
                                 const uint32_t flags = __float_as_uint(r6.x);
                                 const uint32_t code = flags & 0xffu;
@@ -2070,7 +2074,7 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
                                 const uint32_t slot = hit_entry(arena, am, lane);
                                 if (app && slot < RH_HIT_NOROOM) {
                                     hitData[slot] = make_float4(u, v, D, __uint_as_float(hid));
-                                    hitNext[slot] = make_uint2(head, (uint32_t)grids[__float_as_int(recs[r * 8 + 6].y)].prim);
+                                    hitNext[slot] = make_uint2(head, (uint32_t)grids[__float_as_int(recs[r * RH_MB_STRIDE + 6].y)].prim);
                                     head = slot;
                                     ++nh;
                                 }
