@@ -141,6 +141,12 @@ struct PrimDev {
     uint32_t matte;                       // RH_MATTE_*
 };
 
+// What a frame clears as it begins.
+struct FrameClear {
+    unsigned long long* counters;
+    uint32_t *hitCtl, *hitShards, *planCtl;
+};
+
 // Arguments of one sampling launch (see rh_sample in kernels.hip).
 struct SampleLaunch {
     const FrameDev* fr;

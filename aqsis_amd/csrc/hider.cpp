@@ -23,7 +23,7 @@
 #include "front.h"
 
 extern "C" hipError_t rh_launch_dice(hipStream_t, const FrameDev*, const GridDev*, int, const PrimDev*,
-                                     const float*, float*, float4*, float4*);
+                                     const float*, float*, float4*, float4*, const FrameClear*);
 extern "C" hipError_t rh_launch_sample_mb(hipStream_t, const SampleLaunch*, int, const float4*);
 extern "C" hipError_t rh_launch_bin(hipStream_t, const FrameDev*, const BucketDev*, int, const TaskDev*,
                                     const GridDev*, const uint32_t*, const uint32_t*, const uint32_t*, size_t,
@@ -34,7 +34,6 @@ extern "C" hipError_t rh_launch_sample_dof(hipStream_t, const SampleLaunch*, int
 extern "C" hipError_t rh_sample_occupancy(int, int*);
 extern "C" hipError_t rh_launch_plan_items(hipStream_t, const FrameDev*, const TaskDev*, int, const uint32_t*,
                                            uint32_t, int, uint2*, uint32_t*, uint32_t*);
-extern "C" hipError_t rh_launch_frame_begin(hipStream_t, unsigned long long*, uint32_t*, uint32_t*, uint32_t*);
 extern "C" hipError_t rh_launch_combine_long(hipStream_t, const FrameDev*, size_t, const uint2*,
                                              const unsigned long long*, uint32_t*, const float4*, const uint2*,
                                              const PrimDev*, const float*, int, int, const GridDev*, int, float4*,
@@ -1064,10 +1063,10 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
     hipError_t e;
 #define ENQ(x) do { if ((e = (x)) != hipSuccess) return e; } while (0)
     if (timed) ENQ(hipEventRecord(c->ev[0], c->st));
-    ENQ(rh_launch_frame_begin(c->st, k.counters, k.hitCtl, c->dHitShards.as<uint32_t>(), c->dItemCount.as<uint32_t>()));
+    const FrameClear clear{k.counters, k.hitCtl, c->dHitShards.as<uint32_t>(), c->dItemCount.as<uint32_t>()};
     ENQ(rh_launch_dice(c->st, f, c->dGrids.as<GridDev>(), (int)S.grids.size(), c->dPrims.as<PrimDev>(),
                        c->dParams.as<float>(), c->dMprec.as<float>(), c->dMpbound.as<float4>(),
-                       S.motion ? c->dMprecMB.as<float4>() : nullptr));
+                       S.motion ? c->dMprecMB.as<float4>() : nullptr, &clear));
     if (timed) ENQ(hipEventRecord(c->ev[1], c->st));
     ENQ(rh_launch_bin(c->st, f, c->dBuckets.as<BucketDev>(), nb, c->dTasks.as<TaskDev>(), c->dGrids.as<GridDev>(),
                       c->dCandStart.as<uint32_t>(), c->dCandGrid.as<uint32_t>(), c->dSegBucket.as<uint32_t>(),
@@ -1198,12 +1197,11 @@ static hipError_t enqueue_depth_pass(rh_ctx* c, bool sample) {
     const rh::Shape& s = c->shape;
     const FrameDev* f = c->dFrame.as<FrameDev>();
     hipError_t e;
-    if ((e = rh_launch_frame_begin(c->st, c->dCounters.as<unsigned long long>(), c->dHitCtl.as<uint32_t>(),
-                                   c->dHitShards.as<uint32_t>(), c->dItemCount.as<uint32_t>())) != hipSuccess)
-        return e;
+    const FrameClear clear{c->dCounters.as<unsigned long long>(), c->dHitCtl.as<uint32_t>(),
+                           c->dHitShards.as<uint32_t>(), c->dItemCount.as<uint32_t>()};
     if ((e = rh_launch_dice(c->st, f, c->dGrids.as<GridDev>(), (int)S.grids.size(), c->dPrims.as<PrimDev>(),
                             c->dParams.as<float>(), c->dMprec.as<float>(), c->dMpbound.as<float4>(),
-                            S.motion ? c->dMprecMB.as<float4>() : nullptr)) != hipSuccess)
+                            S.motion ? c->dMprecMB.as<float4>() : nullptr, &clear)) != hipSuccess)
         return e;
     if ((e = rh_launch_bin(c->st, f, c->dBuckets.as<BucketDev>(), (int)s.buckets.size(), c->dTasks.as<TaskDev>(),
                            c->dGrids.as<GridDev>(), c->dCandStart.as<uint32_t>(), c->dCandGrid.as<uint32_t>(),

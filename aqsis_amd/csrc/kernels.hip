@@ -253,6 +253,18 @@ __device__ __forceinline__ int key_param_floats(int type, int cu, int cv) {
                                   : (type == RH_PRIM_BICUBIC ? 48 : 12);
 }
 
+// Clears the frame's counters (by a kernel, not a memset, for graphs), one
+// workgroup.  The dice kernel's first does it, since dicing uses none of them
+// and every later kernel waits for it: with a launch of its own a 64x64 frame
+// took 153 us, so 148.
+__device__ __forceinline__ void clear_frame(const FrameClear& c) {
+    const int t = threadIdx.x;
+    for (int k = t; k < RH_PLAN_WORDS; k += blockDim.x) c.planCtl[k] = 0u;
+    if (t < RH_HIT_SHARDS) c.hitShards[t * RH_HIT_SHARD_WORDS] = 0u;
+    if (t < RH_NCOUNTERS) c.counters[t] = 0ull;
+    if (t < RH_HITCTL_WORDS) c.hitCtl[t] = 0u;
+}
+
 // MB: a frame with moving micropolygons (the records the motion sampler reads
 // instead of the static ones).  Bound by the latency of a grid's chain (its
 // parameters, the forward differences) and by HBM writes, so by the grids a CU
@@ -267,11 +279,12 @@ __global__ void __launch_bounds__(256) rh_dice_bust(const FrameDev* __restrict__
                                                     const PrimDev* __restrict__ prims,
                                                     const float* __restrict__ params,
                                                     float* __restrict__ mprec, float4* __restrict__ mpbound,
-                                                    float4* __restrict__ mprecMB) {
+                                                    float4* __restrict__ mprecMB, const FrameClear clear) {
     __shared__ float4 V[RH_MAX_GRID_VERTS];
     __shared__ float4 V1[MB ? RH_MAX_GRID_VERTS : 1];
     __shared__ float rows[4 * RH_MAX_GRID_ROWS * 3];
     const int tid = threadIdx.x;
+    if (blockIdx.x == 0) clear_frame(clear);
     const GridDev G = grids[blockIdx.x];
     const int cu = G.cu, cv = G.cv, nu = cu + 1, nv = (cu + 1) * (cv + 1);
     const float* prm = params + G.paramOff;
@@ -2513,7 +2526,7 @@ rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buc
 // bound: a single workgroup walking the tasks took 92 us for 32,640 of them
 // and 187 for 65,536, the two passes take 11 and 14).
 // ctl: RH_PLAN_HIST.. items per class, RH_PLAN_NEXT.. items handed out, both
-// cleared by rh_frame_begin; [0] the number of items.
+// cleared as the frame begins; [0] the number of items.
 struct PlanTask {
     int nblk, per, nitems, bin;
 };
@@ -2585,15 +2598,8 @@ __global__ void __launch_bounds__(256) rh_plan_items(const FrameDev* __restrict_
     }
 }
 
-// Clears the frame's counters (graph-safe: a kernel, not a memset).
-__global__ void rh_frame_begin(unsigned long long* __restrict__ counters, uint32_t* __restrict__ hitCtl,
-                               uint32_t* __restrict__ hitShards, uint32_t* __restrict__ planCtl) {
-    const int t = threadIdx.x;
-    for (int k = t; k < RH_PLAN_WORDS; k += 64) planCtl[k] = 0u;
-    if (t < RH_HIT_SHARDS) hitShards[t * RH_HIT_SHARD_WORDS] = 0u;
-    if (t < RH_NCOUNTERS) counters[t] = 0ull;
-    if (t < RH_HITCTL_WORDS) hitCtl[t] = 0u;
-}
+// The clearing alone, for a frame without grids.
+__global__ void rh_frame_begin(const FrameClear clear) { clear_frame(clear); }
 
 // ---------------------------------------------------------------------------
 // Combine: samples with transparent hits
@@ -3530,14 +3536,17 @@ extern "C" hipError_t rh_launch_cull_pairs(hipStream_t st, const CullTreeDev* tr
 
 extern "C" hipError_t rh_launch_dice(hipStream_t st, const FrameDev* fr, const GridDev* grids, int ngrids,
                                      const PrimDev* prims, const float* params, float* mprec,
-                                     float4* mpbound, float4* mprecMB) {
-    if (ngrids <= 0) return hipSuccess;
+                                     float4* mpbound, float4* mprecMB, const FrameClear* clear) {
+    if (ngrids <= 0) {
+        hipLaunchKernelGGL(rh_frame_begin, dim3(1), dim3(256), 0, st, *clear);
+        return hipGetLastError();
+    }
     if (mprecMB)
         hipLaunchKernelGGL(rh_dice_bust<true>, dim3(ngrids), dim3(256), 0, st, fr, grids, prims, params, mprec,
-                           mpbound, mprecMB);
+                           mpbound, mprecMB, *clear);
     else
         hipLaunchKernelGGL(rh_dice_bust<false>, dim3(ngrids), dim3(256), 0, st, fr, grids, prims, params, mprec,
-                           mpbound, mprecMB);
+                           mpbound, mprecMB, *clear);
     return hipGetLastError();
 }
 
@@ -3753,12 +3762,6 @@ extern "C" hipError_t rh_launch_combine_long(hipStream_t st, const FrameDev* fr,
     else
         hipLaunchKernelGGL(rh_combine_long<false>, grid, dim3(64), 0, st, fr, heads, deepList, hitCtl, hitData, hitNext,
                            prims, occ, samples, frontDepth, workD, workX, workStk);
-    return hipGetLastError();
-}
-
-extern "C" hipError_t rh_launch_frame_begin(hipStream_t st, unsigned long long* counters, uint32_t* hitCtl,
-                                            uint32_t* hitShards, uint32_t* planCtl) {
-    hipLaunchKernelGGL(rh_frame_begin, dim3(1), dim3(64), 0, st, counters, hitCtl, hitShards, planCtl);
     return hipGetLastError();
 }
 
