@@ -310,18 +310,20 @@ bool make_shape(const rh_options& o, Shape& s, std::string& err) {
     // its time on micropolygons elsewhere in the bucket (sampler at 2x2
     // samples: 258 to 184 us at 637x475, 1098 to 921 at 1920x1080; 2x2-pixel
     // blocks gain 0 to 10% in the sampler and lose more in binning).  The
-    // motion sampler runs one workgroup a task and keeps the larger tasks, as
-    // do frames of so many buckets that their task count would matter (the
-    // no-allocation form holds counters per task).  The lens sampler's blocks
-    // are 8x8 pixels (a lane a pixel), so its tasks are too, up to the same
-    // number of buckets (tasks of 16x4 pixels left half its lanes without a
-    // pixel, of 4x4 three quarters).
-    const bool few = s.buckets.size() <= 16384;
-    const bool wide = o.shutter_open == o.shutter_close && few;
+    // motion sampler runs one workgroup a task and keeps the larger tasks.
+    // The lens sampler's blocks are 8x8 pixels (a lane a pixel), so its tasks
+    // are too (tasks of 16x4 pixels left half its lanes without a pixel, of
+    // 4x4 three quarters).  Both up to 16,384 buckets, and only where the frame
+    // then still has no more tasks than the no-allocation form holds counters
+    // for: a bucket has up to 16, so 3840x3840 at 2x2 samples in 32x32-pixel
+    // buckets would have 230,400 instead of 57,600.
+    bool fine = s.buckets.size() <= 16384;
     auto parts = [&](int bucket, int block) {
-        const int side = s.dof && few ? 8 : (wide ? std::max(2 * block, std::min(8, 4 * block)) : 4 * block);
+        const bool wide = fine && o.shutter_open == o.shutter_close;
+        const int side = s.dof && fine ? 8 : (wide ? std::max(2 * block, std::min(8, 4 * block)) : 4 * block);
         return std::max(1, std::min(4, bucket / side));
     };
+    if (s.buckets.size() * (size_t)(parts(o.bucket_x, s.blockW) * parts(o.bucket_y, s.blockH)) > kNoallocRows) fine = false;
     const int ntx = parts(o.bucket_x, s.blockW), nty = parts(o.bucket_y, s.blockH);
     s.tasks.clear();
     s.taskStart.assign(1, 0);

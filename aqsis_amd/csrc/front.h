@@ -15,6 +15,12 @@
 
 namespace rh {
 
+// Counter rows of the no-allocation form: its scratch array holds the frame's
+// counters and control words, then a row of five words per sampling workgroup,
+// whose number the launches round up to whole 128s.
+constexpr size_t kScratchRowsOffset = 256, kCounterRowBytes = 5 * sizeof(uint32_t);
+constexpr size_t kNoallocRows = (RH_NOALLOC_SCRATCH_BYTES - kScratchRowsOffset) / kCounterRowBytes / 128 * 128;
+
 // Frame shape: everything derived from the options alone.
 struct Shape {
     rh_options o;

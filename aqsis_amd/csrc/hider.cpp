@@ -526,11 +526,11 @@ void cached_plan(const rh::Shape& s, rh::Plan& out) {
 
 // Device memory of rh_render_device_noalloc, for callers that cannot
 // allocate: the frame's counters at 0, its hit-arena control words at 128,
-// the sampling workgroups' counter rows from kScratchRowsOffset.  Every GPU
+// the sampling workgroups' counter rows from kScratchRowsOffset (front.h).  Every GPU
 // holds its own copy until the process ends; host code reaches it only
 // through the address hipGetSymbolAddress gives on that device.
 static __device__ __align__(256) unsigned char scratch[RH_NOALLOC_SCRATCH_BYTES];
-static constexpr size_t kScratchRowsOffset = 256;
+using rh::kScratchRowsOffset;
 
 namespace {
 std::mutex g_scratchMu;
@@ -1496,10 +1496,10 @@ rh_status rh_render_device_noalloc(rh_ctx* c) {
     const int nt = (int)c->shape.tasks.size();
     const size_t rows = (c->sched.motion || c->shape.dof) ? (size_t)nt * (c->sched.motion ? 1 : c->dofSplit)
                                                           : (size_t)((std::max(nt, c->gridItems) + 127) / 128 * 128);
-    if (kScratchRowsOffset + rows * 5 * sizeof(uint32_t) > RH_NOALLOC_SCRATCH_BYTES)
+    if (kScratchRowsOffset + rows * rh::kCounterRowBytes > RH_NOALLOC_SCRATCH_BYTES)
         return fail(RH_ERR_CAPACITY, "the frame has " + std::to_string(nt) + " sampling tasks; the no-allocation "
                                      "form holds the counters of at most " +
-                                     std::to_string((RH_NOALLOC_SCRATCH_BYTES - kScratchRowsOffset) / 20) + " workgroups");
+                                     std::to_string((RH_NOALLOC_SCRATCH_BYTES - kScratchRowsOffset) / rh::kCounterRowBytes) + " workgroups");
     unsigned char* base = static_cast<unsigned char*>(c->scratch);
     const FrameCtl k{reinterpret_cast<unsigned long long*>(base), reinterpret_cast<uint32_t*>(base + 128),
                      reinterpret_cast<uint32_t*>(base + kScratchRowsOffset)};
