@@ -43,7 +43,7 @@ extern "C" hipError_t rh_launch_combine(hipStream_t, const FrameDev*, size_t, co
                                         const GridDev*, int, float4*, float*);
 extern "C" hipError_t rh_launch_reduce_counters(hipStream_t, const uint32_t*, int, const uint32_t*, int,
                                                 unsigned long long*, const uint32_t*, unsigned long long*);
-extern "C" hipError_t rh_launch_read_back(hipStream_t, const void*, void*, size_t, int, uint32_t*, uint32_t*, uint32_t);
+extern "C" hipError_t rh_launch_read_back(hipStream_t, const void*, void*, size_t, uint32_t*, uint32_t);
 extern "C" hipError_t rh_launch_format_display(hipStream_t, int, const DisplayFormat*, const float*, const float*,
                                                size_t, void*);
 extern "C" hipError_t rh_launch_box_classes(hipStream_t, const FrameDev*, int, const uchar4*, const float*, uint32_t*);
@@ -141,14 +141,15 @@ template <typename T> hipError_t upload(DBuf& b, const std::vector<T>& v, hipStr
 constexpr size_t kCtlBytes = 256, kSlabBytes = 64 << 10;
 constexpr int kLanes = 4;
 constexpr size_t kLaneBytes = 16 << 20;   // a 2048x2048 frame's 8-bit image
-constexpr int kLanePieces = kLaneBytes / RH_READ_WG_BYTES;
+constexpr size_t kLaneFlags = kLaneBytes / RH_READ_WG_BYTES;
 
+// Host memory alone, so that a lane serves a context on any device and holds
+// nothing that a failed copy could leave half done: a flag counts as set only
+// if it has its own copy's number.
 struct ReadLane {
-    int dev = 0;
-    uint32_t seq = 0;                     // of its last use: what a piece's flag is set to
-    unsigned char* p = nullptr;           // kLaneBytes, then a flag per piece
+    uint32_t seq = 0;                     // of its last use: what a workgroup's flag is set to
+    unsigned char* p = nullptr;           // kLaneBytes, then a flag per workgroup
     unsigned char* dp = nullptr;          // the device's address of p
-    uint32_t* done = nullptr;             // device: workgroups of each piece that are through
     volatile uint32_t* flags() const { return reinterpret_cast<volatile uint32_t*>(p + kLaneBytes); }
 };
 
@@ -189,25 +190,21 @@ struct PinnedPool {
         for (ReadLane* l : freeLanes) drop(l);
         freeLanes.clear();
     }
-    ReadLane* take_lane(int dev) {
+    ReadLane* take_lane() {
         std::lock_guard<std::mutex> lk(m);
-        for (size_t i = 0; i < freeLanes.size(); ++i)
-            if (freeLanes[i]->dev == dev) {
-                ReadLane* l = freeLanes[i];
-                freeLanes.erase(freeLanes.begin() + (long)i);
-                return l;
-            }
+        if (!freeLanes.empty()) {
+            ReadLane* l = freeLanes.back();
+            freeLanes.pop_back();
+            return l;
+        }
         if ((int)lanes.size() >= kLanes) return nullptr;
         ReadLane* l = new (std::nothrow) ReadLane();
         if (!l) return nullptr;
-        l->dev = dev;
         lanes.push_back(l);
-        const size_t flagBytes = kLanePieces * sizeof(uint32_t);
+        const size_t flagBytes = kLaneFlags * sizeof(uint32_t);
         if (hipHostMalloc(reinterpret_cast<void**>(&l->p), kLaneBytes + flagBytes,
                           hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess ||
-            hipHostGetDevicePointer(reinterpret_cast<void**>(&l->dp), l->p, 0) != hipSuccess ||
-            hipMalloc(reinterpret_cast<void**>(&l->done), flagBytes) != hipSuccess ||
-            hipMemset(l->done, 0, flagBytes) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+            hipHostGetDevicePointer(reinterpret_cast<void**>(&l->dp), l->p, 0) != hipSuccess) {
             (void)hipGetLastError();
             drop(l);
             return nullptr;
@@ -223,7 +220,6 @@ struct PinnedPool {
 
 private:
     void drop(ReadLane* l) {
-        if (l->done) (void)hipFree(l->done);
         if (l->p) (void)hipHostFree(l->p);
         lanes.erase(std::find(lanes.begin(), lanes.end(), l));
         delete l;
@@ -233,18 +229,16 @@ private:
 // Copy a result from the device, on its context's stream.  A plain copy into
 // pageable memory costs about 15 us and runs at 17 GB/s (one thread copies
 // out of the runtime's staging memory), an asynchronous copy of a piece 30
-// us; so a kernel writes the result into a lane and sets a flag after each
-// piece, and up to 8 of the worker pool's threads copy the pieces on as they
+// us; so a kernel writes the result into a lane, each workgroup setting a flag
+// behind its part, and up to 8 of the worker pool's threads copy the pieces on as they
 // arrive: 0.26 MB 127 to 33 us, 2.4 MB 141 to 90, 8.3 MB 485 to 280 (30
 // GB/s), 16.8 MB 966 to 460.
 // dst may be any host memory; src a context's buffer (read to a multiple of 16 bytes).
 constexpr size_t kReadPlain = 64 << 10;   // bytes below which the plain copy stays
 
 hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    ReadLane* lane = bytes >= kReadPlain ? PinnedPool::get().take_lane(dev) : nullptr;
+    ReadLane* lane = bytes >= kReadPlain ? PinnedPool::get().take_lane() : nullptr;
+    hipError_t e = hipSuccess;
     if (!lane) {
         e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
         return e == hipSuccess ? hipStreamSynchronize(st) : e;
@@ -257,22 +251,24 @@ hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st) {
         piece = (piece + RH_READ_WG_BYTES - 1) / RH_READ_WG_BYTES * RH_READ_WG_BYTES;
         const int n = (int)((len + piece - 1) / piece);
         const uint32_t seq = ++lane->seq;
-        e = rh_launch_read_back(st, static_cast<const unsigned char*>(src) + from, lane->dp, len, (int)(piece / RH_READ_WG_BYTES),
-                                lane->done, reinterpret_cast<uint32_t*>(lane->dp + kLaneBytes), seq);
+        e = rh_launch_read_back(st, static_cast<const unsigned char*>(src) + from, lane->dp, len,
+                                reinterpret_cast<uint32_t*>(lane->dp + kLaneBytes), seq);
         if (e != hipSuccess) break;
         std::atomic<bool> lost{false};
         auto take = [&](int i) {
-            const size_t at = (size_t)i * piece;
-            for (uint32_t spin = 0; lane->flags()[i] != seq; ++spin) {
-                // a stream that is through without the flag has failed
-                if ((spin & 0xfff) == 0xfff && hipStreamQuery(st) != hipErrorNotReady && lane->flags()[i] != seq) {
-                    lost = true;
-                    return;
+            const size_t at = (size_t)i * piece, end = std::min(at + piece, len);
+            uint32_t spin = 0;
+            for (size_t w = at / RH_READ_WG_BYTES; w * RH_READ_WG_BYTES < end; ++w)
+                while (lane->flags()[w] != seq) {
+                    // a stream that is through without the flag has failed
+                    if ((++spin & 0xfff) == 0 && hipStreamQuery(st) != hipErrorNotReady && lane->flags()[w] != seq) {
+                        lost = true;
+                        return;
+                    }
+                    __builtin_ia32_pause();
                 }
-                __builtin_ia32_pause();
-            }
             std::atomic_thread_fence(std::memory_order_acquire);
-            std::memcpy(to + at, lane->p + at, std::min(piece, len - at));
+            std::memcpy(to + at, lane->p + at, end - at);
         };
         if (n == 1 || !rh::run_if_free(n, 8, take))
             for (int i = 0; i < n; ++i) take(i);

@@ -2943,11 +2943,9 @@ __device__ __forceinline__ void filter_pixel(const FrameDev* __restrict__ fr, co
 }
 
 // Read-back: `bytes` bytes (rounded up to 16) of a result into pinned host
-// memory, RH_READ_WG_BYTES a workgroup; the last workgroup of each piece of
-// `per` sets the piece's flag in host memory to `seq` (and its device counter
-// back to 0), after every store of the piece is visible to the host.
+// memory, RH_READ_WG_BYTES a workgroup, which sets its flag in host memory to
+// `seq` after all its stores are visible to the host.  Bound by the link.
 __global__ void __launch_bounds__(256) rh_read_back(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t bytes,
-                                                    int per, uint32_t* __restrict__ done,
                                                     volatile uint32_t* __restrict__ flags, uint32_t seq) {
     const size_t n = (bytes + 15) / 16, base = (size_t)blockIdx.x * (RH_READ_WG_BYTES / 16);
     uint4 v[4];
@@ -2965,15 +2963,7 @@ __global__ void __launch_bounds__(256) rh_read_back(const uint4* __restrict__ sr
     }
     __threadfence_system();
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const int piece = (int)blockIdx.x / per;
-        const int wgs = min(per, (int)gridDim.x - piece * per);
-        if (atomicAdd(&done[piece], 1u) == (uint32_t)wgs - 1u) {
-            done[piece] = 0u;
-            __threadfence_system();
-            flags[piece] = seq;
-        }
-    }
+    if (threadIdx.x == 0) flags[blockIdx.x] = seq;
 }
 
 // A display request's values of each pixel (FormatBucketForDisplay,
@@ -3773,12 +3763,12 @@ extern "C" hipError_t rh_launch_reduce_counters(hipStream_t st, const uint32_t* 
                        counters, hitCtl, host);
     return hipGetLastError();
 }
-extern "C" hipError_t rh_launch_read_back(hipStream_t st, const void* src, void* dst, size_t bytes, int per,
-                                          uint32_t* done, uint32_t* flags, uint32_t seq) {
-    if (bytes == 0 || per < 1) return hipErrorInvalidValue;
+extern "C" hipError_t rh_launch_read_back(hipStream_t st, const void* src, void* dst, size_t bytes, uint32_t* flags,
+                                          uint32_t seq) {
+    if (bytes == 0) return hipErrorInvalidValue;
     const unsigned wgs = (unsigned)((bytes + RH_READ_WG_BYTES - 1) / RH_READ_WG_BYTES);
     hipLaunchKernelGGL(rh_read_back, dim3(wgs), dim3(256), 0, st, static_cast<const uint4*>(src),
-                       static_cast<uint4*>(dst), bytes, per, done, flags, seq);
+                       static_cast<uint4*>(dst), bytes, flags, seq);
     return hipGetLastError();
 }
 

@@ -1,0 +1,84 @@
+"""The host side of reading results back, on a HIP runtime that runs on the CPU
+(fake_hip.cpp): where its memory comes from and how long it is kept, what it
+waits for and what it holds meanwhile, and what a failed copy leaves behind.
+Each case is a process of its own; its frames hold no surfaces, so their
+channels are what the fake's new memory holds."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIP = "/opt/rocm/include"
+
+PRELUDE = """
+import ctypes as C, sys, threading, time
+sys.path.insert(0, sys.argv[2])
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+fake.fake_held.restype = C.c_uint64
+import numpy as np
+from aqsis_amd import hider, scenes
+from aqsis_amd.abi import default_options
+
+def rendered(w, h):
+    x = hider.Hider(default_options(xres=w, yres=h, filter="box", filter_xwidth=1.0, filter_ywidth=1.0))
+    x.render()
+    return x
+
+def right(a):
+    v = a.reshape(-1).view(np.uint32)
+    return np.array_equal(v, (np.arange(v.size, dtype=np.uint64) * 2654435761).astype(np.uint32))
+
+LANE, SLAB = 17 << 20, 64 << 10
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if gxx is None or not os.path.exists(os.path.join(HIP, "hip", "hip_runtime_api.h")):
+        pytest.skip("g++ or the HIP headers are not installed")
+    d = tmp_path_factory.mktemp("fake")
+    so = str(d / "libfake.so")
+    subprocess.run([gxx, "-O1", "-std=c++17", "-shared", "-fPIC", "-I", HIP,
+                    os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", so, "-lpthread"], check=True)
+
+    def go(code):
+        src = d / "case.py"
+        src.write_text(PRELUDE + textwrap.dedent(code))
+        r = subprocess.run([sys.executable, str(src), so, ROOT], capture_output=True, text=True, timeout=90)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return go
+
+
+def test_sizes_and_devices(run):
+    # a context on device 1, read while device 0 is current: whole results,
+    # and nothing is allocated on the device that is only current
+    run("""
+    for size in ((32, 32), (61, 31), (64, 65), (401, 325), (1024, 456), (1500, 1001)):
+        fake.hipSetDevice(1)
+        h = rendered(*size)
+        fake.hipSetDevice(0)
+        assert right(h.channels()) and right(h.rgba8()), size
+        assert fake.fake_held(0) == 0, size
+        h.close()
+    """)
+
+
+def test_failed_copy_leaves_nothing(run):
+    # a stream that ends without the data gives an error, and the next copy is whole
+    run("""
+    h = rendered(401, 325)
+    fake.fake_lose(1)
+    try:
+        h.channels()
+        raise SystemExit("no error")
+    except hider.HiderError:
+        pass
+    fake.fake_lose(0)
+    for _ in range(3):
+        assert right(h.channels())
+    """)
