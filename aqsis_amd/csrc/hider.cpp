@@ -136,93 +136,140 @@ template <typename T> hipError_t upload(DBuf& b, const std::vector<T>& v, hipStr
 // Pinned host memory of the process's contexts: a block of counters per
 // context, which the device writes at the end of a frame, and a few lanes
 // through which results are read back.  Taken from the driver when first
-// needed, handed back when the last context is destroyed; at most kLanes
-// lanes, a read that finds none free takes a plain copy.
+// needed, at most kLanes lanes; a read that finds none free takes a plain copy.
+// When the last context goes, all but one slab of blocks and one lane are
+// handed back: those two stay for the next context, since a program may make
+// one for every frame (taking and freeing them each time, a 256x256 frame's
+// first read took 110 us, so 60, and its context's end 1240, so 550).  The
+// driver is asked outside the lock, and only hipHostFree waits for the device.
 constexpr size_t kCtlBytes = 256, kSlabBytes = 64 << 10;
 constexpr int kLanes = 4;
 constexpr size_t kLaneBytes = 16 << 20;   // a 2048x2048 frame's 8-bit image
 constexpr size_t kLaneFlags = kLaneBytes / RH_READ_WG_BYTES;
 
+void* host_memory(size_t bytes) {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, bytes, hipHostMallocCoherent | hipHostMallocPortable) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // Host memory alone, so that a lane serves a context on any device and holds
 // nothing that a failed copy could leave half done: a flag counts as set only
 // if it has its own copy's number.
 struct ReadLane {
+    bool busy = false;
     uint32_t seq = 0;                     // of its last use: what a workgroup's flag is set to
     unsigned char* p = nullptr;           // kLaneBytes, then a flag per workgroup
     unsigned char* dp = nullptr;          // the device's address of p
     volatile uint32_t* flags() const { return reinterpret_cast<volatile uint32_t*>(p + kLaneBytes); }
 };
 
-struct PinnedPool {
-    std::mutex m;
-    int contexts = 0;
-    std::vector<void*> slabs, freeCtl;
-    std::vector<ReadLane*> lanes, freeLanes;
-
+class PinnedPool {
+public:
     static PinnedPool& get() {
         static PinnedPool* p = new PinnedPool();   // kept until the process ends
         return *p;
     }
     // A context's counter block; null when the driver has no pinned memory.
     void* take_ctl() {
-        std::lock_guard<std::mutex> lk(m);
-        if (freeCtl.empty()) {
-            void* s = nullptr;
-            if (hipHostMalloc(&s, kSlabBytes, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
-                (void)hipGetLastError();
-                return nullptr;
-            }
-            slabs.push_back(s);
-            for (size_t o = 0; o < kSlabBytes; o += kCtlBytes) freeCtl.push_back(static_cast<unsigned char*>(s) + o);
+        {
+            std::lock_guard<std::mutex> lk(m);
+            ++contexts;
+            if (void* p = pop_block()) return p;
         }
-        void* p = freeCtl.back();
-        freeCtl.pop_back();
-        ++contexts;
+        Slab* s = static_cast<Slab*>(host_memory(kSlabBytes));
+        std::lock_guard<std::mutex> lk(m);
+        if (s) {
+            s->next = slabs;
+            slabs = s;
+            link_blocks(s);
+        }
+        void* p = pop_block();
+        if (!p) --contexts;
         return p;
     }
-    void give_ctl(void* p) {
-        std::lock_guard<std::mutex> lk(m);
-        freeCtl.push_back(p);
-        if (--contexts > 0) return;
-        for (void* s : slabs) (void)hipHostFree(s);
-        slabs.clear();
-        freeCtl.clear();
-        for (ReadLane* l : freeLanes) drop(l);
-        freeLanes.clear();
+    void give_ctl(void* ctl) {
+        Slab* extra = nullptr;
+        unsigned char* lane[kLanes] = {};
+        {
+            std::lock_guard<std::mutex> lk(m);
+            push_block(ctl);
+            if (--contexts > 0) return;
+            // every block is free
+            extra = slabs->next;
+            slabs->next = nullptr;
+            blocks = nullptr;
+            link_blocks(slabs);
+            bool kept = false;
+            for (int i = 0; i < kLanes; ++i) {
+                ReadLane& l = lanes[i];
+                if (l.busy || !l.p) continue;
+                if (kept) std::swap(lane[i], l.p);
+                kept = true;
+            }
+        }
+        while (extra) {
+            Slab* next = extra->next;
+            (void)hipHostFree(extra);
+            extra = next;
+        }
+        for (unsigned char* p : lane)
+            if (p) (void)hipHostFree(p);
     }
     ReadLane* take_lane() {
-        std::lock_guard<std::mutex> lk(m);
-        if (!freeLanes.empty()) {
-            ReadLane* l = freeLanes.back();
-            freeLanes.pop_back();
-            return l;
+        ReadLane* l = nullptr;
+        {
+            std::lock_guard<std::mutex> lk(m);
+            for (ReadLane& c : lanes)
+                if (!c.busy && (!l || (c.p && !l->p))) l = &c;   // one that has its memory first
+            if (!l) return nullptr;
+            l->busy = true;
         }
-        if ((int)lanes.size() >= kLanes) return nullptr;
-        ReadLane* l = new (std::nothrow) ReadLane();
-        if (!l) return nullptr;
-        lanes.push_back(l);
-        const size_t flagBytes = kLaneFlags * sizeof(uint32_t);
-        if (hipHostMalloc(reinterpret_cast<void**>(&l->p), kLaneBytes + flagBytes,
-                          hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess ||
-            hipHostGetDevicePointer(reinterpret_cast<void**>(&l->dp), l->p, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            drop(l);
-            return nullptr;
+        if (!l->p) {
+            const size_t flagBytes = kLaneFlags * sizeof(uint32_t);
+            l->p = static_cast<unsigned char*>(host_memory(kLaneBytes + flagBytes));
+            if (l->p && hipHostGetDevicePointer(reinterpret_cast<void**>(&l->dp), l->p, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                (void)hipHostFree(l->p);
+                l->p = nullptr;
+            }
+            if (!l->p) {
+                give_lane(l);
+                return nullptr;
+            }
+            l->seq = 0;
+            std::memset(l->p + kLaneBytes, 0, flagBytes);
         }
-        std::memset(l->p + kLaneBytes, 0, flagBytes);
         return l;
     }
     void give_lane(ReadLane* l) {
         std::lock_guard<std::mutex> lk(m);
-        if (contexts > 0) freeLanes.push_back(l);
-        else drop(l);
+        l->busy = false;
     }
 
 private:
-    void drop(ReadLane* l) {
-        if (l->p) (void)hipHostFree(l->p);
-        lanes.erase(std::find(lanes.begin(), lanes.end(), l));
-        delete l;
+    // A slab's first block links the slabs; a free block, the free blocks.
+    struct Slab {
+        Slab* next;
+    };
+    std::mutex m;
+    int contexts = 0;
+    Slab* slabs = nullptr;
+    void* blocks = nullptr;
+    ReadLane lanes[kLanes];
+
+    void push_block(void* p) {
+        std::memcpy(p, &blocks, sizeof(blocks));
+        blocks = p;
+    }
+    void* pop_block() {
+        void* p = blocks;
+        if (p) std::memcpy(&blocks, p, sizeof(blocks));
+        return p;
+    }
+    void link_blocks(Slab* s) {
+        for (size_t o = kCtlBytes; o < kSlabBytes; o += kCtlBytes) push_block(reinterpret_cast<unsigned char*>(s) + o);
     }
 };
 

@@ -82,3 +82,41 @@ def test_failed_copy_leaves_nothing(run):
     for _ in range(3):
         assert right(h.channels())
     """)
+
+
+def test_a_context_a_frame(run):
+    # contexts one after another take pinned memory once, and never wait for the device
+    run("""
+    calls = []
+    for _ in range(6):
+        h = rendered(256, 256)
+        assert right(h.rgba8()) and right(h.channels())
+        h.close()
+        calls.append(fake.fake_pinned_calls())
+    assert calls[0] > 0 and calls == [calls[0]] * 6, calls
+    assert fake.fake_device_syncs() == 0
+    """)
+
+
+def test_pinned_memory_is_bounded_and_handed_back(run):
+    # many contexts read at once on four lanes at most; with the last of them
+    # all goes back but one lane and one slab of counter blocks
+    run("""
+    for _ in range(2):
+        hs = [rendered(401, 325) for _ in range(12)]
+        small = [rendered(16, 16) for _ in range(600)]
+        ok = [True] * len(hs)
+        def work(i):
+            for _ in range(4):
+                ok[i] = ok[i] and right(hs[i].channels())
+        ts = [threading.Thread(target=work, args=(i,)) for i in range(len(hs))]
+        fake.fake_gate(0)
+        for t in ts: t.start()
+        while fake.fake_waiting() < 4: time.sleep(0.01)
+        fake.fake_gate(1)
+        for t in ts: t.join()
+        assert all(ok)
+        assert 4 * (16 << 20) <= fake.fake_held(-1) <= 4 * LANE + 4 * SLAB
+        for h in hs + small: h.close()
+        assert fake.fake_held(-1) <= LANE + SLAB, fake.fake_held(-1)
+    """)
