@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <mutex>
 #include <cstring>
+#include <functional>
 #include <list>
 #include <memory>
 #include <new>
@@ -282,6 +283,11 @@ private:
 // GB/s), 16.8 MB 966 to 460.
 // dst may be any host memory; src a context's buffer (read to a multiple of 16 bytes).
 constexpr size_t kReadPlain = 64 << 10;   // bytes below which the plain copy stays
+// The GPU may be at another context's frame still, and the pool is every
+// context's: a read keeps it for 100 us more than the copy takes at 16 GB/s,
+// waits for data without it and takes it again.  (Taken only once data comes,
+// its threads wake too late: 2.4 MB 39 us longer.)
+constexpr std::chrono::microseconds kPoolHold{100};
 
 hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st) {
     ReadLane* lane = bytes >= kReadPlain ? PinnedPool::get().take_lane() : nullptr;
@@ -301,24 +307,63 @@ hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st) {
         e = rh_launch_read_back(st, static_cast<const unsigned char*>(src) + from, lane->dp, len,
                                 reinterpret_cast<uint32_t*>(lane->dp + kLaneBytes), seq);
         if (e != hipSuccess) break;
-        std::atomic<bool> lost{false};
-        auto take = [&](int i) {
+        using Clock = std::chrono::steady_clock;
+        const volatile uint32_t* flags = lane->flags();
+        // the first workgroup of [at, end) without its flag, from w on (SIZE_MAX: none)
+        auto missing = [&](size_t w, size_t end) {
+            while (w * RH_READ_WG_BYTES < end && flags[w] == seq) ++w;
+            return w * RH_READ_WG_BYTES < end ? w : SIZE_MAX;
+        };
+        // Wait for the workgroups of [at, end); false if the stream is through
+        // without them: it has failed.
+        auto wait = [&](size_t at, size_t end) {
+            uint32_t spin = 0;
+            for (size_t w = missing(at / RH_READ_WG_BYTES, end); w != SIZE_MAX; w = missing(w, end)) {
+                if ((++spin & 0xfff) == 0 && hipStreamQuery(st) != hipErrorNotReady && flags[w] != seq) return false;
+                __builtin_ia32_pause();
+            }
+            return true;
+        };
+        auto copy = [&](int i) {
+            const size_t at = (size_t)i * piece;
+            std::atomic_thread_fence(std::memory_order_acquire);
+            std::memcpy(to + at, lane->p + at, std::min(piece, len - at));
+        };
+        std::atomic<uint32_t> taken{0};                  // pieces copied
+        Clock::time_point until;                         // when the pool is given up
+        auto help = [&](int i) {
+            if ((taken >> i) & 1u) return;
             const size_t at = (size_t)i * piece, end = std::min(at + piece, len);
             uint32_t spin = 0;
-            for (size_t w = at / RH_READ_WG_BYTES; w * RH_READ_WG_BYTES < end; ++w)
-                while (lane->flags()[w] != seq) {
-                    // a stream that is through without the flag has failed
-                    if ((++spin & 0xfff) == 0 && hipStreamQuery(st) != hipErrorNotReady && lane->flags()[w] != seq) {
-                        lost = true;
-                        return;
-                    }
-                    __builtin_ia32_pause();
-                }
-            std::atomic_thread_fence(std::memory_order_acquire);
-            std::memcpy(to + at, lane->p + at, end - at);
+            for (size_t w = missing(at / RH_READ_WG_BYTES, end); w != SIZE_MAX; w = missing(w, end)) {
+                if ((++spin & 0x3f) == 0 && Clock::now() > until) return;
+                __builtin_ia32_pause();
+            }
+            copy(i);
+            taken |= 1u << i;
         };
-        if (n == 1 || !rh::run_if_free(n, 8, take))
-            for (int i = 0; i < n; ++i) take(i);
+        bool lost = false;
+        for (int i = 0; i < n && !lost;) {
+            if ((taken >> i) & 1u) {
+                ++i;
+                continue;
+            }
+            bool shared = false;
+            if (n - i > 1) try {
+                    until = Clock::now() + kPoolHold + std::chrono::nanoseconds(len / 16);
+                    shared = rh::run_if_free(n, 8, std::ref(help));
+                } catch (...) {
+                    // no thread for the pool: alone
+                }
+            if (shared && ((taken >> i) & 1u)) continue;
+            // alone: until the piece's data begins to come, or for the whole piece
+            const size_t at = (size_t)i * piece, end = std::min(at + piece, len);
+            lost = !wait(at, shared ? std::min(at + RH_READ_WG_BYTES, end) : end);
+            if (!lost && !shared) {
+                copy(i);
+                taken |= 1u << i;
+            }
+        }
         // nothing may still be writing to the lane when it is used again
         e = hipStreamSynchronize(st);
         if (e == hipSuccess && lost) e = hipErrorUnknown;

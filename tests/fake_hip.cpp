@@ -34,7 +34,8 @@ struct Block {
 thread_local int t_dev = 0;
 std::mutex g_m;
 std::condition_variable g_gateCv;
-bool g_gate = true, g_lose = false;
+int g_gate = -1;                          // workgroups of each copy let through (-1: all)
+bool g_lose = false;
 bool g_refusePinned = false;
 std::map<void*, Block> g_blocks;
 std::map<const void*, std::string> g_kernels;
@@ -67,14 +68,17 @@ Stream* S(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
 
 // rh_read_back(src, dst, bytes, flags, seq), a workgroup at a time
 void read_back(Stream* st, unsigned grid, const char* src, char* dst, size_t bytes, volatile uint32_t* flags, uint32_t seq) {
-    ++g_waiting;
-    {
-        std::unique_lock<std::mutex> lk(g_m);
-        g_gateCv.wait(lk, [] { return g_gate; });
-    }
-    --g_waiting;
     const size_t per = 65536;
     for (unsigned w = 0; w < grid && !g_lose; ++w) {
+        {
+            std::unique_lock<std::mutex> lk(g_m);
+            auto open = [w] { return g_gate < 0 || (int)w < g_gate; };
+            if (!open()) {
+                ++g_waiting;
+                g_gateCv.wait(lk, open);
+                --g_waiting;
+            }
+        }
         std::memcpy(dst + w * per, src + w * per, std::min(per, bytes - w * per));
         std::atomic_thread_fence(std::memory_order_release);
         flags[w] = seq;
@@ -88,9 +92,9 @@ void read_back(Stream* st, unsigned grid, const char* src, char* dst, size_t byt
 
 extern "C" {
 
-void fake_gate(int open) {
+void fake_gate(int workgroups) {
     std::lock_guard<std::mutex> lk(g_m);
-    g_gate = open != 0;
+    g_gate = workgroups;
     g_gateCv.notify_all();
 }
 void fake_lose(int on) { g_lose = on != 0; }

@@ -113,10 +113,34 @@ def test_pinned_memory_is_bounded_and_handed_back(run):
         fake.fake_gate(0)
         for t in ts: t.start()
         while fake.fake_waiting() < 4: time.sleep(0.01)
-        fake.fake_gate(1)
+        fake.fake_gate(-1)
         for t in ts: t.join()
         assert all(ok)
         assert 4 * (16 << 20) <= fake.fake_held(-1) <= 4 * LANE + 4 * SLAB
         for h in hs + small: h.close()
         assert fake.fake_held(-1) <= LANE + SLAB, fake.fake_held(-1)
     """)
+
+
+@pytest.mark.parametrize("workgroups", [0, 1, 9])
+def test_other_threads_have_the_worker_pool(run, workgroups):
+    # a read whose data has not come, or only its first parts, does not keep a
+    # schedule of another thread from the worker pool
+    run("""
+    opts, prims = scenes.patches_scene(seed=1, n=400, res=(320, 240))
+    h = rendered(1024, 456)
+    out = []
+    fake.fake_gate(%d)
+    a = threading.Thread(target=lambda: out.append(right(h.channels())), daemon=True)
+    a.start()
+    while fake.fake_waiting() < 1: time.sleep(0.01)
+    time.sleep(0.05)
+    b = threading.Thread(target=lambda: hider.estimate(opts, prims), daemon=True)
+    b.start()
+    b.join(20)
+    assert not b.is_alive(), "the schedule waits for the read"
+    assert a.is_alive()
+    fake.fake_gate(-1)
+    a.join()
+    assert out == [True]
+    """ % workgroups)
