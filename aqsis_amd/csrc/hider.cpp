@@ -432,7 +432,8 @@ struct rh_ctx {
         graph = nullptr;
     }
     void* scratch = nullptr;              // this device's scratch array (rh_render_device_noalloc)
-    // pinned: a frame's counters and hit control words as its last kernels leave them
+    // pinned: a frame's counters and hit control words as its last kernels leave
+    // them (null when the driver had no pinned memory: then they are copied)
     unsigned long long* hostCtl = nullptr;
     unsigned long long* hostCtlDev = nullptr;   // the device's address of it
     FrameDev frame;                       // host copy of dFrame
@@ -789,8 +790,7 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
     c->each_buffer([c](DBuf& b) { b.st = c->st; });
     if (e == hipSuccess) {
         c->hostCtl = static_cast<unsigned long long*>(PinnedPool::get().take_ctl());
-        if (!c->hostCtl) { delete c; return fail(RH_ERR_NOMEM, "no pinned host memory"); }
-        e = hipHostGetDevicePointer(reinterpret_cast<void**>(&c->hostCtlDev), c->hostCtl, 0);
+        if (c->hostCtl) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&c->hostCtlDev), c->hostCtl, 0);
     }
     for (int i = 0; i < 6 && e == hipSuccess; ++i) e = hipEventCreate(&c->ev[i]);
     if (e != hipSuccess) { delete c; return fail(RH_ERR_DEVICE, std::string("stream/event creation: ") + hipGetErrorString(e)); }
@@ -1469,10 +1469,15 @@ static rh_status cull_schedule(rh_ctx* c, const rh::Forest& forest) {
 static rh_status finish_frame(rh_ctx* c, const unsigned long long* cnt, bool staged);
 
 // A completed frame's counters and hit control words.
-static void read_ctl(const rh_ctx* c, unsigned long long* cnt, uint32_t* hc) {
+static hipError_t read_ctl(const rh_ctx* c, const FrameCtl& k, unsigned long long* cnt, uint32_t* hc) {
+    if (!c->hostCtl) {
+        const hipError_t e = hipMemcpy(cnt, k.counters, RH_NCOUNTERS * sizeof(*cnt), hipMemcpyDeviceToHost);
+        return e == hipSuccess ? hipMemcpy(hc, k.hitCtl, RH_HOST_HITCTL * sizeof(*hc), hipMemcpyDeviceToHost) : e;
+    }
     const volatile unsigned long long* h = c->hostCtl;
     for (int i = 0; i < RH_NCOUNTERS; ++i) cnt[i] = i < 7 ? h[i] : 0ull;
     for (int i = 0; i < RH_HOST_HITCTL; ++i) hc[i] = (uint32_t)h[RH_NCOUNTERS + i];
+    return hipSuccess;
 }
 
 // One frame on the resident inputs.  The batched form replays its frame
@@ -1513,7 +1518,7 @@ static rh_status render_frame(rh_ctx* c, bool eager) {
         }
         HIP_TRY(hipEventSynchronize(c->ev[4]));
         uint32_t hc[RH_HOST_HITCTL];
-        read_ctl(c, cnt, hc);
+        HIP_TRY(read_ctl(c, context_ctl(c), cnt, hc));
         if (hc[0] > 0) {
             // The arena ran out: redo the frame with room for every hit.
             if (attempt >= 2) return fail(RH_ERR_CAPACITY, "transparent-hit arena kept overflowing");
@@ -1596,7 +1601,7 @@ rh_status rh_render_device_noalloc(rh_ctx* c) {
     HIP_TRY(hipEventSynchronize(c->ev[4]));
     unsigned long long cnt[RH_NCOUNTERS];
     uint32_t hc[RH_HOST_HITCTL];
-    read_ctl(c, cnt, hc);
+    HIP_TRY(read_ctl(c, k, cnt, hc));
     if (hc[0] > 0)
         return fail(RH_ERR_CAPACITY, "the frame needs " + std::to_string((uint64_t)c->frame.hitCapacity + hc[0]) +
                                          " transparent-hit entries and the "

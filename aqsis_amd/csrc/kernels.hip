@@ -705,8 +705,8 @@ __global__ void __launch_bounds__(256) rh_bin_write(const BucketDev* __restrict_
 // Frame counters from the sampling rows and per-bucket rows: counters[0..4] the
 // hider's SPL counts, counters[6] the micropolygon-bucket references.  `host`:
 // the counters and the first hit control words once more, in pinned host
-// memory (hostCtl of a context), so that the host reads them after the frame
-// without a copy (two blocking copies took 25 us of every frame).
+// memory (hostCtl of a context, null without such memory), so that the host reads
+// them after the frame without a copy (two blocking copies took 25 us of every frame).
 // One workgroup.
 __global__ void __launch_bounds__(1024) rh_reduce_counters(const uint32_t* __restrict__ rowCounts, int nrows,
                                                            const uint32_t* __restrict__ bucketRefs, int nbuckets,
@@ -729,10 +729,10 @@ __global__ void __launch_bounds__(1024) rh_reduce_counters(const uint32_t* __res
         unsigned long long v = 0;
         for (int w = 0; w < 16; ++w) v += part[tid][w];
         counters[tid < 5 ? tid : 6] = v;
-        host[tid < 5 ? tid : 6] = v;
-    } else if (tid < 6 + RH_HOST_HITCTL) {
+        if (host) host[tid < 5 ? tid : 6] = v;
+    } else if (host && tid < 6 + RH_HOST_HITCTL) {
         host[RH_NCOUNTERS + tid - 6] = hitCtl[tid - 6];
-    } else if (tid == 6 + RH_HOST_HITCTL) {
+    } else if (host && tid == 6 + RH_HOST_HITCTL) {
         host[5] = counters[5];            // counted while the lists were built
     }
     __threadfence_system();

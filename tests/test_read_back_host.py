@@ -144,3 +144,22 @@ def test_other_threads_have_the_worker_pool(run, workgroups):
     a.join()
     assert out == [True]
     """ % workgroups)
+
+
+def test_without_pinned_memory(run):
+    # the driver refuses pinned memory: contexts are made and frames read by plain copies
+    run("""
+    fake.fake_refuse_pinned(1)
+    for _ in range(2):
+        h = rendered(401, 325)
+        assert right(h.channels()) and right(h.rgba8())
+        h.render_device()
+        h.render_device_noalloc()
+        assert h.stats()["spl_count"] == 0
+        h.close()
+    fake.fake_refuse_pinned(0)
+    h, g = rendered(401, 325), rendered(64, 64)
+    assert right(h.channels())
+    h.close(); g.close()
+    assert fake.fake_held(-1) == LANE // 17 * 16 + 1024 + SLAB
+    """)
