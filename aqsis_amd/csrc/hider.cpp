@@ -650,9 +650,14 @@ hipError_t scratch_address(void** out) {
 // longest workgroup (64x64: 118 to 34 us; 256x256: 112 to 95), and an item's
 // list is staged once per item, so a frame that fills the device keeps whole
 // tasks (512x512 with 8192 items: 318 to 332 us).
-static std::vector<uint2> grid_items(const std::vector<uint2>& tasks, int blocks) {
+static int item_blocks(uint64_t blocks) {
     int per = 16;
     while (per > 4 && blocks / per < 4096) per >>= 1;
+    return per;
+}
+
+static std::vector<uint2> grid_items(const std::vector<uint2>& tasks, int blocks) {
+    const int per = item_blocks(blocks);
     if (per == 16) return tasks;
     std::vector<uint2> out;
     for (const uint2& t : tasks) {
@@ -1902,10 +1907,31 @@ uint64_t rh_internal_device_bytes(const rh_ctx* c) {
 
 extern "C" {
 
+// What rh_create and the frame's shape take on the device.
 static uint64_t frame_bytes(const rh::Shape& s) {
-    uint64_t ext = (uint64_t)s.extW * s.extH;
-    return ext * s.ns * 32 + ext * 4 + (uint64_t)s.width() * s.height() * (9 * 4 + 4 + 4) +
-           s.buckets.size() * (sizeof(BucketDev) + 4 + 8 + 4 + 64);
+    const uint64_t ext = (uint64_t)s.extW * s.extH, ns = s.ns, tasks = s.tasks.size();
+    auto blocks_of = [&](const rh::Shape::TaskInfo& t) {
+        return (uint64_t)((t.x1 - t.x0 + s.blockW - 1) / s.blockW) * ((t.y1 - t.y0 + s.blockH - 1) / s.blockH);
+    };
+    uint64_t blocks = 0, items = tasks;
+    for (const auto& t : s.tasks) blocks += blocks_of(t);
+    const int per = item_blocks(blocks);
+    if (per < 16) {
+        items = 0;
+        for (const auto& t : s.tasks) items += (blocks_of(t) + per - 1) / per;
+    }
+    // samples, sample patterns and their tables, channels, 8-bit image, dither draws
+    uint64_t bytes = ext * (ns * 32 + 4) + 250 * ns * 12 + (uint64_t)s.width() * s.height() * (9 * 4 + 4 + 4);
+    if (s.dof) bytes += ext + 250 * ns * 9 + ns * 16;
+    bytes += s.buckets.size() * (sizeof(BucketDev) + 4 + 4);
+    // list counts and capacities, work items, counter rows; the batched form's items
+    bytes += tasks * (sizeof(TaskDev) + 4 + 8 + 8) + items * (8 + 20) + blocks * 8;
+    bytes += 128 << 10;                    // the other counter rows, the filter's list, control words
+    // The filter's box tests, where they can differ between pixels: a sample of
+    // the outermost column or row lies within the box by where it is in its
+    // pixel, if the box ends inside that pixel.
+    if (s.xfwo2 < s.shiftX + 0.5f || s.yfwo2 < s.shiftY + 0.5f) bytes += ext * (2 * s.shiftX + 2 * s.shiftY + 2) * 8;
+    return bytes;
 }
 
 }  // extern "C"

@@ -194,7 +194,10 @@ typedef struct rh_footprint {
     uint64_t micropolygons;
     uint64_t vertices;
     uint64_t list_capacity;    /* task micropolygon-list entries reserved       */
-    uint64_t device_bytes;     /* device memory of the frame (shape + schedule) */
+    /* device memory of the frame (shape + schedule), rendered and read as
+     * channels or 8-bit values; a context that formats display values on the
+     * device keeps a buffer of a request's values and dither draws besides */
+    uint64_t device_bytes;
 } rh_footprint;
 
 /*

@@ -1,7 +1,7 @@
-"""The host side of reading results back, on a HIP runtime that runs on the CPU
-(fake_hip.cpp): where its memory comes from and how long it is kept, what it
-waits for and what it holds meanwhile, and what a failed copy leaves behind.
-Each case is a process of its own; its frames hold no surfaces, so their
+"""The library's host side on a HIP runtime that runs on the CPU (fake_hip.cpp).
+Reading results back: where its memory comes from and how long it is kept, what
+it waits for and what it holds meanwhile, and what a failed copy leaves behind.
+The estimate of a frame's device memory against what a context takes.  Each case is a process of its own; its frames hold no surfaces, so their
 channels are what the fake's new memory holds."""
 import os
 import shutil
@@ -163,3 +163,25 @@ def test_without_pinned_memory(run):
     h.close(); g.close()
     assert fake.fake_held(-1) == LANE // 17 * 16 + 1024 + SLAB
     """)
+
+
+@pytest.mark.parametrize("samples", [(1, 1), (2, 2), (3, 3), (4, 4), (8, 8)])
+def test_estimate_holds_what_a_context_takes(run, samples):
+    # with even filter widths the box tests may differ between pixels and are
+    # kept by pixel; a job admitted by its estimate has to have room for them
+    run("""
+    for res in ((48, 40), (256, 256), (637, 475)):
+        for width, varies in ((1.0, 0), (2.0, 1), (2.5, 0), (3.0, 0), (4.0, 1), (6.0, 1), (7.0, 0)):
+            for bucket, lens in ((16, 0), (32, 0), (16, 1)):
+                if res[0] > 256 and (bucket != 32 or width not in (1.0, 4.0)): continue
+                o = default_options(xres=res[0], yres=res[1], xsamples=%d, ysamples=%d, filter="gaussian",
+                                    filter_xwidth=width, filter_ywidth=width)
+                o.bucket_x = o.bucket_y = bucket
+                if lens: o.dof[:] = [22.0, 45.0, 1200.0]
+                fake.fake_box_varies(varies)
+                h = hider.Hider(o)
+                h.render()
+                need, said = fake.fake_held(0), hider.estimate(o, [])["device_bytes"]
+                h.close()
+                assert need <= said <= need + need // 20 + (256 << 10), (res, width, bucket, lens, need, said)
+    """ % samples)
