@@ -49,3 +49,20 @@ def test_values_are_the_hosts(frame, kind, q):
         assert z.shape == (h.height, h.width, 1)
     if one == 0.0 and kind == "float32":
         assert np.array_equal(z[..., 0].view(np.uint32), ch[..., 7].copy().view(np.uint32))
+
+
+@pytest.mark.parametrize("q", QUANTIZE)
+@pytest.mark.parametrize("kind", list(DSPY))
+def test_depth_requests_of_each_place(oracle, frame, kind, q):
+    # depths, the background's FLT_MAX among them (past the 64-bit range when
+    # quantised), with the dither draws of each of the two requests
+    from aqsis_amd.hider import mode_bits
+    opts, h = frame
+    ch = h.channels()
+    assert (ch[..., 7] == np.finfo(np.float32).max).any()
+    for index in (0, 1):
+        _, draws = oracle.sample_positions(opts, display=index)
+        for mode in ("z", "rgbaz"):
+            got = h.display_request_values(mode, q, index, kind)
+            want = oracle.display_request_values(q, mode_bits(mode), ch, draws, DSPY[kind])
+            assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want).view(np.uint8)), (mode, index)
