@@ -949,22 +949,24 @@ rh_status rh_clear_surfaces(rh_ctx* c) {
     return RH_OK;
 }
 
+constexpr uint64_t kMaxHits = RH_HIT_NOROOM - 1;
+
 // Transparent-hit arena entries a frame is likely to need: each transparent
 // micropolygon covers about one pixel at ShadingRate 1, so about ns samples
-// (at least 1M entries).  A frame that needs more is redone once with the
-// exact size.
+// (at least 1M entries).  A frame that needs more is redone with a quarter
+// more room than it asked for, at most twice.
 static uint64_t arena_guess(const rh::Shape& s, const rh::Schedule& S, const rh_prim* prims) {
     uint64_t tmp = 0;
     for (const auto& g : S.grids)
         if (rh::hits_listed(s.o, prims[g.prim])) tmp += (uint64_t)g.cu * g.cv;
     if (tmp == 0) return 0;
-    return std::min<uint64_t>(std::max<uint64_t>(1u << 20, tmp * (uint64_t)s.ns), 0x7fffffffull);
+    return std::min<uint64_t>(std::max<uint64_t>(1u << 20, tmp * (uint64_t)s.ns), kMaxHits);
 }
 
 // Size the transparent-hit arena and publish its capacity to the kernels.
 static rh_status set_hit_capacity(rh_ctx* c, uint64_t n) {
     if (n < 64) n = 64;
-    if (n > 0x7fffffffull) return fail(RH_ERR_CAPACITY, "transparent hits exceed 2^31 entries");
+    if (n > kMaxHits) return fail(RH_ERR_CAPACITY, "transparent hits exceed 2^31 entries");
     HIP_TRY(c->dHitData.ensure(n * sizeof(float4)));
     HIP_TRY(c->dHitNext.ensure(n * sizeof(uint2)));
     c->frame.hitCapacity = (uint32_t)n;
@@ -1528,7 +1530,7 @@ static rh_status render_frame(rh_ctx* c, bool eager) {
             // The arena ran out: redo the frame with room for every hit.
             if (attempt >= 2) return fail(RH_ERR_CAPACITY, "transparent-hit arena kept overflowing");
             const uint64_t need = (uint64_t)c->frame.hitCapacity + hc[0];
-            rh_status r = set_hit_capacity(c, need + need / 4 + 64);
+            rh_status r = set_hit_capacity(c, need > kMaxHits ? need : std::min(need + need / 4 + 64, kMaxHits));
             if (r != RH_OK) return r;
             continue;
         }

@@ -39,15 +39,20 @@ bool g_lose = false;
 bool g_refusePinned = false, g_boxVaries = false;
 std::map<void*, Block> g_blocks;
 std::map<const void*, std::string> g_kernels;
+size_t g_most = SIZE_MAX;                 // bytes of the largest allocation granted
+std::atomic<uint32_t> g_noRoom{0};        // transparent hits the next frame has no room for
 std::atomic<int> g_deviceSyncs{0}, g_pinnedCalls{0}, g_plainCopies{0}, g_waiting{0};
 
 struct Config { dim3 grid, wg; size_t lds; hipStream_t st; };
 thread_local Config t_config;
 
 hipError_t take(void** p, size_t bytes, int dev) {
-    void* q = std::aligned_alloc(256, (bytes + 255) / 256 * 256);
+    if (bytes > g_most) return hipErrorOutOfMemory;
+    // (of more than a gigabyte only the first words are there: nothing reads them)
+    const size_t real = bytes > (size_t(1) << 30) ? 4096 : bytes;
+    void* q = std::aligned_alloc(256, (real + 255) / 256 * 256);
     if (!q) return hipErrorOutOfMemory;
-    for (size_t i = 0; i < bytes / 4; ++i) static_cast<uint32_t*>(q)[i] = (uint32_t)i * 2654435761u;
+    for (size_t i = 0; i < real / 4; ++i) static_cast<uint32_t*>(q)[i] = (uint32_t)i * 2654435761u;
     std::lock_guard<std::mutex> lk(g_m);
     g_blocks[q] = Block{bytes, dev};
     *p = q;
@@ -97,6 +102,8 @@ void fake_gate(int workgroups) {
     g_gate = workgroups;
     g_gateCv.notify_all();
 }
+void fake_most(uint64_t bytes) { g_most = bytes; }
+void fake_no_room(uint32_t n) { g_noRoom = n; }
 void fake_lose(int on) { g_lose = on != 0; }
 void fake_box_varies(int on) { g_boxVaries = on != 0; }
 void fake_refuse_pinned(int on) { g_refusePinned = on != 0; }
@@ -133,10 +140,16 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* wg, size_t* lds, hipStrea
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, hipStream_t st) {
     const std::string& name = g_kernels[f];
     if (name.find("rh_reduce_counters") != std::string::npos) {
-        // no hits: rh_reduce_counters(rows, nrows, refs, nbuckets, counters, hitCtl, host)
+        // no hits but those without room: rh_reduce_counters(rows, nrows, refs,
+        // nbuckets, counters, hitCtl, host)
         std::memset(*static_cast<void**>(args[4]), 0, 9 * 8);
-        std::memset(*static_cast<void**>(args[5]), 0, 4 * 4);
-        if (void* host = *static_cast<void**>(args[6])) std::memset(host, 0, 13 * 8);
+        uint32_t* ctl = *static_cast<uint32_t**>(args[5]);
+        std::memset(ctl, 0, 4 * 4);
+        ctl[0] = g_noRoom.exchange(0);
+        if (unsigned long long* host = *static_cast<unsigned long long**>(args[6])) {
+            std::memset(host, 0, 13 * 8);
+            host[9] = ctl[0];
+        }
     }
     if (name.find("rh_box_classes") != std::string::npos) {
         // rh_box_classes(frame, patterns, positions, rows): every test may hold, and does not always or does

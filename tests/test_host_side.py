@@ -1,7 +1,8 @@
 """The library's host side on a HIP runtime that runs on the CPU (fake_hip.cpp).
 Reading results back: where its memory comes from and how long it is kept, what
 it waits for and what it holds meanwhile, and what a failed copy leaves behind.
-The estimate of a frame's device memory against what a context takes.  Each case is a process of its own; its frames hold no surfaces, so their
+The estimate of a frame's device memory against what a context takes.  The
+growth of the transparent-hit arena at its limits.  Each case is a process of its own; its frames hold no surfaces, so their
 channels are what the fake's new memory holds."""
 import os
 import shutil
@@ -185,3 +186,18 @@ def test_estimate_holds_what_a_context_takes(run, samples):
                 h.close()
                 assert need <= said <= need + need // 20 + (256 << 10), (res, width, bucket, lens, need, said)
     """ % samples)
+
+
+@pytest.mark.parametrize("missing,taken", [(1 << 20, True), (1_600_000_000, True), (1_900_000_000, True),
+                                           (2_146_000_000, True), (2_147_483_647, False)])
+def test_arena_grows_to_its_limit(run, missing, taken):
+    # entries below 2^31 in all: the spare quarter does not count against them
+    run("""
+    h = hider.Hider(default_options(xres=64, yres=64))
+    fake.fake_no_room(%d)
+    try:
+        h.render()
+        assert %r
+    except hider.HiderError as e:
+        assert not %r and "2^31" in str(e), e
+    """ % (missing, taken, taken))
