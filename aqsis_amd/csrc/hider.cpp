@@ -967,8 +967,15 @@ static uint64_t arena_guess(const rh::Shape& s, const rh::Schedule& S, const rh_
 static rh_status set_hit_capacity(rh_ctx* c, uint64_t n) {
     if (n < 64) n = 64;
     if (n > kMaxHits) return fail(RH_ERR_CAPACITY, "transparent hits exceed 2^31 entries");
-    HIP_TRY(c->dHitData.ensure(n * sizeof(float4)));
-    HIP_TRY(c->dHitNext.ensure(n * sizeof(uint2)));
+    hipError_t e = c->dHitData.ensure(n * sizeof(float4));
+    if (e == hipSuccess) e = c->dHitNext.ensure(n * sizeof(uint2));
+    if (e != hipSuccess) {
+        // the old arena may be gone while the device's copy of the frame still
+        // has its size: no frame until rh_render has made a new one
+        c->frame.hitCapacity = 0;
+        c->scheduled = false;
+        return fail(RH_ERR_DEVICE, std::string("transparent-hit arena: ") + hipGetErrorString(e));
+    }
     c->frame.hitCapacity = (uint32_t)n;
     c->dropGraph();
     std::vector<FrameDev> fv(1, c->frame);

@@ -20,6 +20,7 @@ import ctypes as C, sys, threading, time
 sys.path.insert(0, sys.argv[2])
 fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 fake.fake_held.restype = C.c_uint64
+fake.fake_most.argtypes = [C.c_uint64]
 import numpy as np
 from aqsis_amd import hider, scenes
 from aqsis_amd.abi import default_options
@@ -201,3 +202,22 @@ def test_arena_grows_to_its_limit(run, missing, taken):
     except hider.HiderError as e:
         assert not %r and "2^31" in str(e), e
     """ % (missing, taken, taken))
+
+
+def test_no_frame_on_an_arena_that_could_not_grow(run):
+    run("""
+    h = hider.Hider(default_options(xres=64, yres=64))
+    h.render()
+    for again in (h.render_device, h.render_device_noalloc, h.render_stages):
+        fake.fake_no_room(1 << 22)
+        fake.fake_most(1 << 20)
+        for f in (h.render_device, again):
+            try:
+                f()
+                raise SystemExit("a frame on a missing arena")
+            except hider.HiderError:
+                pass
+        fake.fake_most(1 << 40)
+        h.render()
+        again()
+    """)
