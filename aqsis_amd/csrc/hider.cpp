@@ -320,7 +320,8 @@ hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st) {
             uint32_t spin = 0;
             for (size_t w = missing(at / RH_READ_WG_BYTES, end); w != SIZE_MAX; w = missing(w, end)) {
                 if ((++spin & 0xfff) == 0 && hipStreamQuery(st) != hipErrorNotReady && flags[w] != seq) return false;
-                __builtin_ia32_pause();
+                if (spin < 0x4000) __builtin_ia32_pause();
+                else std::this_thread::yield();         // the GPU is at something else
             }
             return true;
         };
