@@ -1,15 +1,15 @@
 // HIP kernels of the hider for gfx950 (CDNA4).
 //
 //   rh_dice_bust        one workgroup per grid: dice (sphere / bicubic /
-//                       bilinear), project to raster, and write one hit-test
-//                       record per micropolygon (edge equations, inverse-
-//                       bilinear set-up, depths, bound, opacity).
+//                       bilinear), project to raster, and write one record per
+//                       micropolygon (its vertices and depths, flags, grid and
+//                       surface) and its bound for the binning.
 //   rh_bin_count/scan/write
 //                       per (bucket, candidate grid) segment: keep the
 //                       micropolygons the bucket would have received (AddMPG)
 //                       and append them, in order, to the lists of the tasks
 //                       (parts of the bucket's sample region) they touch.
-//   rh_plan_items       batched form: cut tasks into work items by cost,
+//   rh_plan_count/items batched form: cut tasks into work items by cost,
 //                       largest first.
 //   rh_sample           one wave per block of 64 samples, a workgroup per
 //                       work item: the reference's per-sample tests (bound,
@@ -762,8 +762,8 @@ __global__ void __launch_bounds__(1024) rh_reduce_counters(const uint32_t* __res
 // pixel sub-sample clip, in sub-sample grid units, so every sample sees the
 // reference's sequence of tests.
 // The sampling form of a micropolygon record, from its compact form (the
-// four raster vertices in grid order, their depths, bound, minimum depth,
-// flags and grid): cachePointInPolyTest's edge equations on the vertices in
+// four raster vertices in grid order, their depths, flags and surface):
+// cachePointInPolyTest's edge equations on the vertices in
 // the order the vertex-order code gives (micropolygon.cpp:1346-1392, a
 // degenerate micropolygon repeats its closing edge) and CqInvBilinear's
 // set-up on the grid-order vertices (bilinear.h:260-275).  Out: YM, XM, X, Y,
@@ -989,7 +989,7 @@ rh_sample(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets
           const uint2* __restrict__ items, int itemBase, int nStatic, const uint32_t* __restrict__ nDevice,
           int persistent, uint32_t* __restrict__ queueHead, const unsigned long long* __restrict__ capStart,
           const uint32_t* __restrict__ listCount, const uint32_t* __restrict__ lists,
-          const float4* __restrict__ mprec4, const GridDev* __restrict__ grids, const PrimDev* __restrict__ prims,
+          const float4* __restrict__ mprec4, const PrimDev* __restrict__ prims,
           const float* __restrict__ pos2d, const float* __restrict__ pos1d, const uchar4* __restrict__ pixPattern,
           float4* __restrict__ samples, float4* __restrict__ hitData, uint2* __restrict__ hitNext,
           uint32_t* __restrict__ hitCtl, uint32_t* __restrict__ hitShards, uint2* __restrict__ hitHeads,
@@ -1015,8 +1015,8 @@ rh_sample(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets
     unsigned long long rowRep = 0ull;
     for (int r = 0; r < BH; ++r) rowRep |= 1ull << (r * BW);
     uint32_t nTest = 0;
-    // wave-uniform counts (ballots): nTest's uniform part and the others
-    uint32_t nTestW = 0, nBound = 0, nHit = 0, nIn = 0, nIn2 = 0;
+    // wave-uniform counts (ballots)
+    uint32_t nBound = 0, nHit = 0, nIn = 0, nIn2 = 0;
     HitArena arena = hit_arena(fr->hitCapacity, hitCtl, hitShards, blockIdx.x + wave * (RH_HIT_SHARDS / RH_S_WAVES));
     const int itemEnd = persistent ? (int)nDevice[0] : itemBase + nStatic;
     // isCullable (bucketprocessor.cpp:1076-1081): occlusion tests and the
@@ -1333,7 +1333,6 @@ rh_sample(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets
         }
     }
     }   // items
-    if (lane == 0) nTest += nTestW;
     // The workgroup's hider counters: wave sums, then one row (summed by
     // rh_reduce_counters; same-address atomics from every wave would
     // serialise in L2).
@@ -2245,7 +2244,7 @@ __global__ void __launch_bounds__(RH_DOF_WAVES * 64)
 rh_sample_dof(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets, const TaskDev* __restrict__ tasks,
               int itemBase, int split, const unsigned long long* __restrict__ capStart,
               const uint32_t* __restrict__ listCount, const uint32_t* __restrict__ lists,
-              const float4* __restrict__ mprec4, const GridDev* __restrict__ grids,
+              const float4* __restrict__ mprec4,
               const PrimDev* __restrict__ prims, const float* __restrict__ pos2d, const float* __restrict__ pos1d,
               const uchar4* __restrict__ pixPattern, const uint8_t* __restrict__ shuffled,
               const float2* __restrict__ lensTab, const uint8_t* __restrict__ pixDof, const float4* __restrict__ cells,
@@ -3608,7 +3607,7 @@ template <int CH, int SLOTS, int STORE = RH_STORE_OCCLUDE, int WPE = 4>
 static void launch_sample_t(hipStream_t st, int grid, const SampleLaunch& a) {
     hipLaunchKernelGGL((rh_sample<CH, SLOTS, STORE, WPE>), dim3(grid), dim3(256), 0, st, a.fr, a.buckets, a.tasks, a.items,
                        a.itemBase, a.nStatic, a.nDevice, a.persistent, a.queueHead, a.capStart, a.listCount, a.lists,
-                       reinterpret_cast<const float4*>(a.mprec), a.grids, a.prims, a.pos2d, a.pos1d, a.pixPattern,
+                       reinterpret_cast<const float4*>(a.mprec), a.prims, a.pos2d, a.pos1d, a.pixPattern,
                        a.samples, a.hitData, a.hitNext, a.hitCtl, a.hitShards, a.hitHeads, a.frontDepth, a.rowCounts,
                        a.rowBase, a.idCut, a.itemCut, a.depthOnly);
 }
@@ -3672,7 +3671,7 @@ extern "C" hipError_t rh_launch_sample_dof(hipStream_t st, const SampleLaunch* a
 #define RH_LAUNCH_DOF(STORE)                                                                                       \
     hipLaunchKernelGGL((rh_sample_dof<STORE>), dim3(ntasks * split), dim3(RH_DOF_WAVES * 64), 0, st, a->fr, a->buckets, \
                        a->tasks, a->itemBase, split, a->capStart, a->listCount, a->lists,                                   \
-                       reinterpret_cast<const float4*>(a->mprec), a->grids, a->prims, a->pos2d, a->pos1d,           \
+                       reinterpret_cast<const float4*>(a->mprec), a->prims, a->pos2d, a->pos1d,                     \
                        a->pixPattern, t->shuffled, t->lens, t->pixDof, t->cells, a->samples, a->hitData, a->hitNext, \
                        a->hitCtl, a->hitShards, a->hitHeads, a->frontDepth, a->rowCounts, a->rowBase, a->idCut, a->itemCut, \
                        a->taskList, a->depthOnly)
