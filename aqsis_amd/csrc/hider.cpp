@@ -274,25 +274,29 @@ private:
     }
 };
 
-// Copy a result from the device, on its context's stream.  A plain copy into
-// pageable memory costs about 15 us and runs at 17 GB/s (one thread copies
-// out of the runtime's staging memory), an asynchronous copy of a piece 30
-// us; so a kernel writes the result into a lane, each workgroup setting a flag
-// behind its part, and up to 8 of the worker pool's threads copy the pieces on as they
-// arrive: 0.26 MB 127 to 33 us, 2.4 MB 141 to 90, 8.3 MB 485 to 280 (30
-// GB/s), 16.8 MB 966 to 460.
+// Copy a result from the device once its context's stream is through (`pending`:
+// it may not be).  A plain copy takes 12 us, 20 to 24 at 0.15 MB, 45 to 55 at
+// 0.69 MB and from there on 17 GB/s (one thread copies out of the runtime's
+// staging memory).  So from 1 MB on a kernel writes the result into a lane,
+// each workgroup setting a flag behind its part, and up to 8 of the worker
+// pool's threads copy the pieces on as they arrive: 0.15 MB 42 us, 0.69 MB 75,
+// 1.3 MB 84 (plain 100), 2.4 MB 102 (157), 8.3 MB 280 (485), 16.8 MB 460 (966).
+// (An asynchronous copy on the stream and a wait for it take 35 us where the
+// plain copy takes 12; behind a kernel that is still to run, 47 against 57 for
+// the wait and the plain copy.)
 // dst may be any host memory; src a context's buffer (read to a multiple of 16 bytes).
-constexpr size_t kReadPlain = 64 << 10;   // bytes below which the plain copy stays
+constexpr size_t kReadPlain = 1 << 20;   // bytes below which the plain copy stays
 // The GPU may be at another context's frame still, and the pool is every
 // context's: a read keeps it for 100 us more than the copy takes at 16 GB/s,
 // waits for data without it and takes it again.  (Taken only once data comes,
 // its threads wake too late: 2.4 MB 39 us longer.)
 constexpr std::chrono::microseconds kPoolHold{100};
 
-hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st) {
+hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st, bool pending = false) {
     ReadLane* lane = bytes >= kReadPlain ? PinnedPool::get().take_lane() : nullptr;
     hipError_t e = hipSuccess;
     if (!lane) {
+        if (!pending) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
         e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
         return e == hipSuccess ? hipStreamSynchronize(st) : e;
     }
@@ -1758,7 +1762,7 @@ static rh_status format_frame(rh_ctx* c, const DisplayFormat& f, int32_t type, c
     }
     HIP_TRY(c->dFormat.ensure(bytes));
     HIP_TRY(rh_launch_format_display(c->st, type, &f, c->dChannels.as<float>(), dither, npix, c->dFormat.p));
-    HIP_TRY(read_back(out, c->dFormat.p, bytes, c->st));
+    HIP_TRY(read_back(out, c->dFormat.p, bytes, c->st, true));
     return RH_OK;
 }
 

@@ -41,7 +41,7 @@ std::map<void*, Block> g_blocks;
 std::map<const void*, std::string> g_kernels;
 size_t g_most = SIZE_MAX;                 // bytes of the largest allocation granted
 std::atomic<uint32_t> g_noRoom{0};        // transparent hits the next frame has no room for
-std::atomic<int> g_deviceSyncs{0}, g_pinnedCalls{0}, g_plainCopies{0}, g_waiting{0};
+std::atomic<int> g_deviceSyncs{0}, g_pinnedCalls{0}, g_plainCopies{0}, g_waiting{0}, g_streamWaits{0};
 
 struct Config { dim3 grid, wg; size_t lds; hipStream_t st; };
 thread_local Config t_config;
@@ -110,6 +110,7 @@ void fake_refuse_pinned(int on) { g_refusePinned = on != 0; }
 int fake_waiting() { return g_waiting; }
 int fake_device_syncs() { return g_deviceSyncs; }
 int fake_pinned_calls() { return g_pinnedCalls; }
+int fake_stream_waits() { return g_streamWaits; }
 int fake_plain_copies() { return g_plainCopies; }
 // bytes held: of a device, or pinned (-1)
 uint64_t fake_held(int dev) {
@@ -199,7 +200,10 @@ hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k) {
     std::memcpy(d, s, n);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
     Stream* n = new Stream();
@@ -208,6 +212,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
+    ++g_streamWaits;
     std::unique_lock<std::mutex> lk(S(s)->m);
     S(s)->idle.wait(lk, [&] { return S(s)->pending == 0; });
     return hipSuccess;

@@ -221,3 +221,19 @@ def test_no_frame_on_an_arena_that_could_not_grow(run):
         h.render()
         again()
     """)
+
+
+def test_small_results_take_one_plain_copy(run):
+    # below 1 MB: no lane, and no wait for a stream that is through
+    run("""
+    for size in ((16, 16), (64, 64), (160, 120)):
+        h = rendered(*size)
+        for read in (h.channels, h.rgba8):
+            copies, waits, pinned = fake.fake_plain_copies(), fake.fake_stream_waits(), fake.fake_held(-1)
+            assert right(read())
+            assert (fake.fake_plain_copies(), fake.fake_stream_waits(), fake.fake_held(-1)) == (copies + 1, waits, pinned)
+        h.close()
+    h = rendered(401, 325)
+    copies = fake.fake_plain_copies()
+    assert right(h.channels()) and fake.fake_plain_copies() == copies
+    """)
