@@ -53,6 +53,11 @@ extern "C" hipError_t rh_launch_box_masks(hipStream_t, const FrameDev*, size_t, 
 extern "C" hipError_t rh_launch_filter(hipStream_t, const FrameDev*, int, int, int, int, int, const float4*,
                                        const uint2*, const FilterDev*, const uchar4*, const float*, const float*,
                                        const float*, float*, uchar4*, int);
+extern "C" size_t rh_filter_tile_lds(int, int, int);
+extern "C" hipError_t rh_launch_sample_boxes(hipStream_t, const FrameDev*, size_t, const uchar4*, const float*, uint16_t*);
+extern "C" hipError_t rh_launch_filter_tiled(hipStream_t, const FrameDev*, int, int, int, int, int, const float4*,
+                                             const uint16_t*, const uchar4*, const float*, const float*, const float*,
+                                             float*, uchar4*, int);
 extern "C" hipError_t rh_launch_cull_pyramid(hipStream_t, const FrameDev*, const CullTreeDev*, int, const float4*, float*);
 extern "C" hipError_t rh_launch_cull_pairs(hipStream_t, const CullTreeDev*, int, int, int, const float4*, const int4*,
                                            const unsigned long long*, int, unsigned long long, const float*, float*);
@@ -401,6 +406,7 @@ struct rh_ctx {
     // frame shape
     DBuf dFrame, dBuckets, dTasks, dPos2d, dPos1d, dPix, dDither, dFilter, dBoxMask;
     DBuf dShuffled, dLens, dPixDof, dDofCells;   // depth of field: lens tables (DofTables)
+    bool tiled = false;                   // the frame shape takes rh_filter_tiled
     // the strip filter's list (FilterDev)
     bool boxVaries = false;
     int filtGroups = 0, filtVary = 0;
@@ -682,6 +688,31 @@ static std::pair<int, int> task_grid(const rh::Shape& s, size_t bucket) {
     return {w, w > 0 ? n / w : 0};
 }
 
+// Whether a frame shape takes the tiled filter.  Strips win wherever the box
+// tests are the same for every pixel (1920x1080, 4x4 samples, width 3: 341 us
+// against 675), and lose where most groups of four samples hold one that varies
+// (even widths with an odd number of samples a side): they and every weight
+// with the pixel's tests, and with few samples a pixel their groups are half
+// padding.  Both sides in us, the frame's counters included, strips first:
+//   width 4, 1x1 samples   46/26 at 160x120   139/86 at 640x480   518/464 at 1920x1080
+//   width 6, 2x1 samples   82/31              223/119             818/659
+//   width 4, 3x3 samples   70/34              233/161             902/920
+//   width 2, 3x3 samples   29/24              99/81               382/439
+//   width 6, 3x3 samples   136/47             391/339             1448/2060 (57 KB of LDS a tile)
+//   width 2, 4x3 samples   28/25              84/88               344/487
+//   width 2, 1x1 samples   25/24              70/76               254/402
+// So by the words a strip's row goes through (groups x pixel rows), by how many
+// of them there are for a term, and by the pixels.
+static bool filter_tiled(const rh::Shape& s, int vary, int groups) {
+    const int cols = 2 * s.shiftX + 1, rows = 2 * s.shiftY + 1, words = groups * rows, taps = cols * rows * s.ns;
+    const size_t lds = rh_filter_tile_lds(s.ns, s.shiftX, s.shiftY);
+    if (!lds || 2 * vary <= groups || words < 24) return false;
+    if (2 * words >= taps) return true;
+    const int64_t pixels = (int64_t)s.width() * s.height();
+    if (4 * words >= taps) return pixels <= (lds <= (48 << 10) ? 1280 * 720 : 640 * 480);
+    return pixels <= 100000;
+}
+
 // The strip filter's lists, from the box tests of the frame shape's sample
 // positions: per filter column an entry for each sample that lies in the box
 // of some pixel there, in sample order, with weight 0 in the rows where its
@@ -763,6 +794,12 @@ static hipError_t filter_lists(rh_ctx* c) {
     c->filtVary = (int)std::count_if(groups.begin(), groups.end(), [](uint32_t g) { return (g >> 31) != 0; });
     fill();
     fill();
+    c->tiled = filter_tiled(s, c->filtVary, c->filtGroups);
+    if (c->tiled) {
+        if ((e = c->dBoxMask.ensure(nsamp * sizeof(uint16_t))) != hipSuccess) return e;
+        return rh_launch_sample_boxes(c->st, c->dFrame.as<FrameDev>(), nsamp, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
+                                      c->dBoxMask.as<uint16_t>());
+    }
     // one device copy: entries, always, groups
     c->filtHost.resize(entries.size() + 2 * always.size() + groups.size());
     c->filtAlwaysAt = entries.size();
@@ -1127,14 +1164,19 @@ static FrameCtl context_ctl(rh_ctx* c) {
 // The filter + expose + quantise stage of a frame.
 static hipError_t enqueue_filter(rh_ctx* c) {
     const rh::Shape& s = c->shape;
+    const int gamma = c->frame.exposureGamma != 1.0f ? 1 : 0;
+    if (c->tiled)
+        return rh_launch_filter_tiled(c->st, c->dFrame.as<FrameDev>(), s.width(), s.height(), s.ns, s.shiftX, s.shiftY,
+                                      c->dSamples.as<float4>(), c->dBoxMask.as<uint16_t>(), c->dPix.as<uchar4>(),
+                                      c->dPos2d.as<float>(), c->dFilter.as<float>(), c->dDither.as<float>(),
+                                      c->dChannels.as<float>(), c->dRgba.as<uchar4>(), gamma);
     const uint32_t* list = c->dFiltList.as<uint32_t>();
     const FilterDev fp{reinterpret_cast<const float*>(list), list + c->filtGroupsAt, c->filtGroups, c->filtVary,
                        reinterpret_cast<const uint2*>(list + c->filtAlwaysAt)};
     return rh_launch_filter(c->st, c->dFrame.as<FrameDev>(), s.width(), s.height(), s.ns, s.shiftX, s.shiftY,
                             c->dSamples.as<float4>(), c->boxVaries ? c->dBoxMask.as<uint2>() : nullptr,
                             &fp, c->dPix.as<uchar4>(), c->dPos2d.as<float>(), c->dFilter.as<float>(),
-                            c->dDither.as<float>(), c->dChannels.as<float>(), c->dRgba.as<uchar4>(),
-                            c->frame.exposureGamma != 1.0f ? 1 : 0);
+                            c->dDither.as<float>(), c->dChannels.as<float>(), c->dRgba.as<uchar4>(), gamma);
 }
 
 // Whether the combine takes its full form: a depth filter other than min, or

@@ -3383,6 +3383,209 @@ __global__ void __launch_bounds__(64) rh_filter_strip(const FrameDev* __restrict
     }
 }
 
+// Tiled filter, for frame shapes where most box tests vary and frames that the
+// strips do not fill the device with (filter_tiled in hider.cpp has the line and
+// both sides' times).  One workgroup per RH_FT x RH_FT tile of display pixels,
+// four waves over the channels: wave 0 sums Ci.r and Ci.g (with the weight
+// total and the count), wave 1 Ci.b and z, wave 2 Oi.r and Oi.g, wave 3
+// Oi.b; each lane one pixel, each sum in the reference's order (filter rows,
+// filter columns, samples), so the split changes no rounding.  The tile's halo
+// of samples is staged in LDS once, with RH_FU coalesced loads in flight per
+// lane, as 8 words per sample: Ci.rgb, z, Oi.rgb and a word holding the sample's
+// box tests (box_tests) and whether it holds a surface (bit 31).  Halo pixel
+// records are 8*ns+RH_FPAD words apart so that the lanes of a wave read
+// different LDS banks.  A strip of one row takes every sample's terms for 2*YM+1
+// pixel rows and keeps one, and its masks are and-ed with each weight; here a
+// term is taken once and its test is a compare of the staged word.  Bound by the
+// latency of the staging and of the LDS reads, four samples at a time.
+#define RH_FT 8
+#define RH_FU 16
+#define RH_FTHREADS 256
+#define RH_FPAD 1
+
+// The weighted sums of one pixel over its filter footprint, in the
+// reference's order (filter rows, filter columns, samples): NC channels
+// starting at `rec0` of each staged sample record (8 words apart), the
+// sample's mask word at offset `mw`.  A sample outside the pixel's box adds
+// nothing, one inside adds its weight to gTot, and one holding a surface also
+// adds weight x value to each channel sum (gTot and count only with TOT).
+// The adds are unconditional with the weight zeroed where the reference
+// skips: x + 0 * v == x exactly, since the sums start at +0 and never become
+// -0 and the values are finite (a tile that staged an infinity or NaN takes
+// its pixels by filter_pixel).  Weights are read with uniform (scalar) loads.
+template <int NC, bool TOT>
+__device__ __forceinline__ void filter_taps(const float* __restrict__ rec0, const float* __restrict__ filterTab,
+                                            int ns, int xm, int ym, int HX, int S, int lx, int ly, int mw,
+                                            float* acc, float& gTot, int& count) {
+    for (int fy = -ym; fy <= ym; ++fy)
+        for (int fx = -xm; fx <= xm; ++fx) {
+            const float* rec = rec0 + ((ly + fy + ym) * HX + (lx + fx + xm)) * S;
+            const float* wt = filterTab + ((fy + ym) * (2 * xm + 1) + fx + xm) * ns;
+            const uint32_t need = (1u << (fx + xm)) | (1u << (8 + fy + ym));
+            // four samples at a time, every LDS read issued first
+            int si = 0;
+            for (; si + 4 <= ns; si += 4) {
+                uint32_t m[4];
+                float d[4][NC];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float* r = rec + (si + q) * 8;
+                    m[q] = __float_as_uint(r[mw]);
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) d[q][c] = r[c];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const bool in = (m[q] & need) == need;
+                    const bool hit = in && (m[q] >> 31);
+                    const float g = wt[si + q];
+                    const float ghit = hit ? g : 0.0f;
+                    if (TOT) {
+                        gTot = gTot + (in ? g : 0.0f);
+                        count += hit ? 1 : 0;
+                    }
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) acc[c] = acc[c] + d[q][c] * ghit;
+                }
+            }
+            for (; si < ns; ++si) {
+                const float* r = rec + si * 8;
+                const uint32_t mm = __float_as_uint(r[mw]);
+                const bool in = (mm & need) == need;
+                const bool hit = in && (mm >> 31);
+                const float g = wt[si];
+                const float ghit = hit ? g : 0.0f;
+                if (TOT) {
+                    gTot = gTot + (in ? g : 0.0f);
+                    count += hit ? 1 : 0;
+                }
+#pragma unroll
+                for (int c = 0; c < NC; ++c) acc[c] = acc[c] + r[c] * ghit;
+            }
+        }
+}
+template <bool GAMMA>
+__global__ void __launch_bounds__(RH_FTHREADS) rh_filter_tiled(const FrameDev* __restrict__ fr,
+                                                       const float4* __restrict__ samples,
+                                                       const uint16_t* __restrict__ boxMask,
+                                                       const uchar4* __restrict__ pixPattern,
+                                                       const float* __restrict__ pos2d,
+                                                       const float* __restrict__ filterTab,
+                                                       const float* __restrict__ dither, float* __restrict__ channels,
+                                                       uchar4* __restrict__ rgba8, int tilesX, int ntiles) {
+    // LDS: halo records (RH_FT+2*xm)*(RH_FT+2*ym)*(8*ns+RH_FPAD) floats; the
+    // tail exchange reuses the first 320 floats.
+    extern __shared__ float lds[];
+    // Workgroups are dealt round-robin to the 8 XCDs; give each XCD a
+    // contiguous run of tiles so neighbouring tiles share halos in its L2.
+    // The grid is a multiple of 8 workgroups.
+    const int per = gridDim.x >> 3;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (tile >= ntiles) return;
+    const int ns = fr->ns, xm = fr->shiftX, ym = fr->shiftY;
+    const int extX0 = fr->extX0, extY0 = fr->extY0, extW = fr->extW, extH = fr->extH;
+    const int tx0 = fr->cropX0 + (tile % tilesX) * RH_FT, ty0 = fr->cropY0 + (tile / tilesX) * RH_FT;
+    const int HX = RH_FT + 2 * xm, HY = RH_FT + 2 * ym, NH = HX * HY;
+    const int S = 8 * ns + RH_FPAD;
+    const int tid = threadIdx.x;
+    bool finite = true;               // no infinity or NaN in what the thread staged
+
+    // 1. Stage the halo's sample records (2 float4 per sample) and masks.
+    {
+        const int per_px = 2 * ns, total = NH * per_px;
+        const int dhp = RH_FTHREADS / per_px, dpart = RH_FTHREADS % per_px;
+        int hp = tid / per_px, part = tid % per_px;
+        int hy = hp / HX, hx = hp % HX;
+        for (int base = 0; base < total; base += RH_FTHREADS * RH_FU) {
+            float4 v[RH_FU];
+            uint32_t mk[RH_FU];
+            int dst[RH_FU];
+#pragma unroll
+            for (int u = 0; u < RH_FU; ++u) {
+                const int i = base + u * RH_FTHREADS + tid;
+                v[u] = make_float4(0.0f, 0.0f, 0.0f, (part & 1) ? __uint_as_float(0xffffffffu) : 0.0f);
+                mk[u] = 0;
+                dst[u] = -1;
+                if (i < total) {
+                    const int qx = tx0 - xm + hx, qy = ty0 - ym + hy;
+                    dst[u] = (hp * S + part * 4) * 2 + (part & 1);
+                    if (qx >= extX0 && qx < extX0 + extW && qy >= extY0 && qy < extY0 + extH) {
+                        const size_t q = (size_t)(qy - extY0) * extW + (qx - extX0);
+                        v[u] = samples[q * per_px + part];
+                        if (part & 1) mk[u] = boxMask[q * ns + (part >> 1)];
+                    }
+                }
+                part += dpart;
+                int adv = dhp;
+                if (part >= per_px) { part -= per_px; ++adv; }
+                hp += adv;
+                hx += adv;
+                while (hx >= HX) { hx -= HX; ++hy; }
+            }
+#pragma unroll
+            for (int u = 0; u < RH_FU; ++u) {
+                if (dst[u] < 0) continue;
+                float* d = lds + (dst[u] >> 1);
+                const float c = (dst[u] & 1) ? 0.0f : v[u].w;
+                finite = finite && fmaf(v[u].x, 0.f, fmaf(v[u].y, 0.f, fmaf(v[u].z, 0.f, c * 0.f))) == 0.f;
+                d[0] = v[u].x;
+                d[1] = v[u].y;
+                d[2] = v[u].z;
+                d[3] = (dst[u] & 1) ? __uint_as_float(mk[u] | ((__float_as_uint(v[u].w) != 0xffffffffu) ? 0x80000000u : 0u))
+                                    : v[u].w;
+            }
+        }
+    }
+    const bool taps = __syncthreads_and(finite);
+    // 2. Weighted sums, one lane per pixel per wave's channels.
+    const int lane = tid & 63, part = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lx = lane & (RH_FT - 1), ly = lane / RH_FT;
+    const int x = tx0 + lx, y = ty0 + ly;
+    const bool valid = x < fr->cropX1 && y < fr->cropY1;
+    float gTot = 0.0f;
+    int count = 0;
+    float acc[2] = {0.0f, 0.0f};
+    if (!taps) {
+        if (part == 0 && valid) filter_pixel<GAMMA>(fr, samples, pixPattern, pos2d, filterTab, dither, channels, rgba8, x, y);
+        return;
+    }
+    if (valid) {
+        // record words: Ci.rgb, z, Oi.rgb, mask
+        if (part == 0) filter_taps<2, true>(lds, filterTab, ns, xm, ym, HX, S, lx, ly, 7, acc, gTot, count);
+        else if (part == 1) filter_taps<2, false>(lds + 2, filterTab, ns, xm, ym, HX, S, lx, ly, 5, acc, gTot, count);
+        else if (part == 2) filter_taps<2, false>(lds + 4, filterTab, ns, xm, ym, HX, S, lx, ly, 3, acc, gTot, count);
+        else filter_taps<1, false>(lds + 6, filterTab, ns, xm, ym, HX, S, lx, ly, 1, acc, gTot, count);
+    }
+    __syncthreads();                  // the halo records are no longer read
+    // waves 1..3 hand their sums to wave 0: Ci.b, z, Oi.r, Oi.g, Oi.b
+    if (part == 1) {
+        lds[lane * 5 + 0] = acc[0];
+        lds[lane * 5 + 1] = acc[1];
+    } else if (part == 2) {
+        lds[lane * 5 + 2] = acc[0];
+        lds[lane * 5 + 3] = acc[1];
+    } else if (part == 3) {
+        lds[lane * 5 + 4] = acc[0];
+    }
+    __syncthreads();
+    if (part == 0 && valid) {
+        const float full[7] = {acc[0], acc[1], lds[lane * 5 + 0], lds[lane * 5 + 2], lds[lane * 5 + 3],
+                               lds[lane * 5 + 4], lds[lane * 5 + 1]};
+        const size_t t = (size_t)(y - fr->cropY0) * (fr->cropX1 - fr->cropX0) + (x - fr->cropX0);
+        finish_pixel<GAMMA>(fr, full, gTot, count, ns, t, dither, channels, rgba8);
+    }
+}
+
+// Each sample's box tests (box_tests), for rh_filter_tiled.
+__global__ void __launch_bounds__(256) rh_sample_boxes(const FrameDev* __restrict__ fr,
+                                                       const uchar4* __restrict__ pixPattern,
+                                                       const float* __restrict__ pos2d, uint16_t* __restrict__ masks) {
+    const int ns = fr->ns;
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (size_t)fr->extW * fr->extH * ns) return;
+    masks[t] = (uint16_t)box_tests(fr, pixPattern, pos2d, t / ns, (int)(t % ns));
+}
+
 // ---------------------------------------------------------------------------
 // Host-side launchers
 // ---------------------------------------------------------------------------
@@ -3801,6 +4004,35 @@ extern "C" hipError_t rh_launch_box_masks(hipStream_t st, const FrameDev* fr, si
     if (nwords == 0) return hipSuccess;
     hipLaunchKernelGGL(rh_box_masks, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, st, fr, pixPattern,
                        pos2d, masks);
+    return hipGetLastError();
+}
+
+// LDS bytes of a workgroup of rh_filter_tiled; 0: it cannot take the frame shape.
+extern "C" size_t rh_filter_tile_lds(int ns, int xm, int ym) {
+    const size_t bytes = (size_t)(RH_FT + 2 * xm) * (RH_FT + 2 * ym) * (8 * ns + RH_FPAD) * sizeof(float);
+    return bytes <= 64 * 1024 ? bytes : 0;
+}
+
+extern "C" hipError_t rh_launch_sample_boxes(hipStream_t st, const FrameDev* fr, size_t nsamples,
+                                             const uchar4* pixPattern, const float* pos2d, uint16_t* masks) {
+    if (nsamples == 0) return hipSuccess;
+    hipLaunchKernelGGL(rh_sample_boxes, dim3((unsigned)((nsamples + 255) / 256)), dim3(256), 0, st, fr, pixPattern,
+                       pos2d, masks);
+    return hipGetLastError();
+}
+
+// masks: the samples' box tests (rh_launch_sample_boxes).
+extern "C" hipError_t rh_launch_filter_tiled(hipStream_t st, const FrameDev* fr, int width, int height, int ns, int xm,
+                                             int ym, const float4* samples, const uint16_t* masks,
+                                             const uchar4* pixPattern, const float* pos2d, const float* filterTab,
+                                             const float* dither, float* channels, uchar4* rgba8, int gamma) {
+    if (width <= 0 || height <= 0) return hipSuccess;
+    const size_t lds = rh_filter_tile_lds(ns, xm, ym);
+    if (!lds || xm > 3 || ym > 3) return hipErrorInvalidValue;
+    const int tilesX = (width + RH_FT - 1) / RH_FT, ntiles = tilesX * ((height + RH_FT - 1) / RH_FT);
+    auto* k = gamma ? &rh_filter_tiled<true> : &rh_filter_tiled<false>;
+    hipLaunchKernelGGL(k, dim3((ntiles + 7) / 8 * 8), dim3(RH_FTHREADS), lds, st, fr, samples, masks, pixPattern, pos2d,
+                       filterTab, dither, channels, rgba8, tilesX, ntiles);
     return hipGetLastError();
 }
 

@@ -61,3 +61,40 @@ def test_infinite_values(oracle, filt, w, k):
     for p in prims[::9]:
         p.Cs[:] = [float("inf"), 1.0, -float("inf")]
     _check(oracle, opts, prims)
+
+
+# Even widths with an odd number of samples a side take 8x8-pixel tiles up to a
+# size: tiles cut by the frame's edge, crop windows, gamma, infinities, and the
+# last frame with tiles beside the first without.
+@pytest.mark.parametrize("res", [(8, 8), (9, 33), (200, 31), (7, 130), (64, 40)])
+@pytest.mark.parametrize("samples,w", [((3, 3), 2.0), ((3, 3), 4.0), ((1, 1), 4.0), ((2, 1), 6.0)])
+def test_tiled_frames(oracle, res, samples, w):
+    print(f"tiles {res} {samples} {w}", flush=True)
+    opts, prims = scenes.patches_scene(seed=9, n=40, res=res, samples=samples, filt=("catmull-rom", w, w), size_px=14.0)
+    for p in prims:
+        p.no_cull_hidden = 1          # a frame of one column of buckets may have no culling schedule
+    _check(oracle, opts, prims)
+
+
+@pytest.mark.parametrize("wx,wy,gamma", [(2.0, 4.0, 1.0), (4.0, 1.0, 2.2), (6.0, 2.5, 2.2), (4.0, 4.0, 1.0)])
+def test_tiled_crops(oracle, wx, wy, gamma):
+    print(f"tiles cropped {wx} {wy} {gamma}", flush=True)
+    opts, prims = scenes.patches_scene(seed=9, n=40, res=(90, 70), samples=(1, 3), filt=("gaussian", wx, wy), size_px=14.0)
+    opts.crop[:] = [0.13, 0.87, 0.21, 0.93]
+    opts.exposure_gamma = gamma
+    _check(oracle, opts, prims)
+
+
+@pytest.mark.parametrize("samples,w", [((3, 3), 2.0), ((1, 1), 4.0)])
+def test_tiled_infinite_values(oracle, samples, w):
+    print(f"tiles infinite colours {samples} {w}", flush=True)
+    opts, prims = scenes.patches_scene(seed=9, n=40, res=(64, 40), samples=samples, filt=("gaussian", w, w), size_px=14.0)
+    for p in prims[::9]:
+        p.Cs[:] = [float("inf"), 1.0, -float("inf")]
+    _check(oracle, opts, prims)
+
+
+@pytest.mark.parametrize("res", [(316, 316), (317, 316)])
+def test_tiled_and_first_without(oracle, res):
+    print(f"tiles up to 100000 pixels {res}", flush=True)
+    _check(oracle, *scenes.patches_scene(seed=9, n=12, res=res, samples=(4, 3), filt=("gaussian", 2.0, 2.0), size_px=60.0))
