@@ -230,7 +230,7 @@ struct DisplayFormat {
 struct FilterDev {
     const float* entries;
     const uint32_t* groups;
-    int ngroups, nvary;                   // nvary: groups with bit 31
+    int ngroups;
     const uint2* always;
 };
 #define RH_FILTER_ENTRY(ym) ((ym) < 2 ? 4 : 8)

@@ -409,7 +409,7 @@ struct rh_ctx {
     bool tiled = false;                   // the frame shape takes rh_filter_tiled
     // the strip filter's list (FilterDev)
     bool boxVaries = false;
-    int filtGroups = 0, filtVary = 0;
+    int filtGroups = 0;
     size_t filtAlwaysAt = 0, filtGroupsAt = 0;   // words into dFiltList
     std::vector<uint32_t> filtHost;
     DBuf dFiltList;
@@ -791,10 +791,10 @@ static hipError_t filter_lists(rh_ctx* c) {
     };
     if (groups.size() % 2) fill();
     c->filtGroups = (int)groups.size();
-    c->filtVary = (int)std::count_if(groups.begin(), groups.end(), [](uint32_t g) { return (g >> 31) != 0; });
+    const int vary = (int)std::count_if(groups.begin(), groups.end(), [](uint32_t g) { return (g >> 31) != 0; });
     fill();
     fill();
-    c->tiled = filter_tiled(s, c->filtVary, c->filtGroups);
+    c->tiled = filter_tiled(s, vary, c->filtGroups);
     if (c->tiled) {
         if ((e = c->dBoxMask.ensure(nsamp * sizeof(uint16_t))) != hipSuccess) return e;
         return rh_launch_sample_boxes(c->st, c->dFrame.as<FrameDev>(), nsamp, c->dPix.as<uchar4>(), c->dPos2d.as<float>(),
@@ -1171,7 +1171,7 @@ static hipError_t enqueue_filter(rh_ctx* c) {
                                       c->dPos2d.as<float>(), c->dFilter.as<float>(), c->dDither.as<float>(),
                                       c->dChannels.as<float>(), c->dRgba.as<uchar4>(), gamma);
     const uint32_t* list = c->dFiltList.as<uint32_t>();
-    const FilterDev fp{reinterpret_cast<const float*>(list), list + c->filtGroupsAt, c->filtGroups, c->filtVary,
+    const FilterDev fp{reinterpret_cast<const float*>(list), list + c->filtGroupsAt, c->filtGroups,
                        reinterpret_cast<const uint2*>(list + c->filtAlwaysAt)};
     return rh_launch_filter(c->st, c->dFrame.as<FrameDev>(), s.width(), s.height(), s.ns, s.shiftX, s.shiftY,
                             c->dSamples.as<float4>(), c->boxVaries ? c->dBoxMask.as<uint2>() : nullptr,

@@ -4043,10 +4043,13 @@ static void launch_filter_t(hipStream_t st, const FrameDev* fr, int width, int h
                             float* channels, uchar4* rgba8, bool gamma) {
     const int tilesX = (width + RH_FS_W - 1) / RH_FS_W;
     // Rows a strip: the halo costs (R + 2*YM) / R, so as many as leave the
-    // device 4096 waves, 16 a CU (512x512, 4x4 samples: 60 us at 4096, 77 at
-    // 2048, 134 at 1024); half of that where most tests vary, as a row costs
-    // more there (317x211, 3x3 samples: 37 us at 4096, 31 at 2048).
-    const size_t waves = 2 * fp.nvary > fp.ngroups ? 2048 : 4096;
+    // device 3700 waves, 14 a CU.  Us at 32, 16, 8 and 4 rows (the waves):
+    //   400x300, 4x4 samples, width 2   129 (500)  84 (950)   60 (1900)  49 (3750); 2 rows 60
+    //   512x512, the same               142 (1024) 92 (2048)  68 (4096)  78 (8192)
+    //   800x600, the same               160 (1900) 110 (3800) 115 (7500) 128
+    //   1280x720, 5x5 samples, width 2  414 (3680) 348 (7200) 338        385
+    //   1600x900, 2x2 samples, width 4  209 (5800) 202        223        289
+    constexpr size_t waves = 3700;
     int R = 32;
     while (R > 1 && (size_t)tilesX * ((height + R - 1) / R) < waves) R >>= 1;
     const int ntiles = tilesX * ((height + R - 1) / R);

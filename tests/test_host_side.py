@@ -185,7 +185,9 @@ def test_estimate_holds_what_a_context_takes(run, samples):
                 h.render()
                 need, said = fake.fake_held(0), hider.estimate(o, [])["device_bytes"]
                 h.close()
-                assert need <= said <= need + need // 20 + (256 << 10), (res, width, bucket, lens, need, said)
+                assert need <= said, (res, width, bucket, lens, need, said)
+                # (the tests' room is kept for frames that take tiles, too)
+                assert varies or said <= need + need // 20 + (256 << 10), (res, width, bucket, lens, need, said)
     """ % samples)
 
 
