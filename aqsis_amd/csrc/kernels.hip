@@ -983,18 +983,23 @@ __device__ __forceinline__ uint32_t hit_entry(HitArena& a, unsigned long long am
 // *nDevice).  Each workgroup writes one row of counters at rowBase +
 // blockIdx.x.  STORE selects StoreSample's mode (RH_STORE_*): the usual
 // occluding hit, the midpoint store, or every hit listed (not cullable).
+// (rowCounts stands among the read parameters: the compiler loads neighbouring
+// parameters together, and with the ones after it moved up it held more of them at
+// once and read 335 scalars back from lanes instead of 269: 2048x2048 clustered
+// 5928 us against 5888.)
 template <int CH, int SLOTS, int STORE = RH_STORE_OCCLUDE, int WPE = 4>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 rh_sample(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets, const TaskDev* __restrict__ tasks,
           const uint2* __restrict__ items, int itemBase, int nStatic, const uint32_t* __restrict__ nDevice,
           int persistent, uint32_t* __restrict__ queueHead, const unsigned long long* __restrict__ capStart,
           const uint32_t* __restrict__ listCount, const uint32_t* __restrict__ lists,
-          const float4* __restrict__ mprec4, const PrimDev* __restrict__ prims,
+          const float4* __restrict__ mprec4, uint32_t* __restrict__ rowCounts,
+          const PrimDev* __restrict__ prims,
           const float* __restrict__ pos2d, const float* __restrict__ pos1d, const uchar4* __restrict__ pixPattern,
           float4* __restrict__ samples, float4* __restrict__ hitData, uint2* __restrict__ hitNext,
           uint32_t* __restrict__ hitCtl, uint32_t* __restrict__ hitShards, uint2* __restrict__ hitHeads,
           float* __restrict__ frontDepth,
-          uint32_t* __restrict__ rowCounts, int rowBase, uint32_t idCut, const uint32_t* __restrict__ itemCut,
+          int rowBase, uint32_t idCut, const uint32_t* __restrict__ itemCut,
           int depthOnly) {
     __shared__ float4 recs[CH * 9];
     __shared__ uint32_t wsum[RH_S_WAVES][5];
@@ -3810,8 +3815,8 @@ template <int CH, int SLOTS, int STORE = RH_STORE_OCCLUDE, int WPE = 4>
 static void launch_sample_t(hipStream_t st, int grid, const SampleLaunch& a) {
     hipLaunchKernelGGL((rh_sample<CH, SLOTS, STORE, WPE>), dim3(grid), dim3(256), 0, st, a.fr, a.buckets, a.tasks, a.items,
                        a.itemBase, a.nStatic, a.nDevice, a.persistent, a.queueHead, a.capStart, a.listCount, a.lists,
-                       reinterpret_cast<const float4*>(a.mprec), a.prims, a.pos2d, a.pos1d, a.pixPattern,
-                       a.samples, a.hitData, a.hitNext, a.hitCtl, a.hitShards, a.hitHeads, a.frontDepth, a.rowCounts,
+                       reinterpret_cast<const float4*>(a.mprec), a.rowCounts, a.prims, a.pos2d, a.pos1d, a.pixPattern,
+                       a.samples, a.hitData, a.hitNext, a.hitCtl, a.hitShards, a.hitHeads, a.frontDepth,
                        a.rowBase, a.idCut, a.itemCut, a.depthOnly);
 }
 
