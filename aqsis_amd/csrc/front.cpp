@@ -311,20 +311,32 @@ bool make_shape(const rh_options& o, Shape& s, std::string& err) {
     // samples: 258 to 184 us at 637x475, 1098 to 921 at 1920x1080; 2x2-pixel
     // blocks gain 0 to 10% in the sampler and lose more in binning).  The
     // motion sampler runs one workgroup a task and keeps the larger tasks.
-    // The lens sampler's blocks are 8x8 pixels (a lane a pixel), so its tasks
-    // are too (tasks of 16x4 pixels left half its lanes without a pixel, of
-    // 4x4 three quarters).  Both up to 16,384 buckets, and only where the frame
-    // then still has no more tasks than the no-allocation form holds counters
-    // for: a bucket has up to 16, so 3840x3840 at 2x2 samples in 32x32-pixel
-    // buckets would have 230,400 instead of 57,600.
+    // The lens sampler's blocks are 8x8 pixels (a lane a pixel) for each sample
+    // of a pixel, so its tasks are 8x8 pixels too (tasks of 16x4 pixels left half
+    // its lanes without a pixel, of 4x4 three quarters); with 1 or 2 samples a
+    // workgroup's four waves share one staged list over 2 or 4 tiles where the
+    // frame still has a workgroup for most places on the device: 1x1 samples, 8x8,
+    // 16x8 and 16x16 pixels, 600 and 3000 surfaces: 2483 2006 2677 and 4537 3336
+    // 4914 us at 440x330 (2310 tiles), 2318 1533 1164 and 4604 2950 2180 at
+    // 1280x720; 2x1 samples 2317 2151 3654 and 2194 1570 1874.
+    // Both up to 16,384 buckets, and only where the frame then still has no more
+    // tasks than the no-allocation form holds counters for: a bucket has up to
+    // 16, so 3840x3840 at 2x2 samples in 32x32-pixel buckets would have 230,400
+    // instead of 57,600.
     bool fine = s.buckets.size() <= 16384;
-    auto parts = [&](int bucket, int block) {
+    int lensX = 8, lensY = 8;
+    auto parts = [&](int bucket, int block, int lens) {
         const bool wide = fine && o.shutter_open == o.shutter_close;
-        const int side = s.dof && fine ? 8 : (wide ? std::max(2 * block, std::min(8, 4 * block)) : 4 * block);
+        const int side = s.dof && fine ? lens : (wide ? std::max(2 * block, std::min(8, 4 * block)) : 4 * block);
         return std::max(1, std::min(4, bucket / side));
     };
-    if (s.buckets.size() * (size_t)(parts(o.bucket_x, s.blockW) * parts(o.bucket_y, s.blockH)) > kNoallocRows) fine = false;
-    const int ntx = parts(o.bucket_x, s.blockW), nty = parts(o.bucket_y, s.blockH);
+    auto count = [&](int lx, int ly) {
+        return s.buckets.size() * (size_t)(parts(o.bucket_x, s.blockW, lx) * parts(o.bucket_y, s.blockH, ly));
+    };
+    if (s.ns <= 2 && count(16, 8) >= 1024) lensX = 16;
+    if (s.ns == 1 && count(16, 16) >= 1024) lensY = 16;
+    if (count(lensX, lensY) > kNoallocRows) fine = false;
+    const int ntx = parts(o.bucket_x, s.blockW, lensX), nty = parts(o.bucket_y, s.blockH, lensY);
     s.tasks.clear();
     s.taskStart.assign(1, 0);
     for (size_t k = 0; k < s.buckets.size(); ++k) {
