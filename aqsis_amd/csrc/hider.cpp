@@ -25,7 +25,7 @@
 
 extern "C" hipError_t rh_launch_dice(hipStream_t, const FrameDev*, const GridDev*, int, const PrimDev*,
                                      const float*, float*, float4*, float4*, const FrameClear*);
-extern "C" hipError_t rh_launch_sample_mb(hipStream_t, const SampleLaunch*, int, const float4*);
+extern "C" hipError_t rh_launch_sample_mb(hipStream_t, const SampleLaunch*, int, const float4*, int);
 extern "C" hipError_t rh_launch_bin(hipStream_t, const FrameDev*, const BucketDev*, int, const TaskDev*,
                                     const GridDev*, const uint32_t*, const uint32_t*, const uint32_t*, size_t,
                                     const unsigned long long*, const float4*, uint32_t*, unsigned long long*, uint32_t*,
@@ -1191,6 +1191,12 @@ static int store_mode(const FrameDev& f) {
     return f.midpointStore ? RH_STORE_MIDPOINT : RH_STORE_OCCLUDE;
 }
 
+// Whether the motion sampler's chunks hold fewer records and more sub-bounds
+// (RH_MB_CLOSED_PAIRS): a closed shutter at more than 4 samples a pixel.
+static int mb_many_pairs(const rh_ctx* c) {
+    return (c->frame.shutterOpen == c->frame.shutterClose && c->shape.ns > 4) ? 1 : 0;
+}
+
 // The micropolygon records the combine finds an occluding hit's grid in:
 // the motion records in a frame with moving micropolygons; null when no
 // surface is a matte (the combine then looks up no surface for it).
@@ -1246,7 +1252,7 @@ static hipError_t enqueue_frame(rh_ctx* c, bool timed, const FrameCtl& k, bool g
     if (S.motion) {
         // Frames with moving micropolygons take the motion form of the
         // sampler, whatever the layout.
-        ENQ(rh_launch_sample_mb(c->st, &a, nt, c->dMprecMB.as<float4>()));
+        ENQ(rh_launch_sample_mb(c->st, &a, nt, c->dMprecMB.as<float4>(), mb_many_pairs(c)));
         rows = nt;
     } else if (s.dof) {
         // Depth of field: the lens form of the sampler, whatever the layout.
@@ -1366,7 +1372,7 @@ static hipError_t enqueue_depth_pass(rh_ctx* c, bool sample) {
     if (!sample) return hipSuccess;
     SampleLaunch a = depth_launch(c);
     const int nt = (int)s.tasks.size();
-    if (S.motion) return rh_launch_sample_mb(c->st, &a, nt, c->dMprecMB.as<float4>());
+    if (S.motion) return rh_launch_sample_mb(c->st, &a, nt, c->dMprecMB.as<float4>(), mb_many_pairs(c));
     if (s.dof) {
         const DofTables dt = c->dof();
         return rh_launch_sample_dof(c->st, &a, nt, c->dofSplit, &dt);
@@ -1490,7 +1496,7 @@ static rh_status cull_schedule(rh_ctx* c, const rh::Forest& forest) {
                 a.itemCut = c->dProbeCut.as<uint32_t>();
                 a.taskList = c->dProbeTasks.as<uint32_t>();
                 if (c->sched.motion) {
-                    HIP_TRY(rh_launch_sample_mb(c->st, &a, ni, c->dMprecMB.as<float4>()));
+                    HIP_TRY(rh_launch_sample_mb(c->st, &a, ni, c->dMprecMB.as<float4>(), mb_many_pairs(c)));
                 } else if (s.dof) {
                     const DofTables dt = c->dof();
                     HIP_TRY(rh_launch_sample_dof(c->st, &a, ni, 1, &dt));

@@ -1477,8 +1477,16 @@ __device__ __forceinline__ MBHit quad_hit(const f3d p0, const f3d p1, const f3d 
 // 608 6460 (two workgroups a CU of 8 waves, 192 and 192: 6710).  With a part
 // of padding a record, which takes the lanes' reads of one part of different
 // records off the same banks, 320 and 784 6200, 256 and 1104 6430.
+// With a closed shutter a record's sub-bounds are all at one time and all taken,
+// up to 64 at 64 samples, so there a chunk holds fewer records and more pairs
+// from 5 samples on: 320x320, 300 patches, 16-pixel buckets, 320 and 784 against
+// 128 and 1744: 1062 and 1159 us at 2x2 samples, 7038 and 5567 at 4x4, 15058 and
+// 13461 at 8x8 (64-pixel buckets 52821 and 38920); an open shutter 1951 and 2378
+// at 4x4.
 #define RH_MB_RECS 320
 #define RH_MB_PAIRS 784
+#define RH_MB_CLOSED_RECS 128
+#define RH_MB_CLOSED_PAIRS 1744
 #define RH_MB_STRIDE 9      // float4s of a staged record: one more than it has, off the same banks
 #define RH_MB_RING 128     // visits and results held per wave
 #define RH_MB_STATIC 0xfe00u
@@ -1556,7 +1564,7 @@ __device__ __forceinline__ unsigned long long transpose64(unsigned long long row
     return row;
 }
 
-template <int NW, int STORE>
+template <int NW, int STORE, int RECS, int PAIRS>
 __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __restrict__ fr,
                                                         const BucketDev* __restrict__ buckets,
                                                         const TaskDev* __restrict__ tasks, int ntasks,
@@ -1575,20 +1583,20 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
                                                         uint32_t* __restrict__ rowCounts, int rowBase, int taskBase,
                                                         uint32_t idCut, const uint32_t* __restrict__ itemCut,
                                                         const uint32_t* __restrict__ taskList, int depthOnly) {
-    __shared__ float4 recs[RH_MB_RECS * RH_MB_STRIDE];
-    __shared__ float kbs[RH_MB_RECS][12];          // key bounds, kb[k][c] at [k * 6 + c]
+    __shared__ float4 recs[RECS * RH_MB_STRIDE];
+    __shared__ float kbs[RECS][12];          // key bounds, kb[k][c] at [k * 6 + c]
     // sub-bounds | first taken << 8 | the first of all taken too << 16 | number taken << 24
-    __shared__ uint32_t divs[RH_MB_RECS];
+    __shared__ uint32_t divs[RECS];
     // per number of sub-bounds d their time step, and their end times from d (d - 1) / 2 on
     __shared__ float dts[RH_MB_DIVS + 1], times[RH_MB_DIVS * (RH_MB_DIVS + 1) / 2];
-    __shared__ int offs[RH_MB_RECS + 1];
-    __shared__ uint32_t ids[RH_MB_RECS];
+    __shared__ int offs[RECS + 1];
+    __shared__ uint32_t ids[RECS];
     // entries: (record | sub-bound << 9 (RH_MB_STATIC: static) | index window << 16,
     // sub-sample x range, y range (lo | hi << 16), min z); the bound
     // (min x, max x, min y, max y); the times (time0, time1)
-    __shared__ uint4 E0[RH_MB_PAIRS];
-    __shared__ float4 E1[RH_MB_PAIRS];
-    __shared__ float2 E2[RH_MB_PAIRS];
+    __shared__ uint4 E0[PAIRS];
+    __shared__ float4 E1[PAIRS];
+    __shared__ float2 E2[PAIRS];
     __shared__ uint16_t buf[NW][128];
     __shared__ float4 smp[NW][64];                 // the block's samples: x, y, time, LOD test
     __shared__ unsigned long long winLanes[65];
@@ -1680,7 +1688,7 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
         smp[wave][lane] = make_float4(sx, sy, stime, lodOk ? 1.0f : 0.0f);
 
         for (uint32_t c0 = 0; c0 < n;) {
-            const int cnt = (int)((n - c0) < (uint32_t)RH_MB_RECS ? (n - c0) : (uint32_t)RH_MB_RECS);
+            const int cnt = (int)((n - c0) < (uint32_t)RECS ? (n - c0) : (uint32_t)RECS);
             __syncthreads();
             for (int q = tid; q < cnt * 8; q += NW * 64) {
                 const uint32_t id = L[c0 + q / 8];
@@ -1716,7 +1724,7 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
             __syncthreads();
             // pair offsets, and the records whose pairs fit in one pass
             if (wave == 0) {
-                constexpr int PER = RH_MB_RECS / 64;
+                constexpr int PER = RECS / 64;
                 int dk[PER], incl = 0;
 #pragma unroll
                 for (int j = 0; j < PER; ++j) {
@@ -1734,9 +1742,9 @@ __global__ void __launch_bounds__(NW * 64, 4) rh_sample_mb(const FrameDev* __res
                 for (int j = 0; j < PER; ++j) {
                     offs[PER * lane + j] = run;
                     run += dk[j];
-                    fit += (PER * lane + j < cnt && run <= RH_MB_PAIRS) ? 1 : 0;
+                    fit += (PER * lane + j < cnt && run <= PAIRS) ? 1 : 0;
                 }
-                if (lane == 63) offs[RH_MB_RECS] = incl;
+                if (lane == 63) offs[RECS] = incl;
                 for (int off = 32; off > 0; off >>= 1) fit += __shfl_xor(fit, off);
                 if (lane == 0) nfitShared = fit;
             }
@@ -3851,10 +3859,13 @@ extern "C" hipError_t rh_launch_sample(hipStream_t st, int variant, int grid, co
 #define RH_MB_WAVES 16
 #endif
 extern "C" hipError_t rh_launch_sample_mb(hipStream_t st, const SampleLaunch* a, int ntasks,
-                                          const float4* mprecMB) {
+                                          const float4* mprecMB, int manyPairs) {
     if (ntasks <= 0) return hipSuccess;
 #define RH_LAUNCH_MB(STORE)                                                                                          \
-    hipLaunchKernelGGL((rh_sample_mb<RH_MB_WAVES, STORE>), dim3(ntasks), dim3(RH_MB_WAVES * 64), 0, st, a->fr,        \
+    if (manyPairs) RH_LAUNCH_MB_AS(STORE, RH_MB_CLOSED_RECS, RH_MB_CLOSED_PAIRS);                                     \
+    else RH_LAUNCH_MB_AS(STORE, RH_MB_RECS, RH_MB_PAIRS)
+#define RH_LAUNCH_MB_AS(STORE, RECS, PAIRS)                                                                          \
+    hipLaunchKernelGGL((rh_sample_mb<RH_MB_WAVES, STORE, RECS, PAIRS>), dim3(ntasks), dim3(RH_MB_WAVES * 64), 0, st, a->fr,        \
                        a->buckets, a->tasks, a->itemBase + ntasks, a->capStart, a->listCount, a->lists, mprecMB,       \
                        a->grids, a->prims, a->pos2d, a->pos1d, a->pixPattern, a->samples, a->hitData, a->hitNext,     \
                        a->hitCtl, a->hitShards, a->hitHeads, a->frontDepth, a->rowCounts, a->rowBase, a->itemBase, a->idCut, \
@@ -3866,6 +3877,7 @@ extern "C" hipError_t rh_launch_sample_mb(hipStream_t st, const SampleLaunch* a,
     default: return hipErrorInvalidValue;
     }
 #undef RH_LAUNCH_MB
+#undef RH_LAUNCH_MB_AS
     return hipGetLastError();
 }
 

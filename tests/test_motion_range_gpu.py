@@ -41,3 +41,35 @@ def test_sub_bounds(oracle, k, shutter, keys):
     assert np.array_equal(ch.view(np.uint32), ref["channels"].view(np.uint32))
     for key in ("spl_count", "spl_bound_hits", "spl_hits"):
         assert st[key] == ref["stats"][key], key
+
+
+# A closed shutter takes every sub-bound, from 5 samples on in chunks of fewer
+# records and more pairs: both sides of that line, more records (still ones, of
+# one pair) and more pairs (moving ones) than a chunk holds, and neither.
+@pytest.mark.parametrize("n,bucket", [(4, 16), (40, 64)])
+@pytest.mark.parametrize("k,still", [((2, 2), 2), ((5, 1), 2), ((3, 3), 1), ((4, 4), 9), ((8, 8), 3)])
+def test_closed_shutter_chunks(oracle, k, still, n, bucket):
+    from aqsis_amd.hider import Hider
+    print(f"closed shutter {k} still {still} surfaces {n}", flush=True)
+    opts, prims = scenes.motion_scene(seed=5, n=n, res=(70, 66), size_px=24.0, samples=k, shift_sigma=0.3,
+                                      shutter=(0.3, 0.3), key_times=(0.0, 1.0), shading_rate=0.5)
+    opts.bucket_x = opts.bucket_y = bucket
+    for i, p in enumerate(prims):
+        if i % still == 0:
+            p.nkeys = 1
+        if i % 4 == 0:
+            p.Os[:] = [1.0, 1.0, 1.0]
+    prims[-1].nkeys = 2
+    ref = oracle.render(opts, prims, occlusion_cull=True)
+    with Hider(opts) as h:
+        h.post_surfaces(prims)
+        h.render()
+        ids, depth, rgbaz = h.samples()
+        st = h.stats()
+        ch = h.channels()
+    assert np.array_equal(ids, ref["mp_id"])
+    assert np.array_equal(depth.view(np.uint32), ref["depth"].view(np.uint32))
+    assert np.array_equal(rgbaz.view(np.uint32), ref["rgbaz"].view(np.uint32))
+    assert np.array_equal(ch.view(np.uint32), ref["channels"].view(np.uint32))
+    for key in ("spl_count", "spl_bound_hits", "spl_hits"):
+        assert st[key] == ref["stats"][key], key
