@@ -4060,15 +4060,17 @@ static void launch_filter_t(hipStream_t st, const FrameDev* fr, int width, int h
                             float* channels, uchar4* rgba8, bool gamma) {
     const int tilesX = (width + RH_FS_W - 1) / RH_FS_W;
     // Rows a strip: the halo costs (R + 2*YM) / R, so as many as leave the
-    // device 3700 waves, 14 a CU.  Us at 32, 16, 8 and 4 rows (the waves):
-    //   400x300, 4x4 samples, width 2   129 (500)  84 (950)   60 (1900)  49 (3750); 2 rows 60
-    //   512x512, the same               142 (1024) 92 (2048)  68 (4096)  78 (8192)
-    //   800x600, the same               160 (1900) 110 (3800) 115 (7500) 128
-    //   1280x720, 5x5 samples, width 2  414 (3680) 348 (7200) 338        385
-    //   1600x900, 2x2 samples, width 4  209 (5800) 202        223        289
-    constexpr size_t waves = 3700;
-    int R = 32;
-    while (R > 1 && (size_t)tilesX * ((height + R - 1) / R) < waves) R >>= 1;
+    // device 3700 waves, 14 a CU, and more than 16 only where 8000 are left.  Us
+    // at 32, 16, 8 and 4 rows (the waves):
+    //   400x300, 4x4 samples, width 2    129 (500)  84 (950)    60 (1900)  49 (3750); 2 rows 60
+    //   512x512, the same                142 (1024) 92 (2048)   68 (4096)  78 (8192)
+    //   800x600, the same                160 (1900) 110 (3800)  115 (7500) 128
+    //   1280x720, 5x5 samples, width 2   414 (3680) 348 (7200)  338        385
+    //   1600x900, the same               548 (5800) 500 (11400) 506        581
+    //   1920x1080, 3x3 samples, width 2  367 (8160) 372 (16320) 398        478
+    const auto waves = [&](int rows) { return (size_t)tilesX * ((height + rows - 1) / rows); };
+    int R = waves(32) >= 8000 ? 32 : 16;
+    while (R > 1 && waves(R) < 3700) R >>= 1;
     const int ntiles = tilesX * ((height + R - 1) / R);
     const size_t HX = RH_FS_W + 2 * xm, total = HX * ns;
     const size_t lds = (HX * 8 * (ns | 1) + 64 * RH_FS_OUT) * sizeof(float) + ((total / 32 + 4) & ~size_t(1)) * 4 +
