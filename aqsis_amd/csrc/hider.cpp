@@ -280,17 +280,21 @@ private:
 };
 
 // Copy a result from the device once its context's stream is through (`pending`:
-// it may not be).  A plain copy takes 12 us, 20 to 24 at 0.15 MB, 45 to 55 at
-// 0.69 MB and from there on 17 GB/s (one thread copies out of the runtime's
-// staging memory).  So from 1 MB on a kernel writes the result into a lane,
-// each workgroup setting a flag behind its part, and up to 8 of the worker
-// pool's threads copy the pieces on as they arrive: 0.15 MB 42 us, 0.69 MB 75,
-// 1.3 MB 84 (plain 100), 2.4 MB 102 (157), 8.3 MB 280 (485), 16.8 MB 460 (966).
-// (An asynchronous copy on the stream and a wait for it take 35 us where the
-// plain copy takes 12; behind a kernel that is still to run, 47 against 57 for
-// the wait and the plain copy.)
+// it may not be).  A plain copy into pageable memory takes 12 us, 24 at 37 KB, 15
+// to 69 at 147 KB and 20 to 265 at 0.27 MB (from 64 KB on the runtime pins the
+// caller's pages, and what that costs is up to how they are mapped), and from 1 MB
+// on runs at 17 GB/s (one thread copies out of the runtime's staging memory).  So
+// results go by way of a lane: copied there and on by the calling thread up to
+// 1.5 MB (16 us at 147 KB, 21 at 0.27 MB, 38 at 0.69, 79 at 1.3 and 122 at 2.4),
+// above by a kernel that writes into the lane, each workgroup setting a flag
+// behind its part, while up to 8 of the worker pool's threads copy the pieces on
+// (0.15 MB 42 us, 0.69 75, 1.3 84, 2.4 102, 8.3 280, 16.8 460; plain 157, 485 and
+// 966).  (An asynchronous copy on the stream and a wait for it take 35 us where
+// the plain copy takes 12, so that is for results still to be computed.)
 // dst may be any host memory; src a context's buffer (read to a multiple of 16 bytes).
-constexpr size_t kReadPlain = 1 << 20;   // bytes below which the plain copy stays
+constexpr size_t kReadPlain = 16 << 10;     // bytes of a result at hand below which nothing is gained by a lane
+constexpr size_t kReadShared = 1536 << 10;  // bytes from which the pool's threads take part
+
 // The GPU may be at another context's frame still, and the pool is every
 // context's: a read keeps it for 100 us more than the copy takes at 16 GB/s,
 // waits for data without it and takes it again.  (Taken only once data comes,
@@ -298,12 +302,20 @@ constexpr size_t kReadPlain = 1 << 20;   // bytes below which the plain copy sta
 constexpr std::chrono::microseconds kPoolHold{100};
 
 hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st, bool pending = false) {
-    ReadLane* lane = bytes >= kReadPlain ? PinnedPool::get().take_lane() : nullptr;
+    ReadLane* lane = bytes >= kReadPlain || pending ? PinnedPool::get().take_lane() : nullptr;
     hipError_t e = hipSuccess;
-    if (!lane) {
-        if (!pending) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
-        e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
-        return e == hipSuccess ? hipStreamSynchronize(st) : e;
+    if (!lane || bytes < kReadShared) {
+        void* to = lane ? lane->p : dst;
+        if (pending) {
+            e = hipMemcpyAsync(to, src, bytes, hipMemcpyDeviceToHost, st);
+            if (e == hipSuccess) e = hipStreamSynchronize(st);
+        } else {
+            e = hipMemcpy(to, src, bytes, hipMemcpyDeviceToHost);
+        }
+        if (!lane) return e;
+        if (e == hipSuccess) std::memcpy(dst, lane->p, bytes);
+        PinnedPool::get().give_lane(lane);
+        return e;
     }
     for (size_t from = 0; from < bytes && e == hipSuccess; from += kLaneBytes) {
         const size_t len = std::min(kLaneBytes, bytes - from);
@@ -346,7 +358,9 @@ hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st, b
             const size_t at = (size_t)i * piece, end = std::min(at + piece, len);
             uint32_t spin = 0;
             for (size_t w = missing(at / RH_READ_WG_BYTES, end); w != SIZE_MAX; w = missing(w, end)) {
-                if ((++spin & 0x3f) == 0 && Clock::now() > until) return;
+                // (asking the stream now and then makes its end cheap to wait for:
+                // 9.4 MB 295 us without, 279 so)
+                if ((++spin & 0xfff) == 0 && ((void)hipStreamQuery(st), Clock::now() > until)) return;
                 __builtin_ia32_pause();
             }
             copy(i);

@@ -41,7 +41,7 @@ std::map<void*, Block> g_blocks;
 std::map<const void*, std::string> g_kernels;
 size_t g_most = SIZE_MAX;                 // bytes of the largest allocation granted
 std::atomic<uint32_t> g_noRoom{0};        // transparent hits the next frame has no room for
-std::atomic<int> g_deviceSyncs{0}, g_pinnedCalls{0}, g_plainCopies{0}, g_waiting{0}, g_streamWaits{0};
+std::atomic<int> g_deviceSyncs{0}, g_pinnedCalls{0}, g_plainCopies{0}, g_waiting{0}, g_streamWaits{0}, g_pinnedCopies{0};
 
 struct Config { dim3 grid, wg; size_t lds; hipStream_t st; };
 thread_local Config t_config;
@@ -111,6 +111,7 @@ int fake_waiting() { return g_waiting; }
 int fake_device_syncs() { return g_deviceSyncs; }
 int fake_pinned_calls() { return g_pinnedCalls; }
 int fake_stream_waits() { return g_streamWaits; }
+int fake_pinned_copies() { return g_pinnedCopies; }
 int fake_plain_copies() { return g_plainCopies; }
 // bytes held: of a device, or pinned (-1)
 uint64_t fake_held(int dev) {
@@ -196,7 +197,12 @@ hipError_t hipGetSymbolAddress(void** p, const void*) {
 }
 hipError_t hipMemset(void* p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k) {
-    if (k == hipMemcpyDeviceToHost) ++g_plainCopies;
+    if (k == hipMemcpyDeviceToHost) {
+        ++g_plainCopies;
+        std::lock_guard<std::mutex> lk(g_m);
+        auto b = g_blocks.upper_bound(d);
+        if (b != g_blocks.begin() && (--b)->second.dev < 0 && static_cast<char*>(b->first) + b->second.bytes > d) ++g_pinnedCopies;
+    }
     std::memcpy(d, s, n);
     return hipSuccess;
 }

@@ -225,15 +225,18 @@ def test_no_frame_on_an_arena_that_could_not_grow(run):
     """)
 
 
-def test_small_results_take_one_plain_copy(run):
-    # below 1 MB: no lane, and no wait for a stream that is through
+def test_small_results_take_one_copy(run):
+    # up to 1.5 MB one blocking copy, from 16 KB on into pinned memory, and no wait
+    # for a stream that is through; larger results by the kernel
     run("""
-    for size in ((16, 16), (64, 64), (160, 120)):
+    for size in ((16, 16), (48, 44), (64, 64), (160, 120)):
         h = rendered(*size)
         for read in (h.channels, h.rgba8):
-            copies, waits, pinned = fake.fake_plain_copies(), fake.fake_stream_waits(), fake.fake_held(-1)
-            assert right(read())
-            assert (fake.fake_plain_copies(), fake.fake_stream_waits(), fake.fake_held(-1)) == (copies + 1, waits, pinned)
+            copies, waits, inLane = fake.fake_plain_copies(), fake.fake_stream_waits(), fake.fake_pinned_copies()
+            out = read()
+            assert right(out)
+            assert (fake.fake_plain_copies(), fake.fake_stream_waits()) == (copies + 1, waits)
+            assert fake.fake_pinned_copies() == inLane + (1 if out.nbytes >= 16384 else 0), out.nbytes
         h.close()
     h = rendered(401, 325)
     copies = fake.fake_plain_copies()
