@@ -702,29 +702,36 @@ static std::pair<int, int> task_grid(const rh::Shape& s, size_t bucket) {
     return {w, w > 0 ? n / w : 0};
 }
 
-// Whether a frame shape takes the tiled filter.  Strips win wherever the box
-// tests are the same for every pixel (1920x1080, 4x4 samples, width 3: 341 us
-// against 675), and lose where most groups of four samples hold one that varies
-// (even widths with an odd number of samples a side): they and every weight
-// with the pixel's tests, and with few samples a pixel their groups are half
-// padding.  Both sides in us, the frame's counters included, strips first:
+// Whether a frame shape takes the tiled filter.  Strips win on large frames
+// whose box tests are the same for every pixel (1920x1080, 4x4 samples, width 3:
+// 341 us against 675).  They lose where some test varies (an even width and an
+// odd number of samples a side, or rounding): then a pixel's tests are read with
+// its samples and and-ed with the weights of each group of four that holds such
+// a sample; and with few samples a pixel, whose groups are half padding.  Both
+// sides in us, the frame's counters included, strips first:
 //   width 4, 1x1 samples   46/26 at 160x120   139/86 at 640x480   518/464 at 1920x1080
 //   width 6, 2x1 samples   82/31              223/119             818/659
+//   width 6, 1x4 samples   71/32              192/121             690/698
 //   width 4, 3x3 samples   70/34              233/161             902/920
 //   width 2, 3x3 samples   29/24              99/81               382/439
-//   width 6, 3x3 samples   136/47             391/339             1448/2060 (57 KB of LDS a tile)
+//   width 6, 3x3 samples   136/47             391/339             1448/2060 (57 KB of LDS a tile; 642/640 at 900x675)
 //   width 2, 4x3 samples   28/25              84/88               344/487
 //   width 2, 1x1 samples   25/24              70/76               254/402
+// and where no test varies
+//   width 5, 1x1 samples   30/25              76/80               249/438
+//   width 4, 2x2 samples   29/25              77/88               261/483 (45/38 at 317x211, 22/27 at 33x29)
+//   width 2, 2x2 samples   20/21              46/63               153/328
 // So by the words a strip's row goes through (groups x pixel rows), by how many
 // of them there are for a term, and by the pixels.
 static bool filter_tiled(const rh::Shape& s, int vary, int groups) {
     const int cols = 2 * s.shiftX + 1, rows = 2 * s.shiftY + 1, words = groups * rows, taps = cols * rows * s.ns;
     const size_t lds = rh_filter_tile_lds(s.ns, s.shiftX, s.shiftY);
-    if (!lds || 2 * vary <= groups || words < 24) return false;
-    if (2 * words >= taps) return true;
     const int64_t pixels = (int64_t)s.width() * s.height();
-    if (4 * words >= taps) return pixels <= (lds <= (48 << 10) ? 1280 * 720 : 640 * 480);
-    return pixels <= 100000;
+    if (!lds || words < 24) return false;
+    if (vary == 0) return 4 * words >= taps && pixels > 8192 && pixels <= 150000;
+    if (2 * words >= taps) return true;
+    if (4 * words >= taps) return pixels <= (lds <= (48 << 10) ? 1280 * 720 : 550000);
+    return 2 * vary > groups && pixels <= 100000;
 }
 
 // The strip filter's lists, from the box tests of the frame shape's sample

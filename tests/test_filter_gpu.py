@@ -67,7 +67,7 @@ def test_infinite_values(oracle, filt, w, k):
 # size: tiles cut by the frame's edge, crop windows, gamma, infinities, and the
 # last frame with tiles beside the first without.
 @pytest.mark.parametrize("res", [(8, 8), (9, 33), (200, 31), (7, 130), (64, 40)])
-@pytest.mark.parametrize("samples,w", [((3, 3), 2.0), ((3, 3), 4.0), ((1, 1), 4.0), ((2, 1), 6.0)])
+@pytest.mark.parametrize("samples,w", [((3, 3), 2.0), ((3, 3), 4.0), ((1, 1), 4.0), ((2, 1), 6.0), ((1, 2), 6.0)])
 def test_tiled_frames(oracle, res, samples, w):
     print(f"tiles {res} {samples} {w}", flush=True)
     opts, prims = scenes.patches_scene(seed=9, n=40, res=res, samples=samples, filt=("catmull-rom", w, w), size_px=14.0)
