@@ -141,6 +141,11 @@ struct PrimDev {
     uint32_t matte;                       // RH_MATTE_*
 };
 
+// The persistent sampler's queues and the words between their heads: queue q
+// hands out the items q, q + RH_QUEUES, ...
+#define RH_QUEUES 8
+#define RH_QUEUE_WORDS 32
+
 // What a frame clears as it begins.
 struct FrameClear {
     unsigned long long* counters;

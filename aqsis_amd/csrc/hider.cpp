@@ -974,7 +974,7 @@ rh_status rh_create(const rh_options* opt, rh_ctx** out) {
         if (e == hipSuccess) e = upload(c->dItemsGrid, cut, c->st);
         if (e == hipSuccess) e = c->dItems.ensure((size_t)c->maxItems * sizeof(uint2));
         if (e == hipSuccess) e = c->dItemCount.ensure(RH_PLAN_WORDS * sizeof(uint32_t));
-        if (e == hipSuccess) e = c->dQueue.ensure(16);
+        if (e == hipSuccess) e = c->dQueue.ensure(RH_QUEUES * RH_QUEUE_WORDS * sizeof(uint32_t));
         if (e == hipSuccess) e = c->dRows.ensure((size_t)c->maxRows * 5 * sizeof(uint32_t));
     }
     // The scratch array's address on this device (for the no-allocation

@@ -979,19 +979,23 @@ __device__ __forceinline__ uint32_t hit_entry(HitArena& a, unsigned long long am
 // a static grid over the items (one workgroup each, runs of RH_S_GROUP
 // items per XCD when the grid is a multiple of 8 * RH_S_GROUP), the same per
 // bucket (itemBase/nStatic select the bucket's items), and persistent
-// workgroups pulling items from a queue (persistent != 0; the count is in
-// *nDevice).  Each workgroup writes one row of counters at rowBase +
+// workgroups pulling items from RH_QUEUES queues (PERSISTENT; the count is in
+// *nDevice): atomics that return from one address come about 10 ns apart, which
+// one queue of a sparse frame's many small items waited for (1280x640, 2x2
+// samples, 12,800 items 182 to 88 us).  Each workgroup writes one row of counters at rowBase +
 // blockIdx.x.  STORE selects StoreSample's mode (RH_STORE_*): the usual
 // occluding hit, the midpoint store, or every hit listed (not cullable).
-// (rowCounts stands among the read parameters: the compiler loads neighbouring
-// parameters together, and with the ones after it moved up it held more of them at
-// once and read 335 scalars back from lanes instead of 269: 2048x2048 clustered
-// 5928 us against 5888.)
-template <int CH, int SLOTS, int STORE = RH_STORE_OCCLUDE, int WPE = 4>
+// PERSISTENT is a form of its own, which leaves each form the scalars of its own
+// loop, and the order of the parameters decides which of them the compiler loads
+// together and keeps: 186 scalars read back from lanes (static) and 179 with
+// nDevice before the items and rowCounts among the read parameters, 224 and 325
+// with nDevice behind them, 265 in one kernel for both (1280x720, 4x4 samples 484
+// to 475 us; 2048x2048 clustered 5888 either way, 5928 at 335).
+template <int CH, int SLOTS, int STORE, int WPE, bool PERSISTENT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 rh_sample(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets, const TaskDev* __restrict__ tasks,
-          const uint2* __restrict__ items, int itemBase, int nStatic, const uint32_t* __restrict__ nDevice,
-          int persistent, uint32_t* __restrict__ queueHead, const unsigned long long* __restrict__ capStart,
+          const uint32_t* __restrict__ nDevice, const uint2* __restrict__ items, int itemBase, int nStatic,
+          uint32_t* __restrict__ queueHead, const unsigned long long* __restrict__ capStart,
           const uint32_t* __restrict__ listCount, const uint32_t* __restrict__ lists,
           const float4* __restrict__ mprec4, uint32_t* __restrict__ rowCounts,
           const PrimDev* __restrict__ prims,
@@ -1023,19 +1027,25 @@ rh_sample(const FrameDev* __restrict__ fr, const BucketDev* __restrict__ buckets
     // wave-uniform counts (ballots)
     uint32_t nBound = 0, nHit = 0, nIn = 0, nIn2 = 0;
     HitArena arena = hit_arena(fr->hitCapacity, hitCtl, hitShards, blockIdx.x + wave * (RH_HIT_SHARDS / RH_S_WAVES));
-    const int itemEnd = persistent ? (int)nDevice[0] : itemBase + nStatic;
+    const int itemEnd = PERSISTENT ? (int)nDevice[0] : itemBase + nStatic;
     // isCullable (bucketprocessor.cpp:1076-1081): occlusion tests and the
     // occluding hit apply; else every hit is listed
     constexpr bool cullH = STORE != RH_STORE_LIST_ALL;
     constexpr bool MID = STORE == RH_STORE_MIDPOINT;
 
+    uint32_t queue = blockIdx.x % RH_QUEUES;   // PERSISTENT: the queue served; at its end the next, once round
     for (int round = 0;; ++round) {
     int it;
-    if (persistent) {
-        if (tid == 0) sItem = (int)atomicAdd(queueHead, 1u);
-        __syncthreads();
-        it = sItem;
-        __syncthreads();
+    if (PERSISTENT) {
+        for (;;) {
+            if (tid == 0) sItem = (int)(atomicAdd(queueHead + queue * RH_QUEUE_WORDS, 1u) * RH_QUEUES + queue);
+            __syncthreads();
+            it = sItem;
+            __syncthreads();
+            if (it < itemEnd) break;
+            queue = (queue + 1) % RH_QUEUES;
+            if (queue == blockIdx.x % RH_QUEUES) break;
+        }
     } else {
         if (round > 0) break;
         if (gridDim.x % (8 * RH_S_GROUP) == 0) {
@@ -2596,10 +2606,8 @@ __global__ void __launch_bounds__(256) rh_plan_items(const FrameDev* __restrict_
         uint32_t start = 0;
         for (int b = 32; b > tid; --b) start += ctl[RH_PLAN_HIST + b];
         base[tid] = start + (mine[tid] ? atomicAdd(&ctl[RH_PLAN_NEXT + tid], mine[tid]) : 0u);
-        if (blockIdx.x == 0 && tid == 0) {
-            ctl[0] = start + ctl[RH_PLAN_HIST];
-            queueHead[0] = 0;
-        }
+        if (blockIdx.x == 0 && tid == 0) ctl[0] = start + ctl[RH_PLAN_HIST];
+        if (blockIdx.x == 0 && tid < RH_QUEUES) queueHead[tid * RH_QUEUE_WORDS] = 0;
     }
     __syncthreads();
     if (t >= ntasks) return;
@@ -3821,8 +3829,9 @@ extern "C" hipError_t rh_launch_bin(hipStream_t st, const FrameDev* fr, const Bu
 
 template <int CH, int SLOTS, int STORE = RH_STORE_OCCLUDE, int WPE = 4>
 static void launch_sample_t(hipStream_t st, int grid, const SampleLaunch& a) {
-    hipLaunchKernelGGL((rh_sample<CH, SLOTS, STORE, WPE>), dim3(grid), dim3(256), 0, st, a.fr, a.buckets, a.tasks, a.items,
-                       a.itemBase, a.nStatic, a.nDevice, a.persistent, a.queueHead, a.capStart, a.listCount, a.lists,
+    auto* k = a.persistent ? &rh_sample<CH, SLOTS, STORE, WPE, true> : &rh_sample<CH, SLOTS, STORE, WPE, false>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a.fr, a.buckets, a.tasks, a.nDevice,
+                       a.items, a.itemBase, a.nStatic, a.queueHead, a.capStart, a.listCount, a.lists,
                        reinterpret_cast<const float4*>(a.mprec), a.rowCounts, a.prims, a.pos2d, a.pos1d, a.pixPattern,
                        a.samples, a.hitData, a.hitNext, a.hitCtl, a.hitShards, a.hitHeads, a.frontDepth,
                        a.rowBase, a.idCut, a.itemCut, a.depthOnly);
@@ -3906,14 +3915,14 @@ extern "C" hipError_t rh_launch_sample_dof(hipStream_t st, const SampleLaunch* a
 }
 
 // Workgroups of one sampling variant that fit the device at once.
+// Workgroups of the persistent form a CU holds.
 extern "C" hipError_t rh_sample_occupancy(int variant, int* blocksPerCU) {
+    auto of = [&](auto* k) { return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocksPerCU, k, 256, 0); };
     switch (variant) {
-    case 0: return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocksPerCU, rh_sample<216, 4>, 256, 0);
-    case 1: return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocksPerCU, rh_sample<216, 2>, 256, 0);
-    case 2: return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocksPerCU, rh_sample<96, 4>, 256, 0);
-    case 3:
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocksPerCU, rh_sample<96, 2, RH_STORE_OCCLUDE, RH_WPE_96_2>,
-                                                            256, 0);
+    case 0: return of(rh_sample<216, 4, RH_STORE_OCCLUDE, 4, true>);
+    case 1: return of(rh_sample<216, 2, RH_STORE_OCCLUDE, 4, true>);
+    case 2: return of(rh_sample<96, 4, RH_STORE_OCCLUDE, 4, true>);
+    case 3: return of(rh_sample<96, 2, RH_STORE_OCCLUDE, RH_WPE_96_2, true>);
     default: return hipErrorInvalidValue;
     }
 }

@@ -68,3 +68,23 @@ def test_autotune_keeps_results():
         assert t["mode"] in (0, 2) and t["frame_ms"] > 0
         h.render_device()
         _same(ref, _frame(h))
+
+
+@pytest.mark.parametrize("res,k", [((4, 4), 8), ((16, 16), 4), ((24, 40), 4), ((40, 16), 2), ((130, 70), 1), ((300, 40), 3)])
+def test_few_items(res, k):
+    # fewer work items than the persistent workgroups' queues, as many, some more
+    from aqsis_amd import scenes
+    from aqsis_amd.hider import Hider
+    print(f"few items {res} {k}x{k}", flush=True)
+    opts, prims = scenes.patches_scene(seed=21, n=12, res=res, samples=(k, k), filt=("box", 1.0, 1.0), size_px=9.0)
+    for p in prims:
+        p.no_cull_hidden = 1
+    with Hider(opts) as h:
+        h.post_surfaces(prims)
+        h.render()
+        ref = _frame(h)
+        for bpw in (4, 2):
+            h.set_tuning(mode="batched", blocks_per_wave=bpw, split_cost=1 << 22)
+            for _ in range(3):
+                h.render_device()
+                _same(ref, _frame(h))
