@@ -2010,10 +2010,15 @@ static uint64_t frame_bytes(const rh::Shape& s) {
     // list counts and capacities, work items, counter rows; the batched form's items
     bytes += tasks * (sizeof(TaskDev) + 4 + 8 + 8) + items * (8 + 20) + blocks * 8;
     bytes += 128 << 10;                    // the other counter rows, the filter's list, control words
-    // The filter's box tests, where they can differ between pixels: a sample of
-    // the outermost column or row lies within the box by where it is in its
-    // pixel, if the box ends inside that pixel.
-    if (s.xfwo2 < s.shiftX + 0.5f || s.yfwo2 < s.shiftY + 0.5f) bytes += ext * (2 * s.shiftX + 2 * s.shiftY + 2) * 8;
+    // The filter's box tests.  They can differ between pixels where the box ends
+    // inside the outermost column's or row's pixel; which kernel such a frame
+    // takes depends on its tables, and both their forms fit.  Elsewhere each
+    // column lists all its samples.
+    const uint64_t bySample = ext * ns * 2;
+    if (s.xfwo2 < s.shiftX + 0.5f || s.yfwo2 < s.shiftY + 0.5f)
+        bytes += std::max(ext * (2 * s.shiftX + 2 * s.shiftY + 2) * 8, rh_filter_tile_lds(s.ns, s.shiftX, s.shiftY) ? bySample : 0);
+    else if (filter_tiled(s, 0, ((2 * s.shiftX + 1) * ((s.ns + 3) / 4) + 1) / 2 * 2))
+        bytes += bySample;
     return bytes;
 }
 
