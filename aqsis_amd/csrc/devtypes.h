@@ -222,7 +222,7 @@ struct DisplayFormat {
 #define RH_DSPY_SIGNED8_D 7
 
 // Bytes a read-back workgroup copies.
-#define RH_READ_WG_BYTES 65536
+#define RH_READ_WG_BYTES 16384
 
 // The strip filter's list (rh_filter_strip): the samples of a halo row that
 // add to a pixel, in the reference's order (filter columns, samples), in

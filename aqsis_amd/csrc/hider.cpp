@@ -279,21 +279,22 @@ private:
     }
 };
 
-// Copy a result from the device once its context's stream is through (`pending`:
-// it may not be).  A plain copy into pageable memory takes 12 us, 24 at 37 KB, 15
-// to 69 at 147 KB and 20 to 265 at 0.27 MB (from 64 KB on the runtime pins the
-// caller's pages, and what that costs is up to how they are mapped), and from 1 MB
-// on runs at 17 GB/s (one thread copies out of the runtime's staging memory).  So
-// results go by way of a lane: copied there and on by the calling thread up to
-// 1.5 MB (16 us at 147 KB, 21 at 0.27 MB, 38 at 0.69, 79 at 1.3 and 122 at 2.4),
-// above by a kernel that writes into the lane, each workgroup setting a flag
-// behind its part, while up to 8 of the worker pool's threads copy the pieces on
-// (0.15 MB 42 us, 0.69 75, 1.3 84, 2.4 102, 8.3 280, 16.8 460; plain 157, 485 and
-// 966).  (An asynchronous copy on the stream and a wait for it take 35 us where
-// the plain copy takes 12, so that is for results still to be computed.)
+// Copy a result from the device: a kernel behind whatever computes it writes it
+// into a lane, each workgroup setting a flag behind its part, and parts are copied
+// on as their flags come, by the calling thread up to 1.5 MB and above by up to 8
+// of the worker pool's threads too.  No wait for the stream is left to do then.
+// 9 KB take 10 us, 37 KB 11, 0.11 MB 14, 0.27 20, 0.59 34, 1.3 63, 2.4 83, 8.3 280
+// and 16.8 460.  Plain copies into pageable memory take 12 (or 16), 24, 13 to 130,
+// 20 to 265, 41 to 260, 87, 148, 485 and 966: from 64 KB on the runtime pins the
+// caller's pages, at a price that depends on how they are mapped, and from 1 MB on
+// one thread copies out of the runtime's staging memory.  A blocking copy into the
+// lane takes 17 us for 9 KB, 13 to 130 for 0.11 MB, 33 for 0.59 and 75 for 1.3.
+// With the pool at work from 0.5 MB on, 0.59 MB take 38 to 46 us and 0.69 49, alone
+// 34 and 38; 2.4 MB alone 96.
 // dst may be any host memory; src a context's buffer (read to a multiple of 16 bytes).
-constexpr size_t kReadPlain = 16 << 10;     // bytes of a result at hand below which nothing is gained by a lane
 constexpr size_t kReadShared = 1536 << 10;  // bytes from which the pool's threads take part
+constexpr size_t kPart = 64 << 10;          // bytes the caller alone copies on at a time
+static_assert(kReadShared / kPart <= 32, "a bit of a word each");
 
 // The GPU may be at another context's frame still, and the pool is every
 // context's: a read keeps it for 100 us more than the copy takes at 16 GB/s,
@@ -301,27 +302,20 @@ constexpr size_t kReadShared = 1536 << 10;  // bytes from which the pool's threa
 // its threads wake too late: 2.4 MB 39 us longer.)
 constexpr std::chrono::microseconds kPoolHold{100};
 
-hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st, bool pending = false) {
-    ReadLane* lane = bytes >= kReadPlain || pending ? PinnedPool::get().take_lane() : nullptr;
+hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st) {
+    ReadLane* lane = PinnedPool::get().take_lane();
     hipError_t e = hipSuccess;
-    if (!lane || bytes < kReadShared) {
-        void* to = lane ? lane->p : dst;
-        if (pending) {
-            e = hipMemcpyAsync(to, src, bytes, hipMemcpyDeviceToHost, st);
-            if (e == hipSuccess) e = hipStreamSynchronize(st);
-        } else {
-            e = hipMemcpy(to, src, bytes, hipMemcpyDeviceToHost);
-        }
-        if (!lane) return e;
-        if (e == hipSuccess) std::memcpy(dst, lane->p, bytes);
-        PinnedPool::get().give_lane(lane);
-        return e;
+    if (!lane) {                                         // no pinned memory, or four reads at work
+        // (a copy on the stream takes 35 us where the plain one takes 12)
+        if (hipStreamQuery(st) == hipSuccess) return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+        e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
+        return e == hipSuccess ? hipStreamSynchronize(st) : e;
     }
     for (size_t from = 0; from < bytes && e == hipSuccess; from += kLaneBytes) {
         const size_t len = std::min(kLaneBytes, bytes - from);
         unsigned char* to = static_cast<unsigned char*>(dst) + from;
-        // up to 16 pieces of whole workgroups, 256 KB at least
-        size_t piece = std::max<size_t>(256 << 10, (len + 15) / 16);
+        // pieces of whole workgroups: 64 KB alone, or up to 16 of 256 KB at least
+        size_t piece = len >= kReadShared ? std::max<size_t>(256 << 10, (len + 15) / 16) : kPart;
         piece = (piece + RH_READ_WG_BYTES - 1) / RH_READ_WG_BYTES * RH_READ_WG_BYTES;
         const int n = (int)((len + piece - 1) / piece);
         const uint32_t seq = ++lane->seq;
@@ -373,7 +367,7 @@ hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st, b
                 continue;
             }
             bool shared = false;
-            if (n - i > 1) try {
+            if (n - i > 1 && len >= kReadShared) try {
                     until = Clock::now() + kPoolHold + std::chrono::nanoseconds(len / 16);
                     shared = rh::run_if_free(n, 8, std::ref(help));
                 } catch (...) {
@@ -388,9 +382,9 @@ hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st, b
                 taken |= 1u << i;
             }
         }
-        // nothing may still be writing to the lane when it is used again
-        e = hipStreamSynchronize(st);
-        if (e == hipSuccess && lost) e = hipErrorUnknown;
+        // With every flag up the kernel has written its last; of a failed one
+        // nothing may still be writing to the lane when it is used again.
+        if (lost && (e = hipStreamSynchronize(st)) == hipSuccess) e = hipErrorUnknown;
     }
     PinnedPool::get().give_lane(lane);
     return e;
@@ -1831,7 +1825,7 @@ static rh_status format_frame(rh_ctx* c, const DisplayFormat& f, int32_t type, c
     }
     HIP_TRY(c->dFormat.ensure(bytes));
     HIP_TRY(rh_launch_format_display(c->st, type, &f, c->dChannels.as<float>(), dither, npix, c->dFormat.p));
-    HIP_TRY(read_back(out, c->dFormat.p, bytes, c->st, true));
+    HIP_TRY(read_back(out, c->dFormat.p, bytes, c->st));
     return RH_OK;
 }
 

@@ -73,7 +73,7 @@ Stream* S(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
 
 // rh_read_back(src, dst, bytes, flags, seq), a workgroup at a time
 void read_back(Stream* st, unsigned grid, const char* src, char* dst, size_t bytes, volatile uint32_t* flags, uint32_t seq) {
-    const size_t per = 65536;
+    const size_t per = 16384;
     for (unsigned w = 0; w < grid && !g_lose; ++w) {
         {
             std::unique_lock<std::mutex> lk(g_m);
