@@ -705,9 +705,12 @@ static std::pair<int, int> task_grid(const rh::Shape& s, size_t bucket) {
 // sides in us, the frame's counters included, strips first:
 //   width 4, 1x1 samples   46/26 at 160x120   139/86 at 640x480   518/464 at 1920x1080
 //   width 6, 2x1 samples   82/31              223/119             818/659
-//   width 6, 1x4 samples   71/32              192/121             690/698
-//   width 4, 3x3 samples   70/34              233/161             902/920
-//   width 2, 3x3 samples   29/24              99/81               382/439
+//   width 6, 1x4 samples   71/32              192/121             690/698 (641/555 at 1280x1280)
+//   width 6, 1x5 samples                                          1126/877
+//   width 4, 1x6 samples                                          661/622 (446/376 at 1280x960)
+//   width 6, 2x3 samples                                          1019/1015 (920/812 at 1280x1280)
+//   width 4, 3x3 samples   70/34              233/161             902/920 (785/744 at 1440x1160)
+//   width 2, 3x3 samples   29/24              99/81               382/439 (250/267 at 1280x960)
 //   width 6, 3x3 samples   136/47             391/339             1448/2060 (57 KB of LDS a tile; 642/640 at 900x675)
 //   width 2, 4x3 samples   28/25              84/88               344/487
 //   width 2, 1x1 samples   25/24              70/76               254/402
@@ -724,7 +727,8 @@ static bool filter_tiled(const rh::Shape& s, int vary, int groups) {
     if (!lds || words < 24) return false;
     if (vary == 0) return 4 * words >= taps && pixels > 8192 && pixels <= 150000;
     if (2 * words >= taps) return true;
-    if (4 * words >= taps) return pixels <= (lds <= (48 << 10) ? 1280 * 720 : 550000);
+    if (4 * words >= taps)
+        return pixels <= (lds > (48 << 10) ? 550000 : s.ns <= 8 ? 2100000 : words < 50 ? 1280 * 720 : 1700000);
     return 2 * vary > groups && pixels <= 100000;
 }
 
