@@ -16,11 +16,18 @@
 //                       occlusion, LOD, point-in-quad, inverse bilinear,
 //                       depth, store) in list order; transparent hits go to
 //                       per-sample lists.
+//   rh_sample_mb, rh_sample_dof
+//                       the same for frames with moving surfaces and with
+//                       depth of field.
 //   rh_combine          samples with transparent hits: depth sort as
 //                       std::sort, back-to-front compositing.
-//   rh_box_masks        per frame shape: each sample's filter-box tests.
+//   rh_box_classes/masks, rh_sample_boxes
+//                       per frame shape: the filter-box tests of the samples,
+//                       in all, by pixel or by sample.
 //   rh_filter_strip     strips of 8 pixel columns, a halo row in LDS: the filter,
 //                       exposure, quantise + dither.
+//   rh_filter_tiled     the same by tiles of 8x8 pixels, halo and all in LDS.
+//   rh_read_back        a result into pinned host memory, a flag per part.
 //
 // All single-precision code is built with -ffp-contract=off and correctly
 // rounded division; every expression keeps the operand order of the aqsis
